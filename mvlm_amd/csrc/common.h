@@ -197,10 +197,9 @@ struct Epilogue {
 
 // Kernel launchers (defined in the .hip files).  They assume validated input.
 // A null Epilogue pointer means none.
-hipError_t launch_gemm_naive(hipStream_t s, const uint16_t* A, const uint16_t* B, uint16_t* C,
-                             int M, int N, int K);
-hipError_t launch_gemm_tiled(hipStream_t s, const uint16_t* A, const uint16_t* B, uint16_t* C,
-                             int M, int N, int K);
+// C[M,N] = A[M,K] B[K,N], fp16 row-major, one fp32 fma chain per output in ascending k
+hipError_t launch_gemm_order(hipStream_t s, const uint16_t* A, const uint16_t* B, uint16_t* C, int M, int N, int K,
+                             int num_cus);
 // y[N] = W[N,K] x[K], packed fp16 W, fp16 x and y, the reference gemv's
 // summation order (x 8-byte aligned)
 hipError_t launch_gemv_exact(hipStream_t s, const uint16_t* x, const mvlm_weight* W, uint16_t* y);

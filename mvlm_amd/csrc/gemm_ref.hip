@@ -2,9 +2,9 @@
 //
 // gemm_naive (src/kernels/gemm.cl:26-51) and gemm_tiled (gemm.cl:74-136)
 // compute, per output, acc = fma(A[row,k], B[k,col], acc) over k = 0..K-1 in
-// fp32 from fp16 inputs and store RNE fp16.  Both kernels here keep that
-// exact per-output fma sequence, so their results are bit-identical to each
-// other and to a CPU restatement; only the work partition differs.
+// fp32 from fp16 inputs and store RNE fp16.  gemm_order_kernel keeps that exact
+// per-output fma sequence, so its results are bit-identical to a CPU
+// restatement; only the work partition differs.
 //   A [M,K], B [K,N], C [M,N], fp16 row-major.
 // gemv_exact keeps the reference gemv's split of K over 256 partial sums and
 // its fold order on the packed fp16 weight.
@@ -13,93 +13,161 @@
 
 namespace mvlm {
 
-// One thread per output; threadIdx.x walks columns so B and C accesses are
-// coalesced (the reference maps gid0 to rows, which strides B by N).
-__global__ __launch_bounds__(256) void gemm_naive_kernel(const uint16_t* __restrict__ A,
-                                                         const uint16_t* __restrict__ B,
-                                                         uint16_t* __restrict__ C, int M, int N, int K) {
-    int col = blockIdx.x * 16 + (threadIdx.x & 15);
-    int row = blockIdx.y * 16 + (threadIdx.x >> 4);
-    if (row >= M || col >= N) return;
-    const uint16_t* a = A + (int64_t)row * K;
-    const uint16_t* b = B + col;
-    float acc = 0.0f;
-    for (int k = 0; k < K; ++k)
-        acc = __builtin_fmaf(f16_bits_to_f32(a[k]), f16_bits_to_f32(b[(int64_t)k * N]), acc);
-    C[(int64_t)row * N + col] = f32_to_f16_bits(acc);
-}
+// The products run on v_mfma_f32_16x16x4_f32.  The product of two widened
+// fp16 values is exact in fp32, and that instruction adds its four products to
+// the accumulator one after another in ascending k, each sum rounded to
+// nearest even (checked bit by bit against the fma chain over random, wide
+// range, subnormal and infinite inputs), so a chain of them is the reference's
+// fma sequence at twice the vector ALU's fp32 rate (256 flops per CU and
+// clock).  Zeros past K leave an accumulator as it is: it is never -0, since
+// it starts at +0 and a sum of two values of opposite sign that cancels is +0.
+//
+// Bound: the fp32 matrix rate (157 TFLOP/s at 2.4 GHz).  An MFMA occupies its
+// SIMD for 32 cycles, which leaves room for the two 2-byte LDS reads and the
+// two conversions that feed it, so operands stay fp16 in LDS in the layout
+// they have in memory and are widened on the way into registers.  A block of
+// NW waves owns a BM x BN tile of C, a wave TM x TN tiles of 16 x 16; the next
+// BK-wide slice of A and B is in flight to registers while the current one is
+// multiplied, and the LDS slices alternate (one barrier per slice).  2048^3:
+// 399 -> 156 us (43 -> 110 TFLOP/s) against the vector-ALU kernel of 64 x 64
+// tiles this replaces; 256^3 36 -> 5.2 us, 32 x 2048 x 2048 253 -> 22 us,
+// rows off the 16-byte grid (1500^3) 293 -> 101 us.
+// Operand layout: lane l supplies A[l%16][k + l/16] and B[k + l/16][l%16];
+// accumulator register i of lane l is C[4*(l/16) + i][l%16].
+// Rows start at any 2-byte address (or odd byte, in a view): 16-byte loads take
+// unaligned addresses here, and only the chunk at the end of a row is read
+// element by element.
+template <int BM, int BN, int BK, int WGM, int WGN>
+__global__ __launch_bounds__(64 * WGM * WGN) void gemm_order_kernel(const uint16_t* __restrict__ A,
+                                                                    const uint16_t* __restrict__ B,
+                                                                    uint16_t* __restrict__ C, int M, int N, int K,
+                                                                    int tiles_m) {
+    constexpr int NT = 64 * WGM * WGN;
+    constexpr int WM = BM / WGM, WN = BN / WGN, TM = WM / 16, TN = WN / 16;
+    // LDS pitches (elements): the 16 rows x 4 k of an A read and the 4 k x 16
+    // columns of a B read fall on distinct banks
+    constexpr int PA = BK + 4, PB = BN + 16;
+    constexpr int CA = BM * BK / 8 / NT, CB = BK * BN / 8 / NT;   // 8-element chunks per thread and slice
+    static_assert(CA >= 1 && CB >= 1 && CA * 8 * NT == BM * BK && CB * 8 * NT == BK * BN, "chunks per thread");
+    __shared__ __attribute__((aligned(16))) uint16_t As[2][BM * PA];
+    __shared__ __attribute__((aligned(16))) uint16_t Bs[2][BK * PB];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int l16 = lane & 15, q = lane >> 4;
+    const int wm = (wave / WGN) * WM, wn = (wave % WGN) * WN;
+    // each XCD takes a contiguous run of tiles, the M tiles of one column of
+    // tiles next to each other (they read the same columns of B)
+    int t = blockIdx.x;
+    const int per = (int)gridDim.x / 8;
+    if (t < 8 * per) t = (t % 8) * per + t / 8;
+    const int m0 = (t % tiles_m) * BM, n0 = (t / tiles_m) * BN;
 
-hipError_t launch_gemm_naive(hipStream_t s, const uint16_t* A, const uint16_t* B, uint16_t* C,
-                             int M, int N, int K) {
-    dim3 grid((N + 15) / 16, (M + 15) / 16);
-    launch_kernel(gemm_naive_kernel, grid, dim3(256), 0, s, A, B, C, M, N, K);
-    return hipGetLastError();
-}
-
-// 64x64 output tile per 256-thread block, 4x4 outputs per thread, K staged in
-// 32-wide LDS slices (values widened to fp32 on the way in, which is exact).
-// Each thread walks k in ascending order inside and across slices, so every
-// output sees the same fma sequence as gemm_naive.
-constexpr int TT = 64;    // tile edge
-constexpr int TK = 32;    // K slice
-
-__global__ __launch_bounds__(256) void gemm_tiled_kernel(const uint16_t* __restrict__ A,
-                                                         const uint16_t* __restrict__ B,
-                                                         uint16_t* __restrict__ C, int M, int N, int K) {
-    __shared__ float As[TT][TK + 1];
-    __shared__ float Bs[TK][TT];
-    const int tx = threadIdx.x & 15, ty = threadIdx.x >> 4;
-    const int m0 = blockIdx.y * TT, n0 = blockIdx.x * TT;
-    float acc[4][4];
+    u32x4 ra[CA], rb[CB];
+    auto load8 = [](const uint16_t* p, int left) {   // p[0..8), zeros from `left` on
+        u32x4 v = {0u, 0u, 0u, 0u};
+        if (left >= 8) {
+            __builtin_memcpy(&v, p, 16);
+        } else if (left > 0) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = 0.0f;
-
-    for (int k0 = 0; k0 < K; k0 += TK) {
-        // A slice: 64 rows x 32 k; B slice: 32 k x 64 cols; 8 elements each per thread.
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-            int idx = threadIdx.x + e * 256;
-            int ar = idx / TK, ak = idx % TK;
-            int gr = m0 + ar, gk = k0 + ak;
-            As[ar][ak] = (gr < M && gk < K) ? f16_bits_to_f32(A[(int64_t)gr * K + gk]) : 0.0f;
-            int bk = idx / TT, bc = idx % TT;
-            int gk2 = k0 + bk, gc = n0 + bc;
-            Bs[bk][bc] = (gk2 < K && gc < N) ? f16_bits_to_f32(B[(int64_t)gk2 * N + gc]) : 0.0f;
+            for (int e = 0; e < 7; ++e)
+                if (e < left) v[e >> 1] |= (uint32_t)p[e] << (16 * (e & 1));
         }
-        __syncthreads();
-        const int kn = min(TK, K - k0);   // the zero padding beyond K is never accumulated
-        for (int k = 0; k < kn; ++k) {
-            float a[4], b[4];
+        return v;
+    };
+    auto load = [&](int k0) {
 #pragma unroll
-            for (int i = 0; i < 4; ++i) a[i] = As[ty * 4 + i][k];
-#pragma unroll
-            for (int j = 0; j < 4; ++j) b[j] = Bs[k][tx * 4 + j];
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-#pragma unroll
-                for (int j = 0; j < 4; ++j) acc[i][j] = __builtin_fmaf(a[i], b[j], acc[i][j]);
+        for (int c = 0; c < CA; ++c) {
+            const int i = tid + c * NT, r = i / (BK / 8), k = k0 + 8 * (i % (BK / 8));
+            ra[c] = load8(A + (int64_t)(m0 + r) * K + k, m0 + r < M ? K - k : 0);
         }
+#pragma unroll
+        for (int c = 0; c < CB; ++c) {
+            const int i = tid + c * NT, k = k0 + i / (BN / 8), n = n0 + 8 * (i % (BN / 8));
+            rb[c] = load8(B + (int64_t)k * N + n, k < K ? N - n : 0);
+        }
+    };
+    auto store = [&](int buf) {
+#pragma unroll
+        for (int c = 0; c < CA; ++c) {
+            const int i = tid + c * NT;
+            uint16_t* d = As[buf] + (i / (BK / 8)) * PA + 8 * (i % (BK / 8));   // 8-byte aligned
+            *reinterpret_cast<u32x2*>(d) = u32x2{ra[c][0], ra[c][1]};
+            *reinterpret_cast<u32x2*>(d + 4) = u32x2{ra[c][2], ra[c][3]};
+        }
+#pragma unroll
+        for (int c = 0; c < CB; ++c) {
+            const int i = tid + c * NT;
+            *reinterpret_cast<u32x4*>(Bs[buf] + (i / (BN / 8)) * PB + 8 * (i % (BN / 8))) = rb[c];
+        }
+    };
+
+    f32x4 acc[TM][TN];
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) acc[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+
+    load(0);
+    store(0);
+    __syncthreads();
+    for (int k0 = 0, buf = 0; k0 < K; k0 += BK, buf ^= 1) {
+        const bool more = k0 + BK < K;
+        if (more) load(k0 + BK);
+        const uint16_t* as = As[buf] + (wm + l16) * PA + q;
+        const uint16_t* bs = Bs[buf] + q * PB + wn + l16;
+#pragma unroll
+        for (int k = 0; k < BK; k += 4) {
+            float a[TM], b[TN];
+#pragma unroll
+            for (int i = 0; i < TM; ++i) a[i] = f16_bits_to_f32(as[16 * i * PA + k]);
+#pragma unroll
+            for (int j = 0; j < TN; ++j) b[j] = f16_bits_to_f32(bs[k * PB + 16 * j]);
+#pragma unroll
+            for (int i = 0; i < TM; ++i)
+#pragma unroll
+                for (int j = 0; j < TN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i], b[j], acc[i][j], 0, 0, 0);
+        }
+        // the other slice was last read before the barrier that ended the
+        // previous round
+        if (more) store(buf ^ 1);
         __syncthreads();
     }
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        int row = m0 + ty * 4 + i;
-        if (row >= M) continue;
+    for (int i = 0; i < TM; ++i)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            int col = n0 + tx * 4 + j;
-            if (col < N) C[(int64_t)row * N + col] = f32_to_f16_bits(acc[i][j]);
+        for (int j = 0; j < TN; ++j) {
+            const int col = n0 + wn + 16 * j + l16;
+            if (col >= N) continue;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int row = m0 + wm + 16 * i + 4 * q + r;
+                if (row < M) C[(int64_t)row * N + col] = f32_to_f16_bits(acc[i][j][r]);
+            }
         }
-    }
 }
 
-hipError_t launch_gemm_tiled(hipStream_t s, const uint16_t* A, const uint16_t* B, uint16_t* C,
-                             int M, int N, int K) {
-    dim3 grid((N + TT - 1) / TT, (M + TT - 1) / TT);
-    launch_kernel(gemm_tiled_kernel, grid, dim3(256), 0, s, A, B, C, M, N, K);
+template <int BM, int BN, int BK, int WGM, int WGN>
+static hipError_t launch_order(hipStream_t s, const uint16_t* A, const uint16_t* B, uint16_t* C, int M, int N, int K) {
+    const int tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
+    launch_kernel(gemm_order_kernel<BM, BN, BK, WGM, WGN>, dim3((unsigned)(tiles_m * tiles_n)), dim3(64 * WGM * WGN), 0, s,
+                  A, B, C, M, N, K, tiles_m);
     return hipGetLastError();
+}
+
+// Serves mvlm_gemm_naive and mvlm_gemm_tiled.  The tile with the least work on
+// the busiest CU: block rounds x tile area, the smaller tiles weighted by the
+// operand bytes they move per product.  (1024^3 takes 256 blocks of 64: 30 us;
+// 2048^3 takes 256 blocks of 128.)
+hipError_t launch_gemm_order(hipStream_t s, const uint16_t* A, const uint16_t* B, uint16_t* C, int M, int N, int K,
+                             int num_cus) {
+    const int cus = num_cus > 0 ? num_cus : 256;
+    auto cost = [&](int edge, double weight) {
+        const int64_t tiles = (int64_t)((M + edge - 1) / edge) * ((N + edge - 1) / edge);
+        return (double)((tiles + cus - 1) / cus) * edge * edge * weight;
+    };
+    const double c128 = cost(128, 1.0), c64 = cost(64, 1.1), c32 = cost(32, 1.35);
+    if (c128 <= c64 && c128 <= c32) return launch_order<128, 128, 32, 4, 2>(s, A, B, C, M, N, K);
+    if (c64 <= c32) return launch_order<64, 64, 64, 2, 2>(s, A, B, C, M, N, K);
+    return launch_order<32, 32, 128, 2, 2>(s, A, B, C, M, N, K);
 }
 
 // gemv (gemm.cl:215-270) as launched by dispatch_gemv (compute.cpp:141-147):

@@ -16,7 +16,7 @@ using namespace mvlm;
 
 namespace {
 
-enum OpKind { OP_GEMM_NAIVE, OP_GEMM_TILED, OP_GEMV_EXACT, OP_GEMM_MFMA, OP_GEMV_DENSE, OP_GEMV_QUANT, OP_GEMV_GROUP, OP_ATTENTION,
+enum OpKind { OP_GEMM_ORDER, OP_GEMV_EXACT, OP_GEMM_MFMA, OP_GEMV_DENSE, OP_GEMV_QUANT, OP_GEMV_GROUP, OP_ATTENTION,
               OP_ATTN_STEP, OP_ARGMAX };
 
 struct Op {
@@ -102,7 +102,7 @@ int make_epilogue(mvlm_device* dev, const mvlm_epilogue* in, int M, int N, int c
     return MVLM_OK;
 }
 
-int make_ref_gemm(OpKind kind, mvlm_device* dev, const mvlm_buffer* A, const mvlm_buffer* B, mvlm_buffer* C,
+int make_ref_gemm(mvlm_device* dev, const mvlm_buffer* A, const mvlm_buffer* B, mvlm_buffer* C,
                   int M, int N, int K, const char* fn, Op* op) {
     REQUIRE(dev && A && B && C, "%s: null argument", fn);
     REQUIRE(A->dev == dev && B->dev == dev && C->dev == dev, "%s: buffers belong to another device", fn);
@@ -110,9 +110,10 @@ int make_ref_gemm(OpKind kind, mvlm_device* dev, const mvlm_buffer* A, const mvl
     NEED(A, (size_t)M * K * 2, "A");
     NEED(B, (size_t)K * N * 2, "B");
     NEED(C, (size_t)M * N * 2, "C");
-    op->kind = kind;
+    op->kind = OP_GEMM_ORDER;
     op->a = A->ptr; op->b = B->ptr; op->c = C->ptr;
     op->M = M; op->N = N; op->K = K;
+    op->num_cus = dev->prop.multiProcessorCount;
     return MVLM_OK;
 }
 
@@ -399,10 +400,9 @@ hipError_t enqueue_op(hipStream_t s, const Op& op, bool with_attn = false) {
     switch (op.kind) {
         case OP_GEMV_GROUP:
             return launch_group_op(s, op, with_attn);
-        case OP_GEMM_NAIVE:
-            return launch_gemm_naive(s, (const uint16_t*)op.a, (const uint16_t*)op.b, (uint16_t*)op.c, op.M, op.N, op.K);
-        case OP_GEMM_TILED:
-            return launch_gemm_tiled(s, (const uint16_t*)op.a, (const uint16_t*)op.b, (uint16_t*)op.c, op.M, op.N, op.K);
+        case OP_GEMM_ORDER:
+            return launch_gemm_order(s, (const uint16_t*)op.a, (const uint16_t*)op.b, (uint16_t*)op.c, op.M, op.N, op.K,
+                                     op.num_cus);
         case OP_GEMV_EXACT:
             return launch_gemv_exact(s, (const uint16_t*)op.a, op.w, (uint16_t*)op.c);
         case OP_GEMM_MFMA:
@@ -467,13 +467,13 @@ int then(int st, F&& next) {
 extern "C" int mvlm_gemm_naive(mvlm_device* dev, const mvlm_buffer* A, const mvlm_buffer* B, mvlm_buffer* C,
                                int M, int N, int K, mvlm_event** ev) {
     const char* fn = __func__;
-    RUN(make_ref_gemm(OP_GEMM_NAIVE, dev, A, B, C, M, N, K, fn, &op));
+    RUN(make_ref_gemm(dev, A, B, C, M, N, K, fn, &op));
 }
 
 extern "C" int mvlm_gemm_tiled(mvlm_device* dev, const mvlm_buffer* A, const mvlm_buffer* B, mvlm_buffer* C,
                                int M, int N, int K, mvlm_event** ev) {
     const char* fn = __func__;
-    RUN(make_ref_gemm(OP_GEMM_TILED, dev, A, B, C, M, N, K, fn, &op));
+    RUN(make_ref_gemm(dev, A, B, C, M, N, K, fn, &op));
 }
 
 extern "C" int mvlm_gemv_exact(mvlm_device* dev, const mvlm_buffer* x, const mvlm_weight* W, mvlm_buffer* y,
