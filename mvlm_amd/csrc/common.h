@@ -205,12 +205,7 @@ hipError_t launch_gemm_order(hipStream_t s, const uint16_t* A, const uint16_t* B
 hipError_t launch_gemv_exact(hipStream_t s, const uint16_t* x, const mvlm_weight* W, uint16_t* y);
 hipError_t launch_gemv_dense(hipStream_t s, const void* x, int x_dtype, const mvlm_weight* W,
                              void* y, int y_dtype, int N, int K, const Epilogue* ep = nullptr);
-// Q8_0 / Q4_0 skinny GEMM on the matrix cores, 1 <= M <= 16 (any row length)
-hipError_t launch_gemm_skinny(hipStream_t s, const float* X, const mvlm_weight* W, float* Y, int M, int N, int K,
-                              int num_cus, const Epilogue* ep = nullptr);
-// whether one skinny launch over these weights fits: K a multiple of 32 and,
-// for the tile shape the launch would pick, the LDS (which stages all of a
-// block's row-group scales) within the limit
+// whether the skinny GEMM (launch_gemm_skinny_group) takes these weights
 bool skinny_supported(int count, const mvlm_weight* const* ws, int num_cus);
 // M == 1 streaming GEMV for every weight format (rows of at most 16 KiB), and
 // for quantized weights 2 <= M <= 4 rows of x (launch_gemv_stream_batch).
@@ -259,10 +254,14 @@ hipError_t stream_attn_check(int count, const void* const* xs, int x_dtype, cons
 // The same attention as launches of its own (no sync area needed).
 hipError_t launch_attn_decode(hipStream_t s, const StreamAttnDesc& d, int num_cus);
 // Skinny GEMM over up to 8 independent problems (quantized weights of one
-// dtype, fp32 X [M][K] and Y [M][N] each, 1 <= M <= 16) in one launch.
+// dtype, fp32 X [M][K] and Y [M][N] each, 1 <= M <= 16) in one launch, and a
+// second one that adds the partial sums of rows longer than 2048 weights;
+// those are parked in the workspace (skinny_workspace_bytes; without it one
+// launch does all of it, slower).
+size_t skinny_workspace_bytes(int M, int count, const mvlm_weight* const* ws);
 hipError_t launch_gemm_skinny_group(hipStream_t s, int M, int count, const float* const* Xs,
                                     const mvlm_weight* const* ws, float* const* Ys, int num_cus,
-                                    const Epilogue* eps = nullptr);
+                                    const Epilogue* eps, void* workspace, size_t workspace_bytes);
 inline int64_t weight_row_bytes(const mvlm_weight* w) { return is_dense(w->dtype) ? w->ld * (int64_t)dtype_size(w->dtype) : w->ld; }
 // MFMA GEMM.  Its workspace (gemm_workspace_bytes) holds the fp32 partials
 // of a K split (chosen by the launcher's cost model) and zero-padded copies of

@@ -5,6 +5,7 @@
 #include <hip/hip_fp16.h>
 #include <hip/hip_bf16.h>
 #include <cstdint>
+#include <type_traits>
 
 namespace mvlm {
 
@@ -15,6 +16,15 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+
+// f(std::integral_constant<int, 0>{}), ..., f(std::integral_constant<int, N - 1>{})
+template <int N, int I = 0, class F>
+__device__ __forceinline__ void static_for(F&& f) {
+    if constexpr (I < N) {
+        f(std::integral_constant<int, I>{});
+        static_for<N, I + 1>(f);
+    }
+}
 
 __device__ __forceinline__ float f16_bits_to_f32(uint16_t h) {
     return __half2float(__ushort_as_half(h));
@@ -209,6 +219,12 @@ __device__ __forceinline__ u32x2 asm_lds_read_b64(uint32_t addr) {
     return v;
 }
 template <int OFF = 0>
+__device__ __forceinline__ uint32_t asm_lds_read_b32(uint32_t addr) {
+    uint32_t v;
+    asm volatile("ds_read_b32 %0, %1 offset:%2" : "=v"(v) : "v"(addr), "n"(OFF) : "memory");
+    return v;
+}
+template <int OFF = 0>
 __device__ __forceinline__ uint32_t asm_lds_read_u16(uint32_t addr) {
     uint32_t v;
     asm volatile("ds_read_u16 %0, %1 offset:%2" : "=v"(v) : "v"(addr), "n"(OFF) : "memory");
@@ -230,6 +246,13 @@ __device__ __forceinline__ void asm_global_load_lds_b128(const void* gaddr, uint
                  : "v"(gaddr), "s"(lds_base)
                  : "memory", "m0");
 }
+// the 4-byte form: lane i's 4 bytes land at lds_base + 4 * i
+__device__ __forceinline__ void asm_global_load_lds_b32(const void* gaddr, uint32_t lds_base) {
+    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dword %0, off"
+                 :
+                 : "v"(gaddr), "s"(lds_base)
+                 : "memory", "m0");
+}
 #pragma clang diagnostic pop
 
 // The buffer-addressed form of the same direct load: lane i's 16 bytes at
@@ -247,6 +270,13 @@ __device__ __forceinline__ i32x4 raw_rsrc(const void* base, uint32_t bytes) {
 #pragma clang diagnostic ignored "-Winline-asm"
 __device__ __forceinline__ void asm_buffer_load_lds_b128(i32x4 rsrc, uint32_t voff, uint32_t lds_base) {
     asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, 0 offen lds"
+                 :
+                 : "v"(voff), "s"(rsrc), "s"(lds_base)
+                 : "memory", "m0");
+}
+// the 4-byte form: lane i's 4 bytes land at lds_base + 4 * i
+__device__ __forceinline__ void asm_buffer_load_lds_b32(i32x4 rsrc, uint32_t voff, uint32_t lds_base) {
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tbuffer_load_dword %0, %1, 0 offen lds"
                  :
                  : "v"(voff), "s"(rsrc), "s"(lds_base)
                  : "memory", "m0");

@@ -38,7 +38,6 @@
 
 #include <cstdio>
 #include <cstdlib>
-#include <type_traits>
 
 namespace mvlm {
 
@@ -79,15 +78,6 @@ struct GemmArgs {
     // store writes them
     int vec_c, vec_ws;
 };
-
-// f(std::integral_constant<int, 0>{}), ..., f(std::integral_constant<int, N - 1>{})
-template <int N, int I = 0, class F>
-__device__ __forceinline__ void static_for(F&& f) {
-    if constexpr (I < N) {
-        f(std::integral_constant<int, I>{});
-        static_for<N, I + 1>(f);
-    }
-}
 
 // fp32 partial of 4 consecutive columns (n_left of them below N; the row
 // starts 16-byte aligned)

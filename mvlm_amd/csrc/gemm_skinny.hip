@@ -16,41 +16,55 @@
 //    weights: acc += d * (sum over the block), as in the M = 1 kernel;
 //  * Q4_0 multiplies the raw nibbles c and subtracts 8 * (sum of x over the
 //    block), that sum coming from one more product of the split x with a
-//    ones operand, shared by the block's row groups.
-// One MFMA covers 16 weight rows x one block of 32 weights x 16 rows of X
-// (rows m >= M are zero).  Operand layout of v_mfma_f32_16x16x32_bf16: lane l
-// supplies A[l%16][8*(l/16) .. +7] and B[8*(l/16) .. +7][l%16]; accumulator
-// register i of lane l is D[4*(l/16) + i][l%16].  Here A = X (row m = l%16)
-// and B = w^T (weight row n0 + l%16), so lane l reads 8 consecutive codes of
-// its weight row: Q8_0 bytes 8q..8q+7 of the block (q = l/16), Q4_0 the low
-// (q < 2) or high (q >= 2) nibbles of bytes 8*(q&1)..+7 (byte j holds weights
-// j and j + 16).
+//    ones operand.
+// One MFMA covers 16 weight rows x one block of 32 weights x 16 rows of X.
+// Operand layout of v_mfma_f32_16x16x32_bf16: lane l supplies
+// A[l%16][8*(l/16) .. +7] and B[8*(l/16) .. +7][l%16]; accumulator register i
+// of lane l is D[4*(l/16) + i][l%16].  Here A = X (row m = l%16) and B = w^T
+// (weight row n0 + l%16).  The k order inside a block is free as long as both
+// operands share it: Q8_0 lanes take bytes 8q..8q+7 of the block (q = l/16);
+// Q4_0 lanes take its bytes 4q..4q+3, i.e. weights 4q..4q+3 (low nibbles) and
+// 16+4q..16+4q+3 (high nibbles).
 //
-// A block of NW waves owns R groups of 16 weight rows; wave w takes the w-th
-// NW-th of the K blocks and walks it in steps of G blocks (4, or 2 with four
-// row groups).  Codes do not go straight to registers: in the MFMA layout a
-// wave instruction would touch 16 rows x 32 bytes (16 partly used lines), and
-// such loads ran at a fraction of HBM speed whatever the arithmetic.  Instead
-// each step's codes of the wave's rows (16R rows x 32G bytes for Q8_0, x 16G
-// bytes for Q4_0) are copied
-// into the wave's own LDS slot with direct 16-byte loads (1 KiB contiguous
-// per instruction), double-buffered, and read back per lane (ds_read_b64).
-// The 16-byte pieces of each LDS row are XOR-swizzled with row bits so the
-// 16 lanes of a read hit distinct banks.  The block's scales (all K) are
-// staged once per block.  X goes straight to registers, one step ahead:
-// each block's X registers are refilled for the next step as soon as that
-// block's products are issued.
-// The NW partial tiles meet in LDS.  Splitting K over blocks instead (to give
-// small-N problems more blocks) would need a cross-block combine; on MI355X a
-// device-scope release fence per block costs ~90 ns, serialized (1024 blocks:
-// ~96 us), so small N gets 16-wave blocks instead.
+// X stays in registers.  A workgroup of 8 waves spans up to 64 blocks of K (a
+// chunk of 2048 weights; longer rows are cut into equal chunks), eight blocks a
+// wave: the wave loads and splits its 16 x 256 slice of X once (96 registers)
+// and then streams the same columns of one 16-row group of the weight after
+// another.  Reading X again for every row group, as a kernel with waves of
+// independent rows does, costs 4 * M * K bytes per row group, 14 times the
+// Q4_0 codes of the group at M = 16, and that traffic (from L2, through the
+// CU's one vector cache) set the time.  The waves' partial tiles meet in LDS
+// after every four row groups.  One workgroup per CU; the row groups of a launch
+// are dealt out so that it takes one round (up to 14 row groups per workgroup).
+//
+// Against a kernel whose workgroups each read all of X for one to four row
+// groups, a Phi-1.5 step (49 grouped launches) of M = 16 went 831 -> 680 us
+// (Q4_0) and 867 -> 720 us (Q8_0), of M = 8 785 -> 626 and 806 -> 672 us, its LM
+// head 37 -> 22 and 38 -> 27 us.  What bounds a launch now (time stamps of the
+// M = 16 QKV + fc1 launch, 10.5 us): 128 KiB of X into every CU and its split,
+// 5 us before the first products, then 0.8 us (Q4_0, vector ALU and matrix core
+// in turn) to 1.2 us (Q8_0, HBM) per row group.  Sixteen waves of four blocks
+// each spend longer in the barriers (Q4_0 M = 16 707 us, Q8_0 691 us); codes
+// requested before X, with deeper rings, delay X by more than they gain (697
+// and 822 us).
+//
+// Codes go to the wave's own LDS ring with direct 16-byte loads, several row
+// groups ahead, and are read back per lane (loading the MFMA layout straight
+// from HBM, 16 rows x 32 bytes per instruction, ran at ~1 TB/s whatever the
+// arithmetic).  The workgroup's scales are staged once.
+//
+// Rows of more than one chunk (K > 2048): a workgroup takes one chunk of its
+// rows and writes its sums to the device workspace, and a second launch adds
+// the chunks in order and applies the epilogue.  Without workspace a workgroup
+// walks the chunks itself, reloading X for every row group.  The
+// order of every sum depends on K alone, so an output has the same bits in a
+// single and in a grouped call.
 #include "common.h"
 #include "device_math.h"
 
 #include <algorithm>
 
 namespace mvlm {
-
 
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8v;
 
@@ -77,32 +91,27 @@ __device__ __forceinline__ void split3(const float (&x)[8], u32x4& p1, u32x4& p2
     }
 }
 
-// 8 small integers (exact in bf16) from 8 code bytes / nibbles.  Q4_0 gives
-// the raw nibbles c (0..15): masked into bytes, one byte-to-float conversion
-// each; the -8 of (c - 8) is applied per block through the block sums of x.
+// A lane's 8 codes of a block as bf16 (small integers, exact).  Q4_0: raw is
+// one dword, the result the raw nibbles c (0..15), low nibbles first; the -8
+// of (c - 8) comes in through the block sums of x.  A nibble in a byte is the
+// fp8 (E4M3) number c * 2^-9, denormal or not, so one scaled conversion makes
+// two of them.
 template <bool Q4>
-__device__ __forceinline__ u32x4 codes_to_bf16(u32x2 raw, int q) {
-    float v[8];
+__device__ __forceinline__ u32x4 codes_to_bf16(u32x2 raw) {
+    u32x4 out;
     if constexpr (Q4) {
-        const int shift = (q >> 1) * 4;
-        uint32_t lo = (raw[0] >> shift) & 0x0F0F0F0Fu, hi = (raw[1] >> shift) & 0x0F0F0F0Fu;
-        // opaque to the compiler, which would otherwise fold each byte's
-        // shift and mask into a bit-field extract per code in front of the
-        // conversion; this way v_cvt_f32_ubyte{0..3} read the bytes directly
-        asm_pin(lo);
-        asm_pin(hi);
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            v[j] = (float)((lo >> (8 * j)) & 0xFFu);
-            v[4 + j] = (float)((hi >> (8 * j)) & 0xFFu);
-        }
+        const uint32_t lo = raw[0] & 0x0F0F0F0Fu, hi = (raw[0] >> 4) & 0x0F0F0F0Fu;
+        out[0] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(lo, 512.0f, false));
+        out[1] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(lo, 512.0f, true));
+        out[2] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(hi, 512.0f, false));
+        out[3] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(hi, 512.0f, true));
     } else {
+        float v[8];
 #pragma unroll
         for (int j = 0; j < 8; ++j) v[j] = (float)(int8_t)(raw[j >> 2] >> (8 * (j & 3)));
-    }
-    u32x4 out;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) out[j] = pack_hi16(v[2 * j], v[2 * j + 1]);
+        for (int j = 0; j < 4; ++j) out[j] = pack_hi16(v[2 * j], v[2 * j + 1]);
+    }
     return out;
 }
 
@@ -111,31 +120,42 @@ __device__ __forceinline__ f32x4 mfma16(u32x4 a, u32x4 b, f32x4 c) {
                                                    0, 0, 0);
 }
 
-constexpr size_t SKINNY_LDS_MAX = 160 * 1024;
+// Barrier that orders the workgroup's LDS accesses and leaves loads from
+// memory in flight (__syncthreads() would wait for all of them).
+__device__ __forceinline__ void block_sync() {
+    asm_wait_lgkmcnt<0>();
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+}
 
-// G = K blocks per step.
-template <bool Q4, int G>
+constexpr int SK_WAVES = 8;                           // waves of a workgroup
+constexpr int SK_KB = 8;                              // blocks of K per wave, at most
+constexpr int SK_CHUNK = SK_WAVES * SK_KB;            // blocks of K per chunk, at most
+constexpr int SK_MAX_RG = 14;                         // row groups per workgroup, at most
+constexpr int SK_BATCH = 4;                           // row groups whose partial tiles meet at one barrier
+// a row's staged scales of one chunk: 64 fp16 and one more where the chunk
+// starts at an odd block, in dwords
+constexpr int SK_SCALE_DW = SK_CHUNK / 2 + 2;
+constexpr int SK_SCALE_ROWS = 16 * SK_SCALE_DW * 4;   // bytes of a row group's
+constexpr int SK_PART_BYTES = SK_BATCH * SK_WAVES * 1024;
+constexpr int SK_EP_LOADS = 5;                        // epilogue operands of a thread's two outputs
+constexpr int SK_EP_BYTES = SK_EP_LOADS * SK_WAVES * 256;
+
+template <bool Q4>
 struct SkinnyLayout {
     static constexpr int BB = Q4 ? 16 : 32;           // code bytes per block per row
-    static constexpr int CB = G * BB;                 // code bytes per row per step (32 / 64 / 128)
-    static constexpr int P = CB / 16;                 // 16-byte pieces per row per step
+    static constexpr int CB = SK_KB * BB;             // code bytes per row per wave (128 / 256)
+    static constexpr int P = CB / 16;                 // 16-byte pieces per row
     static constexpr int RPI = 64 / P;                // rows per direct-load instruction
-    static constexpr int RSH = CB == 128 ? 1 : CB == 64 ? 2 : 3;   // 1 << RSH rows per 256 bytes
-    static_assert(CB == 32 || CB == 64 || CB == 128, "step rows of 32, 64 or 128 bytes");
-    // physical piece of logical piece p in LDS row r: the 16 rows of a read
-    // land on distinct banks
-    __device__ static int piece(int p, int r) { return p ^ ((r >> RSH) & (P - 1)); }
+    static constexpr int NDMA = 16 / RPI;             // direct loads per row group
+    static constexpr int SLOT = 16 * CB;              // bytes of one row group's codes
+    static constexpr int DEPTH = Q4 ? 4 : 2;          // row groups in flight: 64 KiB per CU
+    static constexpr int LDS = SK_PART_BYTES + SK_EP_BYTES + SK_MAX_RG * SK_SCALE_ROWS + SK_WAVES * DEPTH * SLOT;
+    // Physical piece of logical piece p in LDS row r: XOR-swizzled with row
+    // bits so the rows of a read land on distinct banks.
+    __device__ static int piece(int p, int r) { return p ^ (Q4 ? (r >> 1) & 7 : r & 15); }
 };
-
-// LDS bytes of a block: the scales of its rows (all K), then two code slots
-// per wave; the partial tiles of the final combine reuse the slots.
-template <bool Q4, int R, int NW, int G>
-__host__ __device__ constexpr int skinny_slot_bytes() { return 16 * R * SkinnyLayout<Q4, G>::CB; }
-template <bool Q4, int R, int NW, int G>
-static size_t skinny_lds_bytes(int K) {
-    const size_t scale_region = ((size_t)16 * R * (K / 32) * 2 + 255) / 256 * 256;
-    return scale_region + (size_t)NW * 2 * skinny_slot_bytes<Q4, R, NW, G>();
-}
+static_assert(SkinnyLayout<true>::LDS <= 160 * 1024 && SkinnyLayout<false>::LDS <= 160 * 1024, "LDS of a CU");
 
 // One problem of a (possibly grouped) launch: Y[M][N] = X[M][K] w^T.
 struct SkinnyProblem {
@@ -143,372 +163,408 @@ struct SkinnyProblem {
     const uint8_t* codes;
     const uint16_t* scales;
     float* Y;
-    int64_t ld;
-    int N, K;
-    int block_begin;               // first block of this problem in the grid
+    float* part;                   // [chunks][M][N] sums of the chunks, or null: one workgroup walks them
+    uint32_t ld;                   // code bytes per row
+    int N, nb;                     // rows, blocks of K
+    int chunks, chunk_blocks;      // chunks of K and blocks per chunk (the last may have fewer)
+    uint32_t chunk_div;            // ceil(2^32 / chunks): b / chunks = b * chunk_div >> 32
+    int rows;                      // row groups per workgroup
     int ep_on;
     Epilogue ep;
 };
 constexpr int SKINNY_MAX_GROUP = 8;
 struct SkinnyGroup {
-    SkinnyProblem p[SKINNY_MAX_GROUP];
     int count, M;
+    int block_begin[SKINNY_MAX_GROUP];   // first workgroup of each problem in the grid
+    SkinnyProblem p[SKINNY_MAX_GROUP];
 };
 
-// XS: odd rows read their X halves in swapped order (M > 8, below).
-template <bool Q4, int R, int NW, int G, bool XS>
-__global__ __launch_bounds__(64 * NW, 4) void gemm_skinny_kernel(const SkinnyGroup g) {
-    using L = SkinnyLayout<Q4, G>;
-    constexpr int ROWS = 16 * R;
-    constexpr int SLOT = skinny_slot_bytes<Q4, R, NW, G>();
-    constexpr int NDMA = ROWS / L::RPI;               // direct loads per step
-    static_assert(NDMA <= 63, "direct loads of one step must fit vmcnt");
-    static_assert(2 * SLOT >= R * 1024, "the partial tiles of the combine must fit the code slots");
-    extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+template <bool Q4>
+__global__ __launch_bounds__(64 * SK_WAVES) void gemm_skinny_kernel(const SkinnyGroup g) {
+    using L = SkinnyLayout<Q4>;
+    extern __shared__ __attribute__((aligned(256))) uint8_t lds[];
+    float* const part = reinterpret_cast<float*>(lds);
 
-    int pi = 0;                                       // blocks are dealt to the problems in order
+    int pi = 0;                                       // workgroups are dealt to the problems in order
 #pragma unroll
     for (int i = 1; i < SKINNY_MAX_GROUP; ++i)
-        if (i < g.count && (int)blockIdx.x >= g.p[i].block_begin) pi = i;
+        if (i < g.count && (int)blockIdx.x >= g.block_begin[i]) pi = i;
     const SkinnyProblem& P = g.p[pi];
-    const float* __restrict__ X = P.X;
-    const uint8_t* __restrict__ codes = P.codes;
-    const uint16_t* __restrict__ scales = P.scales;
-    float* __restrict__ Y = P.Y;
-    const int M = g.M, N = P.N, K = P.K;
-    const int64_t ld = P.ld;
-
+    const int M = g.M, N = P.N, nb = P.nb, chunks = P.chunks, chunk_blocks = P.chunk_blocks, rows = P.rows;
+    const uint32_t ld = P.ld, chunk_div = P.chunk_div;
+    float* const cpart = P.part;
+    const float* const X = P.X;
+    const uint8_t* const codes = P.codes;
+    const uint16_t* const scales = P.scales;
+    const bool ep_on = P.ep_on && !cpart;
+    // one round trip for the fields, before anything waits for one of them
+    asm volatile("" ::"s"(N), "s"(nb), "s"(chunks), "s"(chunk_blocks), "s"(rows), "s"(ld), "s"(chunk_div), "s"(cpart),
+                 "s"(X), "s"(codes), "s"(scales));
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int l16 = lane & 15, q = lane >> 4;
-    const int n0 = ((int)blockIdx.x - P.block_begin) * ROWS;
-    const int nb = K >> 5;
-    const int per = (nb + NW - 1) / NW;
-    const int b0 = wave * per, b1 = min(b0 + per, nb);
-    const int steps = b1 > b0 ? (b1 - b0 + G - 1) / G : 0;
-    const int64_t row_bytes = (int64_t)nb * L::BB;
 
-    // scales of rows n0 .. n0+ROWS-1 (contiguous in the scale array) with
-    // 4-byte direct loads (a direct load writes lane i's data at base + 4i
-    // whatever its width, so 2-byte loads would not pack).  Reads are clamped
-    // to the last whole dword of the array (the allocation pads it); rows
-    // past N read stale scales and are never stored.
-    const int scale_bytes = ROWS * nb * 2;
-    const int scale_region = (scale_bytes + 255) / 256 * 256;
-    uint8_t* slots = lds + scale_region + wave * 2 * SLOT;
-    const int64_t s_first = (int64_t)n0 * nb * 2, s_last = (((int64_t)N * nb * 2 - 1) & ~(int64_t)3);
-    const uint8_t* scale_bytes_ptr = reinterpret_cast<const uint8_t*>(scales);
-    for (int piece = wave; piece * 256 < scale_bytes; piece += NW) {
-        const int64_t off = min(s_first + piece * 256 + lane * 4, s_last);
-        __builtin_amdgcn_global_load_lds(scale_bytes_ptr + off, (lds_void*)(lds + piece * 256), 4, 0, 0);
-    }
+    // this workgroup's row groups [rg0, rg0 + units) and chunks [c_begin, c_end)
+    const int bid = (int)blockIdx.x - g.block_begin[pi];
+    const bool split = cpart != nullptr;
+    const int range = split && chunks > 1 ? (int)__umulhi((uint32_t)bid, chunk_div) : bid;
+    const int c_begin = split ? bid - range * chunks : 0, c_end = split ? c_begin + 1 : chunks;
+    const int rg0 = range * rows;
+    const int units = min(rows, (N + 15) / 16 - rg0);
+    const int n0 = 16 * rg0;
 
-    // one step's direct loads: this wave's code rows into slot (step & 1).
-    // Codes and X are read through buffer descriptors (32-bit offsets; the
-    // host keeps both below 2 GiB on this path).
-    const __amdgpu_buffer_rsrc_t crs = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<uint8_t*>(codes), 0, (int)min((int64_t)N * ld, (int64_t)0x7FFFFFFF), 0x00020000);
-    const i32x4 xrs = raw_rsrc(X, (uint32_t)((int64_t)M * K * 4));
-    const uint32_t xrow = (uint32_t)(((int64_t)min(l16, M - 1) * K + 8 * q) * 4);
+    // Codes, scales and X are read through buffer descriptors (32-bit offsets;
+    // the host keeps all three below 2 GiB).
+    const i32x4 crs = raw_rsrc(codes, (uint32_t)N * ld);
+    const i32x4 srs = raw_rsrc(scales, ((uint32_t)N * (uint32_t)nb * 2 + 3) & ~3u);   // the allocation is padded
+    const i32x4 xrs = raw_rsrc(X, (uint32_t)M * (uint32_t)nb * 128);
+    const uint32_t ep_base = lds_offset(lds) + SK_PART_BYTES + (uint32_t)(wave * SK_EP_LOADS * 256);
+    const uint32_t scale_base = lds_offset(lds) + SK_PART_BYTES + SK_EP_BYTES;
+    const uint32_t ring = scale_base + SK_MAX_RG * SK_SCALE_ROWS + (uint32_t)(wave * L::DEPTH * L::SLOT);
+    // lanes whose X row is past M read row M - 1: they only feed output rows
+    // m >= M, which are never stored
+    const int xm = min(l16, M - 1);
+    // Lanes of odd rows load their two X pieces in swapped order, so the 16
+    // lanes of a quarter-wave (16 rows, one q) read two different offsets of
+    // their lines instead of one (the vector cache serves many lines at one
+    // offset one after another).
+    const bool xodd = (xm & 1) != 0;
+    const int x0 = Q4 ? 4 * q : 8 * q, x1 = Q4 ? 16 + 4 * q : 8 * q + 4;
     const int dma_row = lane / L::P, dma_piece = lane % L::P;
-    auto issue_codes = [&](int step, int slot_idx) {
-        const int kb = b0 + step * G;
-        uint8_t* slot = slots + slot_idx * SLOT;
-#pragma unroll
-        for (int t = 0; t < NDMA; ++t) {
-            const int r = t * L::RPI + dma_row;
-            const int64_t row = min(n0 + r, N - 1);
-            const int64_t off = min((int64_t)kb * L::BB + 16 * L::piece(dma_piece, r), row_bytes - 16);
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(crs, (lds_void*)(slot + t * 1024), 16, (int)(row * ld + off), 0, 0, 0);
-        }
-    };
-    // X of block g of one step into registers.  A lane's 8 floats are two
-    // 16-byte halves of its row's 128-byte line.  With XS, lanes of odd rows
-    // load the second half first, so the 16 lanes of a quarter-wave (16 rows,
-    // one q) read two different offsets of their lines instead of one (the
-    // vector cache serves many lines at one offset one after another: the
-    // Q4_0 M = 16 step 827 -> 766 us, Q8_0 M = 16 895 -> 783 us, Q8_0 M = 12
-    // 797 -> 760 us).  The halves are swapped back where the block is split;
-    // at M <= 8 (at most 8 distinct lines) those selects cost more than the
-    // conflicts (Q4_0 M = 5 707 -> 725 us), so XS is off there.
-    const bool xodd = XS && (min(l16, M - 1) & 1) != 0;   // parity of the row actually read
-    const int xsw = xodd ? 4 : 0;
-    auto load_x = [&](int step, int g, u32x4 (&xg)[2]) {
-        const int bb = min(b0 + step * G + g, nb - 1);
-        xg[0] = asm_buffer_load_b128(xrs, xrow + (uint32_t)(32 * bb + xsw) * 4);
-        xg[1] = asm_buffer_load_b128(xrs, xrow + (uint32_t)(32 * bb + 4 - xsw) * 4);
+
+    // The waves sum the partial tiles of a batch of row groups and store them:
+    // waves 2 k and 2 k + 1 those of row group k of the batch, a lane the
+    // outputs (om, l16) and (om + 4, l16).  Their epilogue operands come in by
+    // direct 4-byte loads, a batch ahead (absent ones repeat a scale).
+    const int om = 8 * (wave & 1) + q, duty = wave >> 1;
+    const bool ep = ep_on && 8 * (wave & 1) < M;
+    auto issue_ep = [&](int u) {
+        const int n = min(n0 + 16 * u + l16, N - 1);
+        const float* none = reinterpret_cast<const float*>(scales);
+        const int64_t i0 = (int64_t)min(om, M - 1) * N + n, i1 = (int64_t)min(om + 4, M - 1) * N + n;
+        const float *b = (const float*)P.ep.bias, *m = (const float*)P.ep.mul, *r = (const float*)P.ep.res;
+        const uint32_t dst = __builtin_amdgcn_readfirstlane(ep_base);
+        asm_global_load_lds_b32(b ? b + n : none, dst);
+        asm_global_load_lds_b32(m ? m + i0 : none, dst + 256);
+        asm_global_load_lds_b32(m ? m + i1 : none, dst + 512);
+        asm_global_load_lds_b32(r ? r + i0 : none, dst + 768);
+        asm_global_load_lds_b32(r ? r + i1 : none, dst + 1024);
     };
 
-    // Lanes whose X row is past M (clamped to row M - 1 above) only feed
-    // output rows m >= M, which are never stored.
-    f32x4 acc[R];
-#pragma unroll
-    for (int r = 0; r < R; ++r) acc[r] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-    u32x4 xr[G][2];                                   // X of the current step
-    if (steps > 0) {
-        issue_codes(0, 0);
-#pragma unroll
-        for (int g = 0; g < G; ++g) load_x(0, g, xr[g]);
-    }
-    asm_wait_vmcnt<0>();
-    __syncthreads();                                  // the staged scales of every wave
+    u32x4 xp[SK_KB][3];                               // the wave's slice of X in three bf16 parts
+    f32x4 sx[SK_KB];                                  // Q4_0: -8 times its block sums
+    f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
 
-    // LDS reads go through inline asm (the compiler would otherwise wait for
-    // every in-flight direct load, including the next step's, before them)
-    const uint32_t lds_base = lds_offset(lds);
-    // Block g's X registers are refilled with the next step's X as soon as
-    // its products are issued, so those loads overlap this step's work.  The
-    // body is straight-line code (blocks past the wave's range get a zero
-    // scale, the refill is unconditional and clamped in bounds): with no
-    // branches the loop-carried X registers need no copies, which would read
-    // them while their loads are still in flight.
-    auto compute = [&](int step, u32x4 (&xr)[G][2], auto refill) {
-        const int kb = b0 + step * G;
-        const uint32_t slot = lds_offset(slots + (step & 1) * SLOT);
-        u32x2 raw[G][R];
-        uint32_t dh[G][R];
+    // Row groups u0..u1 of chunk c.  A workgroup with one chunk has one such
+    // segment; one that walks several takes each row group through all of them.
+    const int span = c_end - c_begin == 1 ? units : 1;
+    for (int u0 = 0; u0 < units; u0 += span) {
+        const int u1 = min(u0 + span, units);
+        for (int c = c_begin; c < c_end; ++c) {
+            const int cb0 = c * chunk_blocks, cb = min(chunk_blocks, nb - cb0);
+            const int per = (cb + SK_WAVES - 1) / SK_WAVES;
+            const int cnt = max(0, min(per, cb - wave * per));   // this wave's blocks
+            const int b0 = cb0 + wave * per;
+            const bool last_chunk = c + 1 == c_end;
+            if (u0 > 0 || c > c_begin) block_sync();             // the scales are about to be replaced
+
+            // a lane's byte of the codes for each direct load of row group 0,
+            // and its last one in bounds (rows past N repeat row N - 1)
+            uint32_t voff[L::NDMA], vmax[L::NDMA];
 #pragma unroll
-        for (int g = 0; g < G; ++g) {
-            const int lpiece = Q4 ? g : 2 * g + (q >> 1);
-            const int bb = min(kb + g, b1 - 1);
-#pragma unroll
-            for (int rr = 0; rr < R; ++rr) {
-                const int r = 16 * rr + l16;
-                raw[g][rr] = asm_lds_read_b64(slot + r * L::CB + 16 * L::piece(lpiece, r) + 8 * (q & 1));
-                dh[g][rr] = asm_lds_read_u16(lds_base + 2 * (r * nb + bb));
+            for (int t = 0; t < L::NDMA; ++t) {
+                const int r = t * L::RPI + dma_row;
+                const uint32_t off = (uint32_t)min(b0 * L::BB + 16 * L::piece(dma_piece, r), nb * L::BB - 16);
+                voff[t] = (uint32_t)(n0 + r) * ld + off;
+                vmax[t] = (uint32_t)(N - 1) * ld + off;
             }
-        }
-        asm_wait_lgkmcnt<0>();
+            auto issue = [&](int u, int slot) {
+                const uint32_t dst = __builtin_amdgcn_readfirstlane(ring + (uint32_t)(slot * L::SLOT));
 #pragma unroll
-        for (int g = 0; g < G; ++g)
+                for (int t = 0; t < L::NDMA; ++t)
+                    asm_buffer_load_lds_b128(crs, min(voff[t] + (uint32_t)(16 * u) * ld, vmax[t]), dst + t * 1024);
+            };
+
+            // The scales, the first epilogue operands, X, then the first row
+            // groups of codes (past the last one, and in waves without blocks,
+            // the clamped addresses repeat loads: no branch may stand between
+            // the X loads and the wait for them, where the compiler could move
+            // their registers).  Scales: dwords of the rows' scales of this
+            // chunk, from the dword its first block lies in; past the array
+            // they are clamped to its last dword.
+            {
+                const int total = (u1 - u0) * 16 * SK_SCALE_DW;
+                const uint32_t last = ((uint32_t)N * (uint32_t)nb * 2 - 1) & ~3u;
+                for (int i = wave * 64; i < total; i += 64 * SK_WAVES) {
+                    const uint32_t e = (uint32_t)min(i + lane, total - 1), r = e / SK_SCALE_DW, dw = e - r * SK_SCALE_DW;
+                    const uint32_t row = min((uint32_t)(n0 + 16 * u0) + r, (uint32_t)(N - 1));
+                    const uint32_t off = (((row * (uint32_t)nb + (uint32_t)cb0) * 2) & ~3u) + 4 * dw;
+                    asm_buffer_load_lds_b32(srs, min(off, last),
+                                            __builtin_amdgcn_readfirstlane(scale_base + 4u * (uint32_t)i));
+                }
+            }
+            if (ep && last_chunk && u0 + duty < u1) issue_ep(u0 + duty);
+            u32x4 xr[SK_KB][2];
 #pragma unroll
-            for (int rr = 0; rr < R; ++rr) {
-                asm_pin(raw[g][rr]);
-                asm_pin(dh[g][rr]);
+            for (int j = 0; j < SK_KB; ++j) {
+                const uint32_t base = (uint32_t)(xm * nb + min(b0 + j, nb - 1)) * 128u;
+                xr[j][0] = asm_buffer_load_b128(xrs, base + 4u * (uint32_t)(xodd ? x1 : x0));
+                xr[j][1] = asm_buffer_load_b128(xrs, base + 4u * (uint32_t)(xodd ? x0 : x1));
             }
 #pragma unroll
-        for (int g = 0; g < G; ++g) {
-            const bool live = kb + g < b1;            // uniform over the wave
-            float x[8];
+            for (int d = 0; d < L::DEPTH; ++d) issue(min(u0 + d, u1 - 1), d);
+            asm_wait_vmcnt<L::DEPTH * L::NDMA>();
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                x[j] = __uint_as_float(xodd ? xr[g][1][j] : xr[g][0][j]);
-                x[4 + j] = __uint_as_float(xodd ? xr[g][0][j] : xr[g][1][j]);
-            }
-            u32x4 p1, p2, p3;
-            split3(x, p1, p2, p3);
-            f32x4 sx = {0.0f, 0.0f, 0.0f, 0.0f};      // Q4_0: sum of the block's x per X row
-            if constexpr (Q4) {
-                const u32x4 ones = {0x3F803F80u, 0x3F803F80u, 0x3F803F80u, 0x3F803F80u};   // bf16 1.0 pairs
-                sx = mfma16(p1, ones, sx);
-                sx = mfma16(p2, ones, sx);
-                sx = mfma16(p3, ones, sx);
+            for (int j = 0; j < SK_KB; ++j) {
+                asm_pin(xr[j][0]);
+                asm_pin(xr[j][1]);
+                if (j >= cnt) xr[j][0] = xr[j][1] = u32x4{0u, 0u, 0u, 0u};   // blocks past the wave's range
             }
 #pragma unroll
-            for (int rr = 0; rr < R; ++rr) {
-                const u32x4 w = codes_to_bf16<Q4>(raw[g][rr], q);
-                f32x4 c = {0.0f, 0.0f, 0.0f, 0.0f};
-                c = mfma16(p1, w, c);
-                c = mfma16(p2, w, c);
-                c = mfma16(p3, w, c);
+            for (int j = 0; j < SK_KB; ++j) {
+                float x[8];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    x[e] = __uint_as_float(xodd ? xr[j][1][e] : xr[j][0][e]);
+                    x[4 + e] = __uint_as_float(xodd ? xr[j][0][e] : xr[j][1][e]);
+                }
+                split3(x, xp[j][0], xp[j][1], xp[j][2]);
+                sx[j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
                 if constexpr (Q4) {
+                    const u32x4 ones = {0x3F803F80u, 0x3F803F80u, 0x3F803F80u, 0x3F803F80u};   // bf16 1.0 pairs
+                    sx[j] = mfma16(xp[j][0], ones, sx[j]);
+                    sx[j] = mfma16(xp[j][1], ones, sx[j]);
+                    sx[j] = mfma16(xp[j][2], ones, sx[j]);
 #pragma unroll
-                    for (int i = 0; i < 4; ++i) c[i] = __builtin_fmaf(-8.0f, sx[i], c[i]);
-                }
-                const float d = live ? f16_bits_to_f32((uint16_t)dh[g][rr]) : 0.0f;
-#pragma unroll
-                for (int i = 0; i < 4; ++i) acc[rr][i] = __builtin_fmaf(d, c[i], acc[rr][i]);
-            }
-            if constexpr (decltype(refill)::value) load_x(step + 1, g, xr[g]);
-        }
-    };
-
-    // Per step: the next step's codes; waiting until only those remain in
-    // flight covers this step's X (requested during the previous step, or
-    // before the loop) and codes.  The last step is peeled: nothing is
-    // requested for it, and it waits for everything.  X goes through
-    // untracked loads, so the compiler adds no waits of its own.
-    for (int step = 0; step + 1 < steps; ++step) {
-        issue_codes(step + 1, (step + 1) & 1);
-        asm_wait_vmcnt<NDMA>();
-#pragma unroll
-        for (int g = 0; g < G; ++g) {
-            asm_pin(xr[g][0]);
-            asm_pin(xr[g][1]);
-        }
-        compute(step, xr, std::true_type{});
-    }
-    asm_wait_vmcnt<0>();
-    if (steps > 0) {
-#pragma unroll
-        for (int g = 0; g < G; ++g) {
-            asm_pin(xr[g][0]);
-            asm_pin(xr[g][1]);
-        }
-        compute(steps - 1, xr, std::false_type{});
-    }
-
-    // combine the NW partial tiles (reusing the code slots)
-    __syncthreads();
-    f32x4* part = reinterpret_cast<f32x4*>(lds + scale_region);
-#pragma unroll
-    for (int r = 0; r < R; ++r) part[(wave * R + r) * 64 + lane] = acc[r];
-    __syncthreads();
-    if (wave < R) {                                   // wave r sums row group r
-        const int r = wave;
-        f32x4 sum = part[r * 64 + lane];
-#pragma unroll
-        for (int w = 1; w < NW; ++w) {
-            const f32x4 t = part[(w * R + r) * 64 + lane];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) sum[i] += t[i];
-        }
-        const int n = n0 + 16 * r + l16;
-        if (n < N) {
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const int m = 4 * q + i;
-                if (m < M) {
-                    const int64_t idx = (int64_t)m * N + n;
-                    Y[idx] = P.ep_on ? apply_epilogue(P.ep, sum[i], idx, n) : sum[i];
+                    for (int i = 0; i < 4; ++i) sx[j][i] *= -8.0f;
                 }
             }
+            if (cnt == 0) asm_wait_vmcnt<0>();        // nothing waits for this wave's repeats below
+            block_sync();                             // the scales of every wave have landed
+
+            // a lane's scales: row l16 of the row group, from the wave's first
+            // block; its codes of block j: a dword (Q4_0) or two (Q8_0)
+            const uint32_t s_lane = scale_base + (uint32_t)(l16 * SK_SCALE_DW * 4 + 2 * (((l16 * nb + cb0) & 1) + wave * per));
+            const uint32_t c_lane = ring + (uint32_t)(l16 * L::CB + 16 * L::piece(Q4 ? 0 : q >> 1, l16) +
+                                                      (Q4 ? 4 * q : 8 * (q & 1)));
+            // extra: epilogue loads of the wave issued after this row group's codes
+            auto unit = [&](int u, int slot, bool extra) {
+                if (cnt == 0) return;
+                if (u + L::DEPTH > u1) asm_wait_vmcnt<0>();
+                else if (extra) asm_wait_vmcnt<(L::DEPTH - 1) * L::NDMA + SK_EP_LOADS>();
+                else asm_wait_vmcnt<(L::DEPTH - 1) * L::NDMA>();
+                const uint32_t src = c_lane + (uint32_t)(slot * L::SLOT);
+                const uint32_t ssrc = s_lane + (uint32_t)((u - u0) * SK_SCALE_ROWS);
+                u32x2 raw[SK_KB];
+                uint32_t dh[SK_KB];
+                static_for<SK_KB>([&](auto J) {
+                    constexpr int j = decltype(J)::value;
+                    // a row's slot is aligned to its size: XOR moves between pieces
+                    if constexpr (Q4) raw[j][0] = asm_lds_read_b32(src ^ (uint32_t)(16 * j));
+                    else raw[j] = asm_lds_read_b64(src ^ (uint32_t)(32 * j));
+                    dh[j] = asm_lds_read_u16<2 * j>(ssrc);
+                });
+                asm_wait_lgkmcnt<0>();
+#pragma unroll
+                for (int j = 0; j < SK_KB; ++j) {
+                    asm_pin(raw[j]);
+                    asm_pin(dh[j]);
+                }
+                if (u + L::DEPTH < u1) issue(u + L::DEPTH, slot);
+                // four blocks at a time (those past the wave's range: X and d are zero)
+#pragma unroll
+                for (int h = 0; h < SK_KB; h += 4) {
+                    if (h >= cnt) break;
+                    f32x4 p[4];
+                    u32x4 w[4];
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) w[j] = codes_to_bf16<Q4>(raw[h + j]);
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) p[j] = mfma16(xp[h + j][0], w[j], sx[h + j]);
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) p[j] = mfma16(xp[h + j][1], w[j], p[j]);
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) p[j] = mfma16(xp[h + j][2], w[j], p[j]);
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) {
+                        const float d = h + j < cnt ? f16_bits_to_f32((uint16_t)dh[h + j]) : 0.0f;
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) acc[i] = __builtin_fmaf(d, p[j][i], acc[i]);
+                    }
+                }
+            };
+
+            int slot = 0;
+            for (int ub = u0; ub < u1; ub += SK_BATCH) {
+                const int un = min(SK_BATCH, u1 - ub);
+                for (int k = 0; k < un; ++k) {
+                    if (c == c_begin) acc = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+                    unit(ub + k, slot, ep && ub > u0 && k < L::DEPTH && ub + duty < u1);
+                    slot = slot + 1 == L::DEPTH ? 0 : slot + 1;
+                    if (last_chunk) *(reinterpret_cast<f32x4*>(part) + (k * SK_WAVES + wave) * 64 + lane) = acc;
+                }
+                if (!last_chunk) continue;
+                block_sync();
+                if (duty < un && 8 * (wave & 1) < M) {
+                    const int u = ub + duty, n = n0 + 16 * u + l16;
+                    const float* from = part + duty * SK_WAVES * 256 + ((wave & 1) * 32 + l16) * 4 + q;
+                    float sum[2] = {from[0], from[64]};
+#pragma unroll
+                    for (int w = 1; w < SK_WAVES; ++w) {        // in wave order
+                        sum[0] += from[w * 256];
+                        sum[1] += from[w * 256 + 64];
+                    }
+                    if (ep) {
+                        // requested before the codes of the batch's refills
+                        if (ub + SK_BATCH + L::DEPTH <= u1) asm_wait_vmcnt<SK_BATCH * L::NDMA>();
+                        else asm_wait_vmcnt<0>();
+                        float v[SK_EP_LOADS];
+#pragma unroll
+                        for (int i = 0; i < SK_EP_LOADS; ++i)
+                            v[i] = __uint_as_float(asm_lds_read_b32(ep_base + (uint32_t)(256 * i + 4 * lane)));
+                        asm_wait_lgkmcnt<0>();
+#pragma unroll
+                        for (int i = 0; i < SK_EP_LOADS; ++i) asm_pin(v[i]);
+                        if (u + SK_BATCH < u1) issue_ep(u + SK_BATCH);
+#pragma unroll
+                        for (int i = 0; i < 2; ++i) {
+                            float o = sum[i];
+                            if (P.ep.bias) o += v[0];
+                            if (P.ep.act == 1) o = gelu_tanh(o);
+                            else if (P.ep.act == 2) o = silu(o);
+                            if (P.ep.mul) o *= v[1 + i];
+                            if (P.ep.res) o += v[3 + i];
+                            sum[i] = o;
+                        }
+                    }
+                    float* out = split ? cpart + (int64_t)c * M * N : P.Y;
+#pragma unroll
+                    for (int i = 0; i < 2; ++i)
+                        if (om + 4 * i < M && n < N) out[(int64_t)(om + 4 * i) * N + n] = sum[i];
+                }
+                if (ub + SK_BATCH < u1) block_sync();   // the sums are read before the next batch's are written
+            }
         }
     }
 }
 
-// Tile shape of a launch by its total 16-row groups.  Every wave reads its X
-// slice from L2 for each K block (2 KiB per block at M = 16, 4x the Q4_0 code
-// bytes of two row groups), so more row groups per wave means less X traffic
-// per weight.  Q4_0 takes four row groups per wave (16-wave blocks, two K
-// blocks per step, one block per CU) when those blocks fill the CUs in one
-// round (Phi-1.5 QKV+fc1, 896 row groups: M = 16 14.5 -> 12.9 us, M = 8
-// 12.7 -> 12.0 us); past one round the two-block-per-CU shape overlaps one
-// block's prologue with the other's loop and wins (LM head, 3200 row groups:
-// 41.0 us against 45.6 us).  Q8_0's codes are twice the bytes per weight, X
-// weighs half as much, and the shorter per-block chain lost (M = 8 QKV+fc1
-// 12.5 -> 13.5 us).  Then two row groups per block when that still gives
-// every CU a block; fewer row groups than CUs get 16-wave blocks (more loads
-// in flight per block), and so do Q4_0 launches of one to two row groups per
-// CU (Phi-1.5 dense+fc2, 256 row groups: half the K steps per wave; Q4_0
-// steps M = 5 708 -> 688 us, M = 8 728 -> 708 us, M = 16 768 -> 765 us, while
-// Q8_0 lost: M = 16 781 -> 788 us).
-enum SkinnyShape { SK_R4_W16, SK_R2_W8, SK_R1_W8, SK_R1_W16 };
-static SkinnyShape skinny_shape(int64_t groups, int num_cus, bool q4) {
-    if (q4 && groups >= 3 * (int64_t)num_cus && groups <= 4 * (int64_t)num_cus) return SK_R4_W16;
-    if (groups >= 2 * (int64_t)num_cus) return SK_R2_W8;
-    if (groups >= num_cus && !q4) return SK_R1_W8;
-    return SK_R1_W16;
+// Adds the chunks of the problems that were split over K, in chunk order.
+__global__ __launch_bounds__(256) void skinny_reduce_kernel(const SkinnyGroup g) {
+    const SkinnyProblem& P = g.p[blockIdx.y];
+    const int64_t mn = (int64_t)g.M * P.N;
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (!P.part || i >= mn) return;
+    float sum = P.part[i];
+    for (int c = 1; c < P.chunks; ++c) sum += P.part[c * mn + i];
+    P.Y[i] = P.ep_on ? apply_epilogue(P.ep, sum, i, i % P.N) : sum;
 }
 
-template <bool Q4>
-static size_t skinny_lds_for(SkinnyShape sh, int K) {
-    switch (sh) {
-        case SK_R4_W16:
-            if constexpr (Q4) return skinny_lds_bytes<Q4, 4, 16, 2>(K);
-            return SKINNY_LDS_MAX + 1;                // Q4_0 only
-        case SK_R2_W8: return skinny_lds_bytes<Q4, 2, 8, 4>(K);
-        case SK_R1_W8: return skinny_lds_bytes<Q4, 1, 8, 4>(K);
-        default: return skinny_lds_bytes<Q4, 1, 16, 4>(K);
+static int skinny_chunks(int K) { return (K / 32 + SK_CHUNK - 1) / SK_CHUNK; }
+
+size_t skinny_workspace_bytes(int M, int count, const mvlm_weight* const* ws) {
+    size_t bytes = 0;
+    for (int i = 0; i < count; ++i) {
+        const int chunks = skinny_chunks(ws[i]->K);
+        if (chunks > 1) bytes += (size_t)chunks * M * ws[i]->N * sizeof(float);
     }
+    return bytes;
 }
 
+// Which launches are taken: K a multiple of 32, codes and X within 32-bit
+// buffer offsets, and rows whose scales fit beside the code slots of the
+// workgroup that a launch of this many row groups took when a workgroup staged
+// whole rows (the limit callers know; nothing below depends on it).
 bool skinny_supported(int count, const mvlm_weight* const* ws, int num_cus) {
     if (num_cus <= 0) num_cus = 256;
     int64_t groups = 0;
     for (int i = 0; i < count; ++i) groups += (ws[i]->N + 15) / 16;
-    const SkinnyShape sh = skinny_shape(groups, num_cus, count > 0 && ws[0]->dtype == MVLM_Q4_0);
+    const bool q4 = count > 0 && ws[0]->dtype == MVLM_Q4_0;
+    int rows = 16;                                    // rows and code-slot bytes of that workgroup
+    size_t slots = q4 ? 32 * 1024 : 64 * 1024;
+    if (q4 && groups >= 3 * (int64_t)num_cus && groups <= 4 * (int64_t)num_cus) { rows = 64; slots = 64 * 1024; }
+    else if (groups >= 2 * (int64_t)num_cus) rows = 32;
+    else if (groups >= num_cus && !q4) slots = 32 * 1024;
     for (int i = 0; i < count; ++i) {
         const mvlm_weight* w = ws[i];
         if (!is_quant(w->dtype) || w->K % 32 != 0) return false;
         if (w->bytes > 0x7FFFFFFF || (int64_t)16 * w->K * 4 > 0x7FFFFFFF) return false;   // 32-bit buffer offsets
-        const size_t lds = w->dtype == MVLM_Q4_0 ? skinny_lds_for<true>(sh, w->K) : skinny_lds_for<false>(sh, w->K);
-        if (lds > SKINNY_LDS_MAX) return false;
+        if (((size_t)rows * (w->K / 32) * 2 + 255) / 256 * 256 + slots > 160 * 1024) return false;
     }
     return true;
 }
 
-template <bool Q4, int R, int NW, int G>
-static hipError_t launch_skinny(hipStream_t s, SkinnyGroup& g) {
-    const bool xs = g.M > 8;
-    auto kernel = xs ? gemm_skinny_kernel<Q4, R, NW, G, true> : gemm_skinny_kernel<Q4, R, NW, G, false>;
-    size_t lds = 0;
-    unsigned blocks = 0;
-    for (int i = 0; i < g.count; ++i) {
-        lds = std::max(lds, skinny_lds_bytes<Q4, R, NW, G>(g.p[i].K));
-        g.p[i].block_begin = (int)blocks;
-        blocks += (unsigned)((g.p[i].N + 16 * R - 1) / (16 * R));
-    }
-    if (const hipError_t e = xs ? allow_dynamic_lds<gemm_skinny_kernel<Q4, R, NW, G, true>>((int)SKINNY_LDS_MAX)
-                                : allow_dynamic_lds<gemm_skinny_kernel<Q4, R, NW, G, false>>((int)SKINNY_LDS_MAX);
-        e != hipSuccess)
-        return e;
-    if (lds > SKINNY_LDS_MAX) return hipErrorInvalidValue;
-    launch_kernel(kernel, dim3(blocks), dim3(64 * NW), (uint32_t)lds, s, g);
-    return hipGetLastError();
-}
-
-// A grouped launch picks the shape from the row groups of all its problems.
 template <bool Q4>
-static hipError_t launch_skinny_shape(hipStream_t s, SkinnyGroup& g, int num_cus) {
-    int64_t groups = 0;
-    for (int i = 0; i < g.count; ++i) groups += (g.p[i].N + 15) / 16;
-    switch (skinny_shape(groups, num_cus, Q4)) {
-        case SK_R4_W16:
-            if constexpr (Q4) return launch_skinny<Q4, 4, 16, 2>(s, g);
-            return hipErrorInvalidValue;              // Q4_0 only
-        case SK_R2_W8: return launch_skinny<Q4, 2, 8, 4>(s, g);
-        case SK_R1_W8: return launch_skinny<Q4, 1, 8, 4>(s, g);
-        default: return launch_skinny<Q4, 1, 16, 4>(s, g);
+static hipError_t launch_skinny(hipStream_t s, SkinnyGroup& g, int num_cus) {
+    constexpr auto kernel = gemm_skinny_kernel<Q4>;
+    constexpr int lds = SkinnyLayout<Q4>::LDS;
+    if (const hipError_t e = allow_dynamic_lds<kernel>(lds); e != hipSuccess) return e;
+    // Row groups per workgroup: the fewest that deal the launch out in whole
+    // rounds of one workgroup per CU.
+    int64_t units = 0;
+    for (int i = 0; i < g.count; ++i) units += (int64_t)((g.p[i].N + 15) / 16) * (g.p[i].part ? g.p[i].chunks : 1);
+    const int64_t rounds = (units + (int64_t)num_cus * SK_MAX_RG - 1) / ((int64_t)num_cus * SK_MAX_RG);
+    int rows = (int)((units + num_cus * rounds - 1) / (num_cus * rounds));
+    unsigned blocks = 0;
+    for (;; ++rows) {
+        blocks = 0;
+        for (int i = 0; i < g.count; ++i) {
+            SkinnyProblem& p = g.p[i];
+            p.rows = rows;
+            g.block_begin[i] = (int)blocks;
+            blocks += (unsigned)(((p.N + 15) / 16 + rows - 1) / rows * (p.part ? p.chunks : 1));
+        }
+        if (blocks <= num_cus * rounds || rows >= SK_MAX_RG) break;
     }
-}
-
-static SkinnyProblem skinny_problem(const float* X, const mvlm_weight* W, float* Y) {
-    SkinnyProblem p{};
-    p.X = X;
-    p.codes = (const uint8_t*)W->data;
-    p.scales = (const uint16_t*)W->scales;
-    p.Y = Y;
-    p.ld = (int64_t)W->ld;
-    p.N = W->N;
-    p.K = W->K;
-    return p;
-}
-
-hipError_t launch_gemm_skinny(hipStream_t s, const float* X, const mvlm_weight* W, float* Y, int M, int N, int K,
-                              int num_cus, const Epilogue* ep) {
-    if (M < 1 || M > 16 || K % 32 != 0 || !is_quant(W->dtype) || W->N != N || W->K != K) return hipErrorInvalidValue;
-    if (num_cus <= 0) num_cus = 256;
-    SkinnyGroup g{};
-    g.count = 1;
-    g.M = M;
-    g.p[0] = skinny_problem(X, W, Y);
-    if (ep && ep->any()) {
-        g.p[0].ep = *ep;
-        g.p[0].ep_on = 1;
+    bool split = false;
+    int64_t most = 0;
+    for (int i = 0; i < g.count; ++i)
+        if (g.p[i].part) {
+            split = true;
+            most = std::max(most, (int64_t)g.M * g.p[i].N);
+        }
+    if (!split) {
+        launch_kernel(kernel, dim3(blocks), dim3(64 * SK_WAVES), (uint32_t)lds, s, g);
+        return hipGetLastError();
     }
-    if (W->dtype == MVLM_Q4_0) return launch_skinny_shape<true>(s, g, num_cus);
-    return launch_skinny_shape<false>(s, g, num_cus);
+    launch_kernel_part(LaunchPart::First, kernel, dim3(blocks), dim3(64 * SK_WAVES), (uint32_t)lds, s, g);
+    launch_kernel_part(LaunchPart::Last, skinny_reduce_kernel, dim3((unsigned)((most + 255) / 256), (unsigned)g.count),
+                       dim3(256), 0, s, g);
+    return hipGetLastError();
 }
 
 hipError_t launch_gemm_skinny_group(hipStream_t s, int M, int count, const float* const* Xs,
                                     const mvlm_weight* const* ws, float* const* Ys, int num_cus,
-                                    const Epilogue* eps) {
+                                    const Epilogue* eps, void* workspace, size_t workspace_bytes) {
     if (M < 1 || M > 16 || count < 1 || count > SKINNY_MAX_GROUP) return hipErrorInvalidValue;
-    if (num_cus <= 0) num_cus = 256;
+    const bool have = workspace && workspace_bytes >= skinny_workspace_bytes(M, count, ws);
+    float* part = (float*)workspace;
     SkinnyGroup g{};
     g.count = count;
     g.M = M;
     for (int i = 0; i < count; ++i) {
         const mvlm_weight* W = ws[i];
         if (W->K % 32 != 0 || !is_quant(W->dtype) || W->dtype != ws[0]->dtype) return hipErrorInvalidValue;
-        g.p[i] = skinny_problem(Xs[i], W, Ys[i]);
+        SkinnyProblem& p = g.p[i];
+        p.X = Xs[i];
+        p.codes = (const uint8_t*)W->data;
+        p.scales = (const uint16_t*)W->scales;
+        p.Y = Ys[i];
+        p.ld = (uint32_t)W->ld;
+        p.N = W->N;
+        p.nb = W->K / 32;
+        p.chunks = skinny_chunks(W->K);
+        p.chunk_blocks = (W->K / 32 + p.chunks - 1) / p.chunks;
+        p.chunk_div = (uint32_t)((((uint64_t)1 << 32) + p.chunks - 1) / p.chunks);   // (not used for one chunk)
+        if (p.chunks > 1 && have) {
+            p.part = part;
+            part += (size_t)p.chunks * M * W->N;
+        }
         if (eps && eps[i].any()) {
-            g.p[i].ep = eps[i];
-            g.p[i].ep_on = 1;
+            p.ep = eps[i];
+            p.ep_on = 1;
         }
     }
-    if (ws[0]->dtype == MVLM_Q4_0) return launch_skinny_shape<true>(s, g, num_cus);
-    return launch_skinny_shape<false>(s, g, num_cus);
+    if (num_cus <= 0) num_cus = 256;
+    return ws[0]->dtype == MVLM_Q4_0 ? launch_skinny<true>(s, g, num_cus) : launch_skinny<false>(s, g, num_cus);
 }
 
 }  // namespace mvlm

@@ -9,6 +9,7 @@
 #include "common.h"
 
 #include <cmath>
+#include <cstdlib>
 #include <new>
 #include <vector>
 
@@ -288,6 +289,25 @@ int make_argmax(mvlm_device* dev, const mvlm_buffer* x, int dtype, int rows, int
     return MVLM_OK;
 }
 
+// Whether a quantized weight's product with M rows of x runs on the streaming
+// kernel rather than the skinny GEMM.  The streaming kernel multiplies each
+// weight on the vector ALU once per row, the skinny GEMM pays ~5 us per launch
+// to bring X into its registers whatever M is: a Phi-1.5 step of M = 4 takes
+// 586 us (Q4_0) and 633 us (Q8_0) streaming and 612 / 656 us skinny, one of
+// M = 8 would be twice the former.
+constexpr int STREAM_ROWS = 4;
+bool stream_serves(const mvlm_weight* w, int M) { return M <= STREAM_ROWS && stream_supported(w, M); }
+
+// Workspace of a skinny GEMM over op->gw[0..count).  An op that gets none still
+// runs (launch_gemm_skinny_group), so a failed allocation is not an error.
+// MVLM_SKINNY_WORKSPACE=0: take none (tests).
+void skinny_workspace(mvlm_device* dev, int count, Op* op) {
+    const char* use = std::getenv("MVLM_SKINNY_WORKSPACE");
+    if (use && use[0] == '0') return;
+    const size_t bytes = skinny_workspace_bytes(op->M, count, op->gw);
+    if (bytes > 0 && device_scratch(dev, bytes, &op->workspace) == MVLM_OK) op->workspace_bytes = bytes;
+}
+
 // Dense GEMV (M == 1) or dequantizing GEMV / skinny GEMM (M <= 16).
 // want_dtype: required weight dtype, or -1 for any.
 int make_gemv(mvlm_device* dev, const mvlm_buffer* x, int x_dtype, const mvlm_weight* W, mvlm_buffer* y,
@@ -307,11 +327,13 @@ int make_gemv(mvlm_device* dev, const mvlm_buffer* x, int x_dtype, const mvlm_we
         REQUIRE(x_dtype == MVLM_F32 && y_dtype == MVLM_F32, "%s: quantized weights take fp32 x and y", fn);
         NEED(x, (size_t)M * K * 4, "x");
         NEED(y, (size_t)M * N * 4, "y");
-        const bool streams = M == 1 ? stream_supported(W) : (M <= 4 && stream_supported(W, M));
+        const bool streams = stream_serves(W, M);
         if (!streams && !skinny_supported(1, &W, op->num_cus))
             return set_error(MVLM_ERR_UNSUPPORTED, "%s: K=%d is outside the skinny kernel's range (a multiple of 32 "
                              "whose block scales fit in LDS, weight below 2 GiB)", fn, K);
         op->kind = OP_GEMV_QUANT;
+        op->gw[0] = W;
+        if (!streams) skinny_workspace(dev, 1, op);
         return MVLM_OK;
     }
     REQUIRE(M == 1, "%s: dense weights take M == 1 (M=%d); use mvlm_gemm_packed", fn, M);
@@ -358,10 +380,11 @@ int make_gemv_group(mvlm_device* dev, int M, int count, const mvlm_gemv_desc* de
     op->a_dtype = descs[0].x_dtype;
     op->num_cus = dev->prop.multiProcessorCount;
     if (M > 1) {   // the skinny kernel serves the group unless every entry streams (launch_group_op)
-        bool stream = M <= 4;
-        for (int i = 0; i < count && stream; ++i) stream = stream_supported(op->gw[i], M);
+        bool stream = true;
+        for (int i = 0; i < count && stream; ++i) stream = stream_serves(op->gw[i], M);
         if (!stream && !skinny_supported(count, op->gw, op->num_cus))
             return set_error(MVLM_ERR_UNSUPPORTED, "%s: the group's block scales exceed the skinny kernel's LDS", fn);
+        if (!stream) skinny_workspace(dev, count, op);
     }
     return MVLM_OK;
 }
@@ -372,8 +395,8 @@ static hipError_t launch_group_op(hipStream_t s, const Op& op, bool with_attn) {
     if (op.M == 1)
         return launch_gemv_stream_group(s, op.gcount, op.gx, op.a_dtype, op.gw, op.gy, op.gyd, op.num_cus, op.gep, 1,
                                         with_attn ? &op.attn : nullptr);
-    bool stream = op.M <= 4;
-    for (int i = 0; i < op.gcount && stream; ++i) stream = stream_supported(op.gw[i], op.M);
+    bool stream = true;
+    for (int i = 0; i < op.gcount && stream; ++i) stream = stream_serves(op.gw[i], op.M);
     if (stream)
         return launch_gemv_stream_group(s, op.gcount, op.gx, op.a_dtype, op.gw, op.gy, op.gyd, op.num_cus, op.gep,
                                         op.M);
@@ -383,7 +406,8 @@ static hipError_t launch_group_op(hipStream_t s, const Op& op, bool with_attn) {
         xs[i] = (const float*)op.gx[i];
         ys[i] = (float*)op.gy[i];
     }
-    return launch_gemm_skinny_group(s, op.M, op.gcount, xs, op.gw, ys, op.num_cus, op.gep);
+    return launch_gemm_skinny_group(s, op.M, op.gcount, xs, op.gw, ys, op.num_cus, op.gep, op.workspace,
+                                    op.workspace_bytes);
 }
 
 // Per-entry epilogues of a grouped op (eps may be null: none).
@@ -394,6 +418,12 @@ int make_group_epilogues(mvlm_device* dev, const mvlm_epilogue* eps, const char*
         if (st != MVLM_OK) return st;
     }
     return MVLM_OK;
+}
+
+static hipError_t launch_skinny_op(hipStream_t s, const Op& op) {
+    const float* x = (const float*)op.a;
+    float* y = (float*)op.c;
+    return launch_gemm_skinny_group(s, op.M, 1, &x, &op.w, &y, op.num_cus, &op.ep, op.workspace, op.workspace_bytes);
 }
 
 hipError_t enqueue_op(hipStream_t s, const Op& op, bool with_attn = false) {
@@ -420,10 +450,9 @@ hipError_t enqueue_op(hipStream_t s, const Op& op, bool with_attn = false) {
         case OP_GEMV_QUANT:
             if (op.M == 1 && stream_supported(op.w))
                 return launch_gemv_stream(s, op.a, MVLM_F32, op.w, op.c, MVLM_F32, op.num_cus, &op.ep);
-            if (op.M <= 4 && stream_supported(op.w, op.M))
+            if (stream_serves(op.w, op.M))
                 return launch_gemv_stream_batch(s, (const float*)op.a, op.w, (float*)op.c, op.M, op.num_cus, &op.ep);
-            return launch_gemm_skinny(s, (const float*)op.a, op.w, (float*)op.c, op.M, op.N, op.K, op.num_cus,
-                                      &op.ep);
+            return launch_skinny_op(s, op);
         case OP_ARGMAX:
             return launch_argmax(s, op.a, op.a_dtype, op.M, op.N, op.lda, (int*)op.c, op.workspace);
         case OP_ATTENTION:

@@ -1,0 +1,93 @@
+"""The skinny GEMM over quantized weights (5 to 16 rows of x) where its work is
+cut: K of one chunk, of a full one (64 blocks), of two and more chunks that
+start at even and odd blocks, with fewer blocks than waves; row counts that are
+no multiple of 16; one row group per workgroup, more than a batch of four, and
+more than one round of workgroups; each epilogue operand; and the form that
+walks the chunks without workspace."""
+import numpy as np
+import pytest
+
+import mvlm_amd as m
+from tests.test_gpu_parity import make_quant, within
+
+pytestmark = pytest.mark.gpu
+
+F32, Q8, Q4 = m.F32, m.Q8_0, m.Q4_0
+
+
+def reference(orc, qt, X, blocks, M, N, K):
+    kind, deq = ("q8_0", orc.dequant_q8_0) if qt == Q8 else ("q4_0", orc.dequant_q4_0)
+    ref = orc.gemm_nk(kind, X, blocks, M, N, K).reshape(M, N)
+    _, S = orc.gemm_f64(X.astype(np.float64).reshape(M, K), deq(blocks).astype(np.float64).reshape(N, K), M, N, K)
+    return ref, S.reshape(M, N)
+
+
+def run(dev, orc, qt, M, N, K, seed=611):
+    X, blocks = orc.normal_f32(M * K, seed), make_quant(orc, qt, N, K, seed + 1)
+    dY = dev.upload(np.full(M * N, np.nan, np.float32))
+    dev.gemm_quant(dev.upload(X), dev.pack(blocks, qt, N, K), dY, M, N, K)
+    got = dY.download(np.float32).reshape(M, N)
+    ref, S = reference(orc, qt, X, blocks, M, N, K)
+    ok, worst = within(got, ref, S, 1e-5)
+    assert ok, worst
+    return got
+
+
+@pytest.mark.parametrize("qt", [Q8, Q4])
+@pytest.mark.parametrize("M,N,K", [(5, 1, 32), (16, 16, 7 * 32), (9, 47, 33 * 32), (8, 100, 2048), (16, 33, 65 * 32),
+                                   (7, 50, 130 * 32), (13, 64, 8192), (16, 21, 191 * 32), (6, 20485, 96),
+                                   (16, 57400, 64), (10, 57361, 32)])
+def test_cuts(dev, orc, qt, M, N, K):
+    run(dev, orc, qt, M, N, K)
+
+
+@pytest.mark.parametrize("qt", [Q8, Q4])
+@pytest.mark.parametrize("M,N,K", [(16, 37, 65 * 32), (5, 4200, 130 * 32), (12, 300, 8192)])
+def test_without_workspace(dev, orc, monkeypatch, qt, M, N, K):
+    """the same sums, chunk by chunk in one workgroup"""
+    with_ws = run(dev, orc, qt, M, N, K)
+    monkeypatch.setenv("MVLM_SKINNY_WORKSPACE", "0")
+    # fma chains that run through the chunks against chunk sums that are added
+    assert np.allclose(run(dev, orc, qt, M, N, K), with_ws, rtol=0, atol=1e-5 * np.abs(with_ws).max())
+
+
+@pytest.mark.parametrize("qt", [Q8, Q4])
+@pytest.mark.parametrize("M", [5, 9, 16])
+@pytest.mark.parametrize("ep", ["bias", "mul", "residual", "all"])
+def test_epilogue_operands(dev, orc, qt, M, ep):
+    """three problems in one launch: seven row groups per workgroup, a short
+    one, and one of two chunks (its epilogue is the second launch's)"""
+    shapes = [(16 * 1600 + 5, 64), (40, 96), (50, 70 * 32)]
+    descs, eps, want = [], [], []
+    for i, (N, K) in enumerate(shapes):
+        X, blocks = orc.normal_f32(M * K, 631 + i), make_quant(orc, qt, N, K, 641 + i)
+        ref, S = reference(orc, qt, X, blocks, M, N, K)
+        bias, mul, res = orc.normal_f32(N, 651), orc.normal_f32(M * N, 652), orc.normal_f32(M * N, 653)
+        out, size, e = ref.astype(np.float64), S, {}
+        if ep in ("bias", "all"):
+            e["bias"], out, size = dev.upload(bias), out + bias, size + np.abs(bias)
+        if ep in ("mul", "all"):
+            mm = mul.reshape(M, N)
+            e["mul"], out, size = dev.upload(mul), out * mm, size * np.abs(mm)
+        if ep in ("residual", "all"):
+            rr = res.reshape(M, N)
+            e["residual"], out, size = dev.upload(res), out + rr, size + np.abs(rr)
+        y = dev.upload(np.full(M * N, np.nan, np.float32))
+        descs.append((dev.upload(X), F32, dev.pack(blocks, qt, N, K), y, F32))
+        eps.append(e)
+        want.append((y, out, size))
+    dev.gemm_quant_grouped(M, descs, epilogues=eps)
+    for (y, out, size), (N, K) in zip(want, shapes):
+        ok, worst = within(y.download(np.float32).reshape(M, N), out, size, 1e-5)
+        assert ok, (N, K, worst)
+
+
+@pytest.mark.parametrize("qt", [Q8, Q4])
+def test_not_a_number_stays_in_its_row(dev, orc, qt):
+    M, N, K = 9, 70, 300 * 32
+    X, blocks = orc.normal_f32(M * K, 661).reshape(M, K), make_quant(orc, qt, N, K, 662)
+    X[3, 17], X[6, 9000], X[8, 40] = np.nan, np.inf, -np.inf
+    dY = dev.alloc(M * N * 4)
+    dev.gemm_quant(dev.upload(X), dev.pack(blocks, qt, N, K), dY, M, N, K)
+    bad = ~np.isfinite(dY.download(np.float32).reshape(M, N))
+    assert bad[[3, 6, 8]].all() and not bad[[0, 1, 2, 4, 5, 7]].any()
