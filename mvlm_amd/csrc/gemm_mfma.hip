@@ -10,12 +10,10 @@
 // Structure.  A block of WGM x WGN waves owns a BM x BN tile of C; each wave a
 // (BM/WGM) x (BN/WGN) sub-tile of 32x32 v_mfma_f32_32x32x16 tiles.
 // K advances in 64-wide stages held in an LDS ring of STAGES slots:
-//  * global -> LDS with direct 16-byte loads (buffer_load_dwordx4 ... lds
-//    through a descriptor over the tile's rows on the large tiles,
-//    global_load_lds_dwordx4 on the others): one wave instruction moves
-//    8 rows x 128 bytes (a 64-element K slice of 8 rows) straight into LDS,
-//    no registers involved, so up to STAGES-1 stages are in flight while the
-//    MFMAs work on the oldest;
+//  * global -> LDS with direct 16-byte loads (global_load_lds_dwordx4): one
+//    wave instruction moves 8 rows x 128 bytes (a 64-element K slice of 8
+//    rows) straight into LDS, no registers involved, so up to STAGES-1 stages
+//    are in flight while the MFMAs work on the oldest;
 //  * LDS rows are 128 bytes; the 16-byte slot s of row r is stored at slot
 //    s ^ ((r >> 1) & 7).  gfx950's LDS serves a ds_read_b128 16 lanes at a
 //    time from 64 four-byte banks (a 256-byte period, two rows), so the 16
@@ -27,6 +25,9 @@
 //    (i & 7) ^ ((4g + (i >> 4)) & 7);
 //  * one barrier per stage: after it, the slot computed in the previous
 //    iteration is refilled.
+// That is the kernel of the small tiles (gemm_mfma_kernel); tiles from 128 x
+// 128 up share its layouts but alternate two groups of waves
+// (gemm_pingpong_kernel).
 // Rows beyond M / N are clamped to the last valid row (their products land in
 // outputs that are never stored).  K beyond the operand's readable width is
 // zero-filled by a guarded load path used only for the last stage.
@@ -154,26 +155,6 @@ __device__ __forceinline__ void stage_direct(const uint16_t* __restrict__ base, 
     }
 }
 
-// stage_direct through a buffer descriptor whose base is the tile's first row:
-// a 32-bit offset per lane instead of a 64-bit address (fewer VGPRs, and the
-// Phi-1.5 M = 768 shapes and 4096^3 2-5% faster; the SigLIP tiles keep the
-// global form, which measured as fast or faster there)
-template <int BK, int ROWS, int NW>
-__device__ __forceinline__ void stage_direct_buf(i32x4 rsrc, int64_t ld, int r0, int rmax, int k0, uint16_t* lds,
-                                                 int wave, int lane) {
-    using G = StageGeom<BK>;
-    static_assert((ROWS / G::RPI) % NW == 0, "row groups must split evenly over the waves");
-#pragma unroll
-    for (int t = 0; t < ROWS / (G::RPI * NW); ++t) {
-        const int g = wave + NW * t;
-        const int lr = G::RPI * g + lane / G::LPR;
-        const int ls = (lane % G::LPR) ^ G::swz(lr);
-        const int r = min(r0 + lr, rmax) - r0;
-        const uint32_t off = (uint32_t)(((int64_t)r * ld + k0 + ls * 8) * 2);
-        asm_buffer_load_lds_b128(rsrc, off, __builtin_amdgcn_readfirstlane(lds_offset(lds + G::RPI * g * G::ROWH)));
-    }
-}
-
 // Guarded loads of the last stage: 16-byte chunks at or beyond kread are zero.
 template <int BK, int ROWS, int NW>
 __device__ __forceinline__ void stage_guarded(const uint16_t* __restrict__ base, int64_t ld, int r0, int rmax, int k0,
@@ -193,7 +174,92 @@ __device__ __forceinline__ void stage_guarded(const uint16_t* __restrict__ base,
     }
 }
 
-template <bool BF16, int BM, int BN, int BK, int STAGES, int WGM, int WGN, bool BUF>
+// The wave's TM x TN accumulator tiles to C (with the epilogue) or to the split
+// partials ws: tile (i, j) has its first element at row row_of(i), column
+// col_of(j).  cst: the wave's 32 x CSTAGE floats of LDS staging.
+constexpr int CSTAGE = 36;
+template <int TM, int TN, typename RowOf, typename ColOf>
+__device__ __forceinline__ void store_tiles(const GemmArgs& p, f32x16 (&acc)[TM][TN], float* cst, int64_t c_off,
+                                            float* ws, int lane, RowOf row_of, ColOf col_of) {
+    const bool vec = ws ? p.vec_ws : p.vec_c;
+    if (!vec) {   // rows off the vector grid: straight from the accumulators, 32 columns per row
+        if (ws) {
+#pragma unroll
+            for (int i = 0; i < TM; ++i)
+#pragma unroll
+                for (int j = 0; j < TN; ++j) {
+                    const int col = col_of(j) + (lane & 31);
+                    if (col >= p.N) continue;
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) {
+                        const int row = row_of(i) + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
+                        if (row < p.M) ws[(int64_t)row * p.N + col] = acc[i][j][r];
+                    }
+                }
+        } else if (!p.ep_on) {
+#pragma unroll
+            for (int i = 0; i < TM; ++i)
+#pragma unroll
+                for (int j = 0; j < TN; ++j) {
+                    const int col = col_of(j) + (lane & 31);
+                    if (col >= p.N) continue;
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) {
+                        const int row = row_of(i) + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
+                        if (row < p.M) store_out(p.C, c_off + (int64_t)row * p.ldc + col, acc[i][j][r], p.c_dtype);
+                    }
+                }
+        } else {   // fused epilogue: the per-element code is larger, so only the tile loops unroll
+#pragma unroll
+            for (int i = 0; i < TM; ++i)
+#pragma unroll
+                for (int j = 0; j < TN; ++j) {
+                    const int col = col_of(j) + (lane & 31);
+                    if (col >= p.N) continue;
+#pragma unroll 4
+                    for (int r = 0; r < 16; ++r) {
+                        const int row = row_of(i) + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
+                        if (row < p.M) {
+                            const int64_t idx = c_off + (int64_t)row * p.ldc + col;
+                            store_out(p.C, idx, apply_epilogue(p.ep, acc[i][j][r], idx, col), p.c_dtype);
+                        }
+                    }
+                }
+        }
+        return;
+    }
+    // Aligned rows: through LDS.  Each wave writes one 32x32 accumulator tile
+    // at a time into its own region of the (now idle) ring, row-major with a
+    // 36-float pitch (rows r and r+4, written by lanes l and l+32, land 16
+    // banks apart), and reads it back as 4 consecutive columns per lane, 8 rows
+    // per pass: 16-byte global stores, and per-element code (epilogue, dtype)
+    // in a loop rather than unrolled over the 16 * TM * TN accumulators.
+    __syncthreads();   // every wave is done with the ring (all its loads have landed)
+    constexpr int CS = CSTAGE;
+    const int srow = lane >> 3, scol = (lane & 7) * 4;
+    // (compile-time tile indices: a rolled tile loop would index acc at run time
+    // and move it to scratch memory)
+    static_for<TM * TN>([&](auto IJ) {
+        constexpr int i = decltype(IJ)::value / TN, j = decltype(IJ)::value % TN;
+        {
+#pragma unroll
+            for (int r = 0; r < 16; ++r)
+                cst[(8 * (r >> 2) + 4 * (lane >> 5) + (r & 3)) * CS + (lane & 31)] = acc[i][j][r];
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // this wave's writes, before its reads
+            const int row0 = row_of(i), col = col_of(j) + scol;
+            for (int t = 0; t < 4; ++t) {
+                const int row = row0 + srow + 8 * t;
+                const f32x4 v = *reinterpret_cast<const f32x4*>(cst + (srow + 8 * t) * CS + scol);
+                if (row >= p.M) continue;
+                if (ws) store_partial4(ws, (int64_t)row * p.N + col, v, p.N - col);
+                else store_c4(p, c_off + (int64_t)row * p.ldc, col, v);
+            }
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // reads done before the next tile's writes
+        }
+    });
+}
+
+template <bool BF16, int BM, int BN, int BK, int STAGES, int WGM, int WGN>
 __global__ __launch_bounds__(64 * WGM * WGN) void gemm_mfma_kernel(const GemmArgs p) {
     using G = StageGeom<BK>;
     constexpr int ROWH = G::ROWH;
@@ -204,7 +270,7 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_mfma_kernel(const GemmArg
     constexpr int SLOT = (BM + BN) * ROWH;       // elements per ring slot
     static_assert(TM + TN <= 15, "fragment reads must fit the lgkmcnt field");
     // the store pass reuses the ring: a 32 x 36 fp32 staging tile per wave
-    static_assert(STAGES * SLOT * 2 >= NW * 32 * 36 * 4, "ring too small for the store staging");
+    static_assert(STAGES * SLOT * 2 >= NW * 32 * CSTAGE * 4, "ring too small for the store staging");
     __shared__ __attribute__((aligned(1024))) uint16_t smem[STAGES * SLOT];
 
     // Tile order: blocks are dealt round-robin to the 8 XCDs; give each XCD a
@@ -231,20 +297,14 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_mfma_kernel(const GemmArg
     const bool tail_a = (nk_all * BK > K) && kt0 + nk == nk_all;
     const bool tail_b = (nk_all * BK > p.kread_b) && kt0 + nk == nk_all;
 
-    // BUF: descriptors over the tile's rows of A and B (every offset stays below
-    // the 32-bit size, checked by the launcher)
-    const i32x4 ra = raw_rsrc(A + (int64_t)m0 * p.lda, BUF ? (uint32_t)((int64_t)(p.M - m0) * p.lda * 2) : 0u);
-    const i32x4 rb = raw_rsrc(B + (int64_t)n0 * p.ldb, BUF ? (uint32_t)((int64_t)(p.N - n0) * p.ldb * 2) : 0u);
     auto issue = [&](int kt) {
         uint16_t* slot = smem + (kt % STAGES) * SLOT;
         const int k0 = (kt0 + kt) * BK;
         const bool last = (kt == nk - 1);
         if (last && tail_a) stage_guarded<BK, BM, NW>(A, p.lda, m0, p.M - 1, k0, K, slot, wave, lane);
-        else if constexpr (BUF) stage_direct_buf<BK, BM, NW>(ra, p.lda, m0, p.M - 1, k0, slot, wave, lane);
         else stage_direct<BK, BM, NW>(A, p.lda, m0, p.M - 1, k0, slot, wave, lane);
         if (last && tail_b)
             stage_guarded<BK, BN, NW>(B, p.ldb, n0, p.N - 1, k0, p.kread_b, slot + BM * ROWH, wave, lane);
-        else if constexpr (BUF) stage_direct_buf<BK, BN, NW>(rb, p.ldb, n0, p.N - 1, k0, slot + BM * ROWH, wave, lane);
         else stage_direct<BK, BN, NW>(B, p.ldb, n0, p.N - 1, k0, slot + BM * ROWH, wave, lane);
     };
 
@@ -345,83 +405,243 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_mfma_kernel(const GemmArg
 
     const int64_t c_off = (int64_t)batch * p.sC;
     float* ws = p.splits > 1 ? p.ws + (int64_t)blockIdx.z * p.M * p.N : nullptr;
-    const bool vec = ws ? p.vec_ws : p.vec_c;
-    if (!vec) {   // rows off the vector grid: straight from the accumulators, 32 columns per row
-        if (ws) {
+    store_tiles<TM, TN>(p, acc, reinterpret_cast<float*>(smem) + wave * 32 * CSTAGE, c_off, ws, lane,
+                        [&](int i) { return m0 + wm * WM + i * 32; }, [&](int j) { return n0 + wn * WN + j * 32; });
+}
+
+// Tiles whose eight waves form two groups of four, one wave of each per SIMD,
+// and work in alternating intervals divided by barriers: while one group
+// multiplies, the other reads its next fragments from LDS and issues its share
+// of the global -> LDS loads, so neither the LDS reads nor the ~16 clocks that a
+// load instruction occupies the address unit stand in front of the matrix
+// cores.  (With all waves in step, loads and products took turns: 4096^3 with
+// 256 x 256 tiles ran 134 us, its loads alone 97, its products alone 99.)
+//
+// A stage (64 of K) is NA units of UA rows of A and NB units of 128 rows of B.
+// Waves form a 2 x 4 grid in each pair of units (group = grid row); a phase,
+// one memory and one matrix interval, multiplies one A unit by one B unit.  Each
+// unit of the S-slot ring is refilled in the phase after the one that read it
+// (reads are waited for before the barrier that ends their interval, so both
+// groups are done with it):
+//   NB = 2, NA = 2, S = 2 (256 x 256)      NB = 1
+//   phase reads        products refills      phase  reads             products refills
+//   0     A0           A0 B0    B0           0      A0                A0 B     B, the last A unit
+//   1     B1           A0 B1    A0           q      Aq                Aq B     A(q-1)
+//   2     A1           A1 B1    B1           last   Aq, B of kt + 1   Aq B     A(q-1)
+//   3     B0 of kt + 1 A1 B0    A1
+// Loads complete in issue order and every phase issues a fixed number, so "the
+// units read next have landed" is a constant vmcnt at the end of each memory
+// interval, and nearly the whole ring is in flight.  Loads past the split's K are
+// issued out of the descriptor's range: they write zeros to LDS and move
+// nothing, which serves the K tail and keeps the counts the same to the end.
+template <bool BF16, int NA, int NB, int UA, int S>
+__global__ __launch_bounds__(512, 2) void gemm_pingpong_kernel(const GemmArgs p) {
+    constexpr int BM = NA * UA, BN = NB * 128, BK = 64;
+    constexpr int ABYTES = UA * BK * 2, BBYTES = 128 * BK * 2, STAGE = NA * ABYTES + NB * BBYTES;
+    constexpr int LA = UA / 64;                        // load instructions per wave of an A unit (2 of a B unit)
+    constexpr int TA = UA / 64;                        // 32-row tiles per wave of an A unit (1 column tile of a B unit)
+    static_assert((NB == 2 && NA == 2 && S == 2) || (NB == 1 && UA == 64), "phase tables above");
+    using G = StageGeom<BK>;
+    __shared__ __attribute__((aligned(1024))) uint8_t smem[S * STAGE];
+    static_assert(S * STAGE >= 8 * 32 * CSTAGE * 4, "ring too small for the store staging");
+
+    // tile order as in gemm_mfma_kernel
+    const int tiles = p.tiles_m * p.tiles_n;
+    int t = blockIdx.x;
+    const int per = tiles / 8;
+    if (t < 8 * per) t = (t % 8) * per + t / 8;
+    const int tm = t % p.tiles_m, tn = t / p.tiles_m;
+    const int m0 = tm * BM, n0 = tn * BN;
+    const int batch = blockIdx.z / p.splits, split = blockIdx.z % p.splits;
+    const uint16_t* __restrict__ A = p.A + (int64_t)batch * p.sA;
+    const uint16_t* __restrict__ B = p.B + (int64_t)batch * p.sB;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int wm = wave >> 2, wn = wave & 3;
+    const int nk_all = (p.K + BK - 1) / BK;
+    const int kt0 = split * p.split_stages;
+    const int nk = min(nk_all - kt0, p.split_stages);
+
+    const i32x4 rsa = raw_rsrc(A + (int64_t)m0 * p.lda, (uint32_t)((int64_t)(p.M - m0) * p.lda * 2));
+    const i32x4 rsb = raw_rsrc(B + (int64_t)n0 * p.ldb, (uint32_t)((int64_t)(p.N - n0) * p.ldb * 2));
+    // load instruction g = wave + 8 q of a unit fills its rows 8 g .. 8 g + 7
+    const int lrow = 8 * wave + lane / 8;
+    const int ls = (lane % 8) ^ G::swz(lrow);          // the same for every q
+    uint32_t va[NA][LA], vb[NB][2];                    // byte offsets at K column kt0 * BK
 #pragma unroll
-            for (int i = 0; i < TM; ++i)
+    for (int u = 0; u < NA; ++u)
 #pragma unroll
-                for (int j = 0; j < TN; ++j) {
-                    const int col = n0 + wn * WN + j * 32 + (lane & 31);
-                    if (col >= p.N) continue;
+        for (int q = 0; q < LA; ++q)
+            va[u][q] = (uint32_t)(((int64_t)min(UA * u + 64 * q + lrow, p.M - 1 - m0) * p.lda + kt0 * BK + ls * 8) * 2);
 #pragma unroll
-                    for (int r = 0; r < 16; ++r) {
-                        const int row = m0 + wm * WM + i * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
-                        if (row < p.M) ws[(int64_t)row * p.N + col] = acc[i][j][r];
-                    }
-                }
-        } else if (!p.ep_on) {
+    for (int u = 0; u < NB; ++u)
 #pragma unroll
-            for (int i = 0; i < TM; ++i)
+        for (int q = 0; q < 2; ++q)
+            vb[u][q] = (uint32_t)(((int64_t)min(128 * u + 64 * q + lrow, p.N - 1 - n0) * p.ldb + kt0 * BK + ls * 8) * 2);
+    // a lane's 16 bytes of stage kt are in range while kt * BK < klim
+    const int klim = min(p.K - kt0 * BK, nk * BK) - ls * 8;
+    const uint32_t lds0 = lds_offset(smem);
+    const uint32_t wave_lds = lds0 + wave * 1024;
+    auto refill_a = [&](int u, uint32_t slot, int kt) {
 #pragma unroll
-                for (int j = 0; j < TN; ++j) {
-                    const int col = n0 + wn * WN + j * 32 + (lane & 31);
-                    if (col >= p.N) continue;
+        for (int q = 0; q < LA; ++q)
+            asm_buffer_load_lds_b128(rsa, kt * BK < klim ? va[u][q] + kt * (BK * 2) : 0xFFFFFF00u,
+                                     wave_lds + slot + u * ABYTES + q * 8192);
+    };
+    auto refill_b = [&](int u, uint32_t slot, int kt) {
 #pragma unroll
-                    for (int r = 0; r < 16; ++r) {
-                        const int row = m0 + wm * WM + i * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
-                        if (row < p.M) store_out(p.C, c_off + (int64_t)row * p.ldc + col, acc[i][j][r], p.c_dtype);
-                    }
-                }
-        } else {   // fused epilogue: the per-element code is larger, so only the tile loops unroll
+        for (int q = 0; q < 2; ++q)
+            asm_buffer_load_lds_b128(rsb, kt * BK < klim ? vb[u][q] + kt * (BK * 2) : 0xFFFFFF00u,
+                                     wave_lds + slot + NA * ABYTES + u * BBYTES + q * 8192);
+    };
+
+    f32x16 acc[NA * TA][NB];
 #pragma unroll
-            for (int i = 0; i < TM; ++i)
+    for (int i = 0; i < NA * TA; ++i)
 #pragma unroll
-                for (int j = 0; j < TN; ++j) {
-                    const int col = n0 + wn * WN + j * 32 + (lane & 31);
-                    if (col >= p.N) continue;
-#pragma unroll 4
-                    for (int r = 0; r < 16; ++r) {
-                        const int row = m0 + wm * WM + i * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
-                        if (row < p.M) {
-                            const int64_t idx = c_off + (int64_t)row * p.ldc + col;
-                            store_out(p.C, idx, apply_epilogue(p.ep, acc[i][j][r], idx, col), p.c_dtype);
-                        }
-                    }
-                }
-        }
-        return;
+        for (int j = 0; j < NB; ++j)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
+
+    // fragments: row lane & 31 of a 32-row tile, 16-byte slot 2 ks + lane / 32
+    uint32_t aaddr[4], baddr[4];
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) {
+        const uint32_t c = (uint32_t)((2 * ks + (lane >> 5)) ^ G::swz(lane & 31)) << 4;
+        aaddr[ks] = lds0 + (wm * (UA / 2) + (lane & 31)) * 128 + c;
+        baddr[ks] = lds0 + NA * ABYTES + (wn * 32 + (lane & 31)) * 128 + c;
     }
-    // Aligned rows: through LDS.  Each wave writes one 32x32 accumulator tile
-    // at a time into its own region of the (now idle) ring, row-major with a
-    // 36-float pitch (rows r and r+4, written by lanes l and l+32, land 16
-    // banks apart), and reads it back as 4 consecutive columns per lane, 8 rows
-    // per pass: 16-byte global stores, and per-element code (epilogue, dtype)
-    // in a loop rather than unrolled over the 16 * TM * TN accumulators.
-    __syncthreads();   // every wave is done with the ring (all its loads have landed)
-    constexpr int CS = 36;
-    float* cst = reinterpret_cast<float*>(smem) + wave * 32 * CS;
-    const int srow = lane >> 3, scol = (lane & 7) * 4;
-    // (compile-time tile indices: a rolled tile loop would index acc at run time
-    // and move it to scratch memory)
-    static_for<TM * TN>([&](auto IJ) {
-        constexpr int i = decltype(IJ)::value / TN, j = decltype(IJ)::value % TN;
-        {
+    // fb: the first B unit of even and odd stages, the second B unit
+    u32x4 fa[TA][4], fb[NB + 1][4];
+    auto read_a = [&](auto U, uint32_t slot) {
 #pragma unroll
-            for (int r = 0; r < 16; ++r)
-                cst[(8 * (r >> 2) + 4 * (lane >> 5) + (r & 3)) * CS + (lane & 31)] = acc[i][j][r];
-            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // this wave's writes, before its reads
-            const int row0 = m0 + wm * WM + i * 32, col = n0 + wn * WN + j * 32 + scol;
-            for (int t = 0; t < 4; ++t) {
-                const int row = row0 + srow + 8 * t;
-                const f32x4 v = *reinterpret_cast<const f32x4*>(cst + (srow + 8 * t) * CS + scol);
-                if (row >= p.M) continue;
-                if (ws) store_partial4(ws, (int64_t)row * p.N + col, v, p.N - col);
-                else store_c4(p, c_off + (int64_t)row * p.ldc, col, v);
-            }
-            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // reads done before the next tile's writes
+        for (int ks = 0; ks < 4; ++ks) {
+            fa[0][ks] = asm_lds_read_b128<decltype(U)::value * ABYTES>(aaddr[ks] + slot);
+            if constexpr (TA == 2) fa[1][ks] = asm_lds_read_b128<decltype(U)::value * ABYTES + 4096>(aaddr[ks] + slot);
         }
-    });
+    };
+    auto read_b = [&](auto U, uint32_t slot, u32x4 (&f)[4]) {
+#pragma unroll
+        for (int ks = 0; ks < 4; ++ks) f[ks] = asm_lds_read_b128<decltype(U)::value * BBYTES>(baddr[ks] + slot);
+    };
+    auto pin = [&](u32x4 (&f)[4]) {
+#pragma unroll
+        for (int ks = 0; ks < 4; ++ks) asm_pin(f[ks]);
+    };
+    auto pin_a = [&]() {
+        pin(fa[0]);
+        if constexpr (TA == 2) pin(fa[1]);
+    };
+    // end of a memory interval: this wave's reads are done, all but the newest
+    // PENDING of its loads have landed
+    auto mem_end = [&](auto PENDING) {
+        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"(decltype(PENDING)::value) : "memory");
+    };
+    auto products = [&](auto I, auto J, u32x4 (&f)[4]) {
+        constexpr int i = TA * decltype(I)::value, j = decltype(J)::value;
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_sched_barrier(0);
+        __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+        for (int ks = 0; ks < 4; ++ks)
+#pragma unroll
+            for (int x = 0; x < TA; ++x) acc[i + x][j] = mfma32<BF16>(fa[x][ks], f[ks], acc[i + x][j]);
+        __builtin_amdgcn_s_setprio(0);
+        __builtin_amdgcn_sched_barrier(0);
+        __builtin_amdgcn_s_barrier();
+    };
+    constexpr std::integral_constant<int, 0> c0{};
+    constexpr std::integral_constant<int, 1> c1{};
+    // stage kt in ring slot `cur` (byte offset); `next` is the slot of kt + 1,
+    // `prev` that of kt - 1
+    auto stage = [&](int kt, uint32_t prev, uint32_t cur, uint32_t next, u32x4 (&b0)[4], u32x4 (&b0_next)[4]) {
+        if constexpr (NB == 2) {
+            constexpr std::integral_constant<int, 12> pending{};
+            read_a(c0, cur);
+            refill_b(0, cur, kt + S);
+            mem_end(pending);
+            pin_a();
+            products(c0, c0, b0);
+            read_b(c1, cur, fb[2]);
+            refill_a(0, cur, kt + S);
+            mem_end(pending);
+            pin(fb[2]);
+            products(c0, c1, fb[2]);
+            read_a(c1, cur);
+            refill_b(1, cur, kt + S);
+            mem_end(pending);
+            pin_a();
+            products(c1, c1, fb[2]);
+            read_b(c0, next, b0_next);
+            refill_a(1, cur, kt + S);
+            mem_end(pending);
+            pin(b0_next);
+            products(c1, c0, b0);
+        } else {
+            constexpr int L = NA + 2;                  // loads per wave and stage
+            static_for<NA>([&](auto Q) {
+                constexpr int q = decltype(Q)::value;
+                read_a(Q, cur);
+                if constexpr (q == NA - 1) read_b(c0, next, b0_next);
+                if constexpr (q == 0) {
+                    refill_b(0, cur, kt + S);
+                    refill_a(NA - 1, prev, kt + S - 1);
+                } else {
+                    refill_a(q - 1, cur, kt + S);
+                }
+                mem_end(std::integral_constant<int, (S - 1) * L + (q < NA - 2 ? NA : NA - 2)>{});
+                pin_a();
+                if constexpr (q == NA - 1) pin(b0_next);
+                products(Q, c0, b0);
+            });
+        }
+    };
+
+    // the ring's first stages, in the order the phases issue them
+    if constexpr (NB == 2) {
+        for (int k = 0; k < S; ++k) {
+            refill_b(0, k * STAGE, k);
+            refill_a(0, k * STAGE, k);
+            refill_b(1, k * STAGE, k);
+            refill_a(1, k * STAGE, k);
+        }
+        asm_wait_vmcnt<12>();
+    } else {
+        for (int k = 0; k < S; ++k) {
+            refill_b(0, k * STAGE, k);
+            if (k > 0) refill_a(NA - 1, (k - 1) * STAGE, k - 1);
+#pragma unroll
+            for (int u = 0; u < NA - 1; ++u) refill_a(u, k * STAGE, k);
+        }
+        asm_wait_vmcnt<(S - 1) * (NA + 2) + NA - 2>();
+    }
+    __builtin_amdgcn_s_barrier();
+    read_b(c0, 0, fb[0]);
+    asm_wait_lgkmcnt<0>();
+    pin(fb[0]);
+    __builtin_amdgcn_s_barrier();                // B0's slot may be refilled
+    if (wm == 1) __builtin_amdgcn_s_barrier();   // the second group runs one interval behind
+    uint32_t prev = (S - 1) * STAGE, cur = 0, next = STAGE;
+    auto advance = [&]() {
+        prev = cur;
+        cur = next;
+        next = next == (S - 1) * STAGE ? 0 : next + STAGE;
+    };
+    int kt = 0;
+    for (; kt + 1 < nk; kt += 2) {
+        stage(kt, prev, cur, next, fb[0], fb[1]);
+        advance();
+        stage(kt + 1, prev, cur, next, fb[1], fb[0]);
+        advance();
+    }
+    if (kt < nk) stage(kt, prev, cur, next, fb[0], fb[1]);
+    if (wm == 0) __builtin_amdgcn_s_barrier();
+    asm_wait_vmcnt<0>();                         // the out-of-range loads write LDS too
+
+    const int64_t c_off = (int64_t)batch * p.sC;
+    float* ws = p.splits > 1 ? p.ws + (int64_t)blockIdx.z * p.M * p.N : nullptr;
+    store_tiles<NA * TA, NB>(p, acc, reinterpret_cast<float*>(smem) + wave * 32 * CSTAGE, c_off, ws, lane,
+                             [&](int i) { return m0 + UA * (i / TA) + wm * (UA / 2) + 32 * (i % TA); },
+                             [&](int j) { return n0 + 128 * j + wn * 32; });
 }
 
 // Sums the split-K partials in split order (deterministic), applies the
@@ -470,41 +690,39 @@ typedef void (*GemmKernel)(const GemmArgs);
 struct TileCfg {
     int bm, bn, bk, stages, waves;
     int per_cu;       // resident blocks per CU (LDS ring and registers)
-    int eff;          // TFLOP/s of a full-wave 4096^3 fp16 run (selection weight)
+    int eff;          // TFLOP/s of a launch that fills every slot (selection weight)
     bool buf;         // buffer-addressed direct loads: operands below 4 GiB only
     GemmKernel f16, bf16;
 };
 
-#define MVLM_TILE_X(BMv, BNv, BKv, Sv, WMv, WNv, PER_CU, EFF, BUFv)                                         \
-    TileCfg{BMv, BNv, BKv, Sv, WMv * WNv, PER_CU, EFF, BUFv, gemm_mfma_kernel<false, BMv, BNv, BKv, Sv, WMv, WNv, BUFv>, \
-            gemm_mfma_kernel<true, BMv, BNv, BKv, Sv, WMv, WNv, BUFv>}
-#define MVLM_TILE(BMv, BNv, BKv, Sv, WMv, WNv, PER_CU, EFF) MVLM_TILE_X(BMv, BNv, BKv, Sv, WMv, WNv, PER_CU, EFF, false)
-#define MVLM_TILE_B(BMv, BNv, BKv, Sv, WMv, WNv, PER_CU, EFF) MVLM_TILE_X(BMv, BNv, BKv, Sv, WMv, WNv, PER_CU, EFF, true)
-// The first nine are the automatic choices (eff measured at 4096^3, fp16 in,
-// fp32 out); the others are kept for tuning.  The 128-wide stages halve a
-// block's stage count (and its waits and barriers), which pays on the short-K
-// SigLIP shapes (729 x 1152 x 1152: 11.4 -> 9.4 us with 64 x 64 tiles; 729 x
-// 4304 x 1152: 18.7 -> 16.9 us with 128 x 128) and, as two 80 KiB stages of
-// 192 x 128, a little on 768-row shapes (~1%) and 1536 x 6144 x 2048 (73.3 ->
-// 70.1 us); the 64-wide 64 x 64 tile stays for the many-way K splits of
-// few-row products.  96 x 192 with six waves of 32 x 96 cuts 768 x 6144 into
-// exactly 256 blocks (192 with 192 x 128): 35.4 -> 34.3 us at that shape.
+#define MVLM_TILE(BMv, BNv, BKv, Sv, WMv, WNv, PER_CU, EFF)                                     \
+    TileCfg{BMv, BNv, BKv, Sv, WMv * WNv, PER_CU, EFF, false, gemm_mfma_kernel<false, BMv, BNv, BKv, Sv, WMv, WNv>, \
+            gemm_mfma_kernel<true, BMv, BNv, BKv, Sv, WMv, WNv>}
+#define MVLM_PINGPONG(NAv, NBv, UAv, Sv, EFF)                                                   \
+    TileCfg{NAv * UAv, NBv * 128, 64, Sv, 8, 1, EFF, true, gemm_pingpong_kernel<false, NAv, NBv, UAv, Sv>, \
+            gemm_pingpong_kernel<true, NAv, NBv, UAv, Sv>}
+// All but the last are the automatic choices.  eff: fp16 rate of a launch that
+// fills every slot at K = 2048 .. 4096.  Plain fp16 products, the tile's time
+// against the best tile with all waves in step: 4096^3 113 us (256 x 256; 134),
+// 1536 x 6144 x 2048 44 (256 x 256; 67), 2048 x 4096 x 600 16.6 (256 x 128; 18.0),
+// 768 x 6144 x 2048 28.3 (192 x 128; 31.9), 768 x 8192 x 2048 30.1 (192 x 128;
+// 33.7), 729 x 3456 x 1152 13.0 (128 x 128; 14.1), 729 x 4304 x 1152 13.5 (128 x
+// 128; 15.3), 2048^3 22.8 (128 x 128; 25.7).  A fifth slot for 128 x 128 (160
+// KiB) is slower, 13.9 us at 729 x 3456 x 1152.  Products of few tiles stay with
+// 64 x 64, two blocks to a CU: 729 x 1152 x 1152 takes 8.8 us with two 128-wide
+// stages, 12.8 with 128 x 128; 64-wide stages serve the many-way K splits of
+// few-row products.  128 x 128 in step (two 128-wide stages) serves operands
+// beyond the buffer descriptors' 4 GiB.
 static const TileCfg kTiles[] = {
-    MVLM_TILE_B(256, 256, 64, 2, 4, 2, 1, 907), MVLM_TILE_B(256, 128, 64, 2, 4, 2, 1, 785),
-    MVLM_TILE_B(192, 128, 64, 3, 2, 4, 1, 636), MVLM_TILE(128, 128, 64, 4, 4, 2, 1, 619),
-    MVLM_TILE(64, 64, 64, 4, 2, 2, 2, 401), MVLM_TILE(128, 128, 128, 2, 4, 2, 1, 682),
-    MVLM_TILE(64, 64, 128, 2, 2, 2, 2, 460), MVLM_TILE_B(192, 128, 128, 2, 2, 4, 1, 700),
-    MVLM_TILE_B(96, 192, 128, 2, 3, 2, 1, 564),
-    MVLM_TILE(256, 128, 64, 3, 4, 2, 1, 628), MVLM_TILE(128, 128, 64, 4, 2, 2, 1, 502),
-    MVLM_TILE(128, 64, 64, 4, 2, 2, 1, 375),
-    MVLM_TILE(256, 256, 32, 4, 4, 2, 1, 849), MVLM_TILE(256, 256, 32, 5, 4, 2, 1, 828),
-    MVLM_TILE(256, 128, 32, 6, 4, 2, 1, 686), MVLM_TILE(128, 128, 32, 8, 4, 2, 1, 541),
-    MVLM_TILE(128, 128, 32, 4, 4, 2, 2, 689), MVLM_TILE(192, 128, 32, 6, 2, 2, 1, 460),
+    MVLM_PINGPONG(2, 2, 128, 2, 1216), MVLM_PINGPONG(4, 1, 64, 3, 1000),
+    MVLM_PINGPONG(3, 1, 64, 4, 880), MVLM_PINGPONG(2, 1, 64, 4, 760),
+    MVLM_TILE(64, 64, 64, 4, 2, 2, 2, 401), MVLM_TILE(64, 64, 128, 2, 2, 2, 2, 460),
+    MVLM_TILE(128, 128, 128, 2, 4, 2, 1, 682),
+    MVLM_TILE(128, 128, 32, 4, 4, 2, 2, 689),
 };
-constexpr int kAutoTiles = 9;
+constexpr int kAutoTiles = 7;
 #undef MVLM_TILE
-#undef MVLM_TILE_B
-#undef MVLM_TILE_X
+#undef MVLM_PINGPONG
 
 struct GemmPlan {
     const TileCfg* tile;
@@ -553,8 +771,7 @@ static GemmPlan plan_gemm(int M, int N, int K, int batch, int num_cus, bool buf_
             const int64_t slots = (int64_t)num_cus * c.per_cu;
             const int64_t rounds = (tiles + slots - 1) / slots;
             const double block_flops = 2.0 * c.bm * c.bn * (double)ss * c.bk;
-            const double eff = c.eff > 0 ? c.eff : 100.0;              // unmeasured tuning tiles
-            double t = rounds * block_flops / (eff * 1e12 / (double)slots);
+            double t = rounds * block_flops / (c.eff * 1e12 / (double)slots);
             if (splits > 1) t += (double)M * N * batch * 4.0 * (2.0 * splits + 1.0) / 4e12 + 3e-6;
             if (t < best_t) { best_t = t; best = GemmPlan{&c, splits, ss}; }
         }
