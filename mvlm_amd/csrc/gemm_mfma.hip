@@ -78,6 +78,8 @@ struct GemmArgs {
     // aligned in C (vec_c) and in the split partials (vec_ws), so one vector
     // store writes them
     int vec_c, vec_ws;
+    // the epilogue's operands too, and N % 4 == 0: they are read four at a time
+    int vec_ep;
 };
 
 // fp32 partial of 4 consecutive columns (n_left of them below N; the row
@@ -92,13 +94,48 @@ __device__ __forceinline__ void store_partial4(float* ws, int64_t i, f32x4 v, in
         if (e < n_left) ws[i + e] = v[e];
 }
 
-// C row `row_off` (element offset of the row), columns col..col+3: epilogue,
-// output dtype, one 16- or 8-byte store when the row is aligned for it,
-// written through L2 (C is tens of MB at the prefill shapes)
-__device__ __forceinline__ void store_c4(const GemmArgs& p, int64_t row_off, int col, f32x4 v) {
+// Four consecutive epilogue operands (16-byte / 8-byte aligned), as stored and
+// widened.
+__device__ __forceinline__ u32x4 load_operand4(const void* base, int64_t i, int dtype) {
+    if (dtype == 0) return *reinterpret_cast<const u32x4*>((const float*)base + i);
+    const u32x2 h = *reinterpret_cast<const u32x2*>((const uint16_t*)base + i);
+    return u32x4{h[0], h[1], 0, 0};
+}
+__device__ __forceinline__ f32x4 widen_operand4(u32x4 r, int dtype) {
+    if (dtype == 0) return __builtin_bit_cast(f32x4, r);
+    const uint16_t h[4] = {(uint16_t)r[0], (uint16_t)(r[0] >> 16), (uint16_t)r[1], (uint16_t)(r[1] >> 16)};
+    f32x4 v;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] = dtype == 1 ? f16_bits_to_f32(h[e]) : bf16_bits_to_f32(h[e]);
+    return v;
+}
+// apply_epilogue's two halves on four consecutive columns, the operands loaded
+// before: act(v + bias), then * mul + res
+__device__ __forceinline__ f32x4 activate4(const Epilogue& e, f32x4 v, u32x4 bias) {
+    if (e.bias) v += widen_operand4(bias, e.dtype);
+    if (e.act == 1) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[i] = gelu_tanh(v[i]);
+    } else if (e.act == 2) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[i] = silu(v[i]);
+    }
+    return v;
+}
+__device__ __forceinline__ f32x4 combine4(const Epilogue& e, f32x4 v, u32x4 mul, u32x4 res) {
+    if (e.mul) v *= widen_operand4(mul, e.dtype);
+    if (e.res) v += widen_operand4(res, e.dtype);
+    return v;
+}
+
+// C row `row_off` (element offset of the row), columns col..col+3: epilogue
+// (`ep`; false where it has been applied), output dtype, one 16- or 8-byte
+// store when the row is aligned for it, written through L2 (C is tens of MB at
+// the prefill shapes)
+__device__ __forceinline__ void store_c4(const GemmArgs& p, int64_t row_off, int col, f32x4 v, bool ep) {
     const int n_left = p.N - col;
     if (n_left <= 0) return;
-    if (p.ep_on) {
+    if (ep) {
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
             const int64_t idx = row_off + col + e;
@@ -234,28 +271,75 @@ __device__ __forceinline__ void store_tiles(const GemmArgs& p, f32x16 (&acc)[TM]
     // banks apart), and reads it back as 4 consecutive columns per lane, 8 rows
     // per pass: 16-byte global stores, and per-element code (epilogue, dtype)
     // in a loop rather than unrolled over the 16 * TM * TN accumulators.
-    __syncthreads();   // every wave is done with the ring (all its loads have landed)
-    constexpr int CS = CSTAGE;
+    // The epilogue's operands are requested four columns at a time for GT tiles
+    // at once (all of a wave's, but for the 128 accumulators of 256 x 256),
+    // before the tiles pass through LDS: one wait for a group's operands and
+    // not one per operand and row (768 x 8192 x 2048 with bias and GELU: see
+    // the launch table below).  In-place operands are safe: an element's are
+    // read by the thread that later stores it.
+    constexpr int CS = CSTAGE, T = TM * TN, GT = T <= 4 ? T : 2;
+    static_assert(T % GT == 0, "whole groups");
     const int srow = lane >> 3, scol = (lane & 7) * 4;
+    const bool epv = !ws && p.vec_ep;
+    u32x4 bias[TN], mul[GT][4], res[GT][4];
+    auto load_group = [&](auto G) {
+        static_for<GT>([&](auto X) {
+            constexpr int x = decltype(X)::value, ij = decltype(G)::value * GT + x, i = ij / TN, j = ij % TN;
+            const int col = min(col_of(j) + scol, p.N - 4);
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+                const int64_t idx = c_off + (int64_t)min(row_of(i) + srow + 8 * t, p.M - 1) * p.ldc + col;
+                if (p.ep.mul) mul[x][t] = load_operand4(p.ep.mul, idx, p.ep.dtype);
+                if (p.ep.res) res[x][t] = load_operand4(p.ep.res, idx, p.ep.dtype);
+            }
+        });
+    };
+    if (epv) {
+        if (p.ep.bias)
+#pragma unroll
+            for (int j = 0; j < TN; ++j)
+                bias[j] = load_operand4(p.ep.bias, min(col_of(j) + scol, p.N - 4), p.ep.dtype);
+        load_group(std::integral_constant<int, 0>{});
+    }
+    __syncthreads();   // every wave is done with the ring (all its loads have landed)
     // (compile-time tile indices: a rolled tile loop would index acc at run time
     // and move it to scratch memory)
-    static_for<TM * TN>([&](auto IJ) {
-        constexpr int i = decltype(IJ)::value / TN, j = decltype(IJ)::value % TN;
-        {
+    static_for<T>([&](auto IJ) {
+        constexpr int ij = decltype(IJ)::value, i = ij / TN, j = ij % TN;
+        if constexpr (ij > 0 && ij % GT == 0)
+            if (epv) load_group(std::integral_constant<int, ij / GT>{});
 #pragma unroll
-            for (int r = 0; r < 16; ++r)
-                cst[(8 * (r >> 2) + 4 * (lane >> 5) + (r & 3)) * CS + (lane & 31)] = acc[i][j][r];
-            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // this wave's writes, before its reads
-            const int row0 = row_of(i), col = col_of(j) + scol;
+        for (int r = 0; r < 16; ++r)
+            cst[(8 * (r >> 2) + 4 * (lane >> 5) + (r & 3)) * CS + (lane & 31)] = acc[i][j][r];
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // this wave's writes, before its reads
+        const int row0 = row_of(i), col = col_of(j) + scol;
+        if (epv) {
+            // in a loop and back to LDS: unrolled over every element of the
+            // wave this code alone would be tens of KB, run once
+            if (p.ep.bias || p.ep.act) {
+#pragma unroll 1
+                for (int t = 0; t < 4; ++t) {
+                    f32x4* v = reinterpret_cast<f32x4*>(cst + (srow + 8 * t) * CS + scol);
+                    *v = activate4(p.ep, *v, bias[j]);
+                }
+            }
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+                const int row = row0 + srow + 8 * t;
+                const f32x4 v = combine4(p.ep, *reinterpret_cast<const f32x4*>(cst + (srow + 8 * t) * CS + scol),
+                                         mul[ij % GT][t], res[ij % GT][t]);
+                if (row < p.M) store_c4(p, c_off + (int64_t)row * p.ldc, col, v, false);
+            }
+        } else {
             for (int t = 0; t < 4; ++t) {
                 const int row = row0 + srow + 8 * t;
                 const f32x4 v = *reinterpret_cast<const f32x4*>(cst + (srow + 8 * t) * CS + scol);
                 if (row >= p.M) continue;
                 if (ws) store_partial4(ws, (int64_t)row * p.N + col, v, p.N - col);
-                else store_c4(p, c_off + (int64_t)row * p.ldc, col, v);
+                else store_c4(p, c_off + (int64_t)row * p.ldc, col, v, p.ep_on);
             }
-            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // reads done before the next tile's writes
         }
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // reads done before the next tile's writes
     });
 }
 
@@ -648,13 +732,33 @@ __global__ __launch_bounds__(512, 2) void gemm_pingpong_kernel(const GemmArgs p)
 // epilogue and stores C: thread = V consecutive output elements of the
 // flattened [M][N] (V = 4 reads the partials as 16-byte vectors; it needs
 // M*N % 4 == 0 so every split's partial stays 16-byte aligned).
-template <int V>
+template <int V, bool EP>
 __global__ __launch_bounds__(256) void gemm_splitk_reduce_kernel(const GemmArgs p) {
     const int64_t mn = (int64_t)p.M * p.N;
     const int64_t i0 = ((int64_t)blockIdx.x * 256 + threadIdx.x) * V;
     const int b = blockIdx.y;
     if (i0 >= mn) return;
     const float* ws = p.ws + (int64_t)b * p.splits * mn + i0;
+    if constexpr (V == 4) {
+        // N % 4 == 0: the four elements share a row, and with vec_c they are
+        // one aligned 16-byte (fp32) or 8-byte (16-bit) piece of C; the
+        // operands are requested before the first sum
+        if (p.vec_c && p.N % 4 == 0) {
+            const int row = (int)(i0 / p.N), col = (int)(i0 - (int64_t)row * p.N);
+            const int64_t idx = (int64_t)b * p.sC + (int64_t)row * p.ldc + col;
+            f32x4 acc = *reinterpret_cast<const f32x4*>(ws);
+            u32x4 bias{}, mul{}, res{};
+            if (EP && p.vec_ep) {
+                if (p.ep.bias) bias = load_operand4(p.ep.bias, col, p.ep.dtype);
+                if (p.ep.mul) mul = load_operand4(p.ep.mul, idx, p.ep.dtype);
+                if (p.ep.res) res = load_operand4(p.ep.res, idx, p.ep.dtype);
+            }
+            for (int s = 1; s < p.splits; ++s) acc += *reinterpret_cast<const f32x4*>(ws + s * mn);
+            if (EP && p.vec_ep) acc = combine4(p.ep, activate4(p.ep, acc, bias), mul, res);
+            store_c4(p, idx - col, col, acc, EP && !p.vec_ep);
+            return;
+        }
+    }
     float v[V];
     if constexpr (V == 4) {
         f32x4 acc = *reinterpret_cast<const f32x4*>(ws);
@@ -664,22 +768,12 @@ __global__ __launch_bounds__(256) void gemm_splitk_reduce_kernel(const GemmArgs 
         v[0] = 0.0f;
         for (int s = 0; s < p.splits; ++s) v[0] += ws[s * mn];
     }
-    if constexpr (V == 4) {
-        // N % 4 == 0: the four elements share a row, and with vec_c they are
-        // one aligned 16-byte (fp32) or 8-byte (16-bit) piece of C
-        if (p.vec_c && p.N % 4 == 0) {
-            const int row = (int)(i0 / p.N), col = (int)(i0 - (int64_t)row * p.N);
-            const int64_t idx = (int64_t)b * p.sC + (int64_t)row * p.ldc + col;
-            store_c4(p, idx - col, col, (f32x4){v[0], v[1], v[2], v[3]});
-            return;
-        }
-    }
 #pragma unroll
     for (int e = 0; e < V; ++e) {
         const int64_t i = i0 + e;
         const int row = (int)(i / p.N), col = (int)(i - (int64_t)row * p.N);
         const int64_t idx = (int64_t)b * p.sC + (int64_t)row * p.ldc + col;
-        store_out(p.C, idx, p.ep_on ? apply_epilogue(p.ep, v[e], idx, col) : v[e], p.c_dtype);
+        store_out(p.C, idx, EP ? apply_epilogue(p.ep, v[e], idx, col) : v[e], p.c_dtype);
     }
 }
 
@@ -869,6 +963,8 @@ hipError_t launch_gemm_mfma(hipStream_t s, const void* A, int ab_dtype, const vo
         const int es = c_dtype == MVLM_F32 ? 4 : 2;
         a.vec_c = ((uintptr_t)C % (4 * es) == 0) && (ldc % 4 == 0) && (strideC % 4 == 0);
         a.vec_ws = N % 4 == 0;
+        const uintptr_t operands = (uintptr_t)a.ep.bias | (uintptr_t)a.ep.mul | (uintptr_t)a.ep.res;
+        a.vec_ep = a.ep_on && a.vec_c && N % 4 == 0 && operands % (4 * es) == 0;
     }
     const int n = (int)w.pad_a + (int)w.pad_b + 1 + (g.splits > 1 ? 1 : 0);
     int idx = 0;
@@ -891,12 +987,10 @@ hipError_t launch_gemm_mfma(hipStream_t s, const void* A, int ab_dtype, const vo
     launch_seq(idx++, n, k, grid, dim3(64 * t.waves), s, a);
     if (g.splits > 1) {
         const int64_t mn = (int64_t)M * N;
-        if (mn % 4 == 0)
-            launch_seq(idx++, n, gemm_splitk_reduce_kernel<4>, dim3((unsigned)((mn / 4 + 255) / 256), (unsigned)batch),
-                       dim3(256), s, a);
-        else
-            launch_seq(idx++, n, gemm_splitk_reduce_kernel<1>, dim3((unsigned)((mn + 255) / 256), (unsigned)batch),
-                       dim3(256), s, a);
+        const int v = mn % 4 == 0 ? 4 : 1;
+        const auto reduce = v == 4 ? (a.ep_on ? gemm_splitk_reduce_kernel<4, true> : gemm_splitk_reduce_kernel<4, false>)
+                                   : (a.ep_on ? gemm_splitk_reduce_kernel<1, true> : gemm_splitk_reduce_kernel<1, false>);
+        launch_seq(idx++, n, reduce, dim3((unsigned)((mn / v + 255) / 256), (unsigned)batch), dim3(256), s, a);
     }
     return hipGetLastError();
 }
