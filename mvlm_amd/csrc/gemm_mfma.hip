@@ -274,9 +274,11 @@ __device__ __forceinline__ void store_tiles(const GemmArgs& p, f32x16 (&acc)[TM]
     // The epilogue's operands are requested four columns at a time for GT tiles
     // at once (all of a wave's, but for the 128 accumulators of 256 x 256),
     // before the tiles pass through LDS: one wait for a group's operands and
-    // not one per operand and row (768 x 8192 x 2048 with bias and GELU: see
-    // the launch table below).  In-place operands are safe: an element's are
-    // read by the thread that later stores it.
+    // not one per element, which with a tanhf per element made 768 x 8192 x
+    // 2048 with bias and GELU take 51 us against 34 without; a Phi-1.5 block of
+    // 768 rows went 170 -> 153 us, a SigLIP block of 729 101 -> 91.  In-place
+    // operands are safe: an element's are read by the thread that later stores
+    // it.
     constexpr int CS = CSTAGE, T = TM * TN, GT = T <= 4 ? T : 2;
     static_assert(T % GT == 0, "whole groups");
     const int srow = lane >> 3, scol = (lane & 7) * 4;
@@ -315,7 +317,8 @@ __device__ __forceinline__ void store_tiles(const GemmArgs& p, f32x16 (&acc)[TM]
         const int row0 = row_of(i), col = col_of(j) + scol;
         if (epv) {
             // in a loop and back to LDS: unrolled over every element of the
-            // wave this code alone would be tens of KB, run once
+            // wave this code alone would be tens of KB, run once (the Phi-1.5
+            // block: 159 -> 153 us)
             if (p.ep.bias || p.ep.act) {
 #pragma unroll 1
                 for (int t = 0; t < 4; ++t) {

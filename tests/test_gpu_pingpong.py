@@ -1,12 +1,13 @@
-"""The tiles whose two wave groups alternate (gemm_pingpong_kernel), forced, where the phase tables, the ring and
+"""The GEMM tiles whose two wave groups alternate (gemm_pingpong_kernel), forced, where the phase tables, the ring and
 the out-of-range loads can go wrong: fewer stages than ring slots, odd and even stage counts, K tails, partial tiles,
-K splits whose last part is short, batches."""
+K splits whose last part is short, batches; and the store pass with its epilogue."""
 import numpy as np
 import pytest
 
 import mvlm_amd as m
-from mvlm_amd import BF16, F16, F32
-from test_gpu_parity import check_packed, within
+from mvlm_amd import BF16, F16, F32, native
+from test_gpu_epilogue import check, from_storage, make_operands, to_storage
+from test_gpu_parity import check_packed, gen, widen, within
 
 pytestmark = pytest.mark.gpu
 
@@ -53,3 +54,46 @@ def test_batches(dev, orc, monkeypatch, tile):
         _, bound = orc.gemm_f64(orc.f16_to_f32(a).astype(np.float64), orc.f16_to_f32(b).astype(np.float64), S, S, D)
         ok, worst = within(got[h, :S * S].reshape(S, S), ref, bound, 1e-3)
         assert ok, (h, worst)
+
+
+@pytest.mark.parametrize("tile", TILES + ["64x64s4w4", "64x64s2w4k128"])
+@pytest.mark.parametrize("dt,offset,splits,act,names", [
+    (F32, 0, 1, native.ACT_GELU_TANH, ("bias", "mul", "residual")),
+    (F16, 0, 1, native.ACT_SILU, ("bias", "residual")),
+    (BF16, 0, 1, native.ACT_NONE, ("bias", "mul")),
+    (F16, 1, 1, native.ACT_GELU_TANH, ("bias", "residual")),     # operands off the 8-byte grid: read one by one
+    (F16, 0, 2, native.ACT_GELU_TANH, ("bias", "mul", "residual")),   # applied by the split-K reduction
+])
+def test_epilogue(dev, orc, monkeypatch, tile, dt, offset, splits, act, names):
+    """operands read four columns at a time for groups of tiles: rows and columns that end inside a tile"""
+    monkeypatch.setenv("MVLM_GEMM_TILE", tile)
+    monkeypatch.setenv("MVLM_GEMM_SPLITS", str(splits))
+    M, N, K, ab = 201, 332, 520, BF16 if dt == BF16 else F16
+    A, Wt = gen(orc, ab, M * K, 0x430), gen(orc, ab, N * K, 0x431, 0.05)
+    _, vals = make_operands(dev, orc, M, N, dt, 0x432, *(n in names for n in ("bias", "mul", "residual")))
+    es = 4 if dt == F32 else 2
+    ops = {}
+    for n in names:
+        raw = to_storage(orc, vals[n].astype(np.float32), dt)[0]
+        buf = dev.upload(np.concatenate([np.zeros(offset, raw.dtype), raw]))
+        ops[n] = buf.view(offset * es, raw.size * es) if offset else buf
+    C = dev.alloc(M * N * es)
+    dev.gemm_packed_ex(dev.upload(A), ab, dev.pack(Wt, ab, N, K), C, dt, M, N, K, act=act, **ops)
+    got = from_storage(orc, C.download(np.float32 if dt == F32 else np.uint16, M * N), dt).reshape(M, N)
+    Y64, S = orc.gemm_f64(widen(orc, A, ab).reshape(M, K), widen(orc, Wt, ab).reshape(N, K), M, N, K)
+    check(orc, got, Y64, S, vals, act, dt, 1e-4)
+
+
+def test_gelu_extremes(dev, orc):
+    """the values that the tanh form gives: inf and large x pass, large -x is zero, -inf (0 times inf) is NaN"""
+    x = np.array([np.inf, 65504.0, 12.0, 0.0, -12.0, -65504.0, -np.inf, np.nan], np.float16)
+    A = np.zeros((x.size, 8), np.float16)
+    A[:, 0] = x
+    Wt = np.zeros((4, 8), np.float16)
+    Wt[:, 0] = 1.0
+    C = dev.alloc(x.size * 4 * 4)
+    dev.gemm_packed_ex(dev.upload(A.view(np.uint16)), F16, dev.pack(Wt.view(np.uint16), F16, 4, 8), C, F32, x.size, 4, 8,
+                       act=native.ACT_GELU_TANH)
+    got = C.download(np.float32).reshape(x.size, 4)[:, 0]
+    assert np.array_equal(got[:6], np.float32([np.inf, 65504.0, 12.0, 0.0, 0.0, 0.0])), got
+    assert np.isnan(got[6:]).all(), got
