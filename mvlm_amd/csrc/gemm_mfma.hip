@@ -271,6 +271,30 @@ __device__ __forceinline__ void store_tiles(const GemmArgs& p, f32x16 (&acc)[TM]
     // banks apart), and reads it back as 4 consecutive columns per lane, 8 rows
     // per pass: 16-byte global stores, and per-element code (epilogue, dtype)
     // in a loop rather than unrolled over the 16 * TM * TN accumulators.
+    constexpr int CS = CSTAGE, T = TM * TN, GT = T <= 4 ? T : 2;
+    static_assert(T % GT == 0, "whole groups");
+    const int srow = lane >> 3, scol = (lane & 7) * 4;
+    auto stage_tile = [&](f32x16& c) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) cst[(8 * (r >> 2) + 4 * (lane >> 5) + (r & 3)) * CS + (lane & 31)] = c[r];
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // this wave's writes, before its reads
+    };
+    // (compile-time tile indices: a rolled tile loop would index acc at run time
+    // and move it to scratch memory)
+    if (ws) {
+        __syncthreads();   // every wave is done with the ring (all its loads have landed)
+        static_for<T>([&](auto IJ) {
+            constexpr int ij = decltype(IJ)::value, i = ij / TN, j = ij % TN;
+            stage_tile(acc[i][j]);
+            for (int t = 0; t < 4; ++t) {
+                const int row = row_of(i) + srow + 8 * t, col = col_of(j) + scol;
+                const f32x4 v = *reinterpret_cast<const f32x4*>(cst + (srow + 8 * t) * CS + scol);
+                if (row < p.M) store_partial4(ws, (int64_t)row * p.N + col, v, p.N - col);
+            }
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // reads done before the next tile's writes
+        });
+        return;
+    }
     // The epilogue's operands are requested four columns at a time for GT tiles
     // at once (all of a wave's, but for the 128 accumulators of 256 x 256),
     // before the tiles pass through LDS: one wait for a group's operands and
@@ -279,10 +303,7 @@ __device__ __forceinline__ void store_tiles(const GemmArgs& p, f32x16 (&acc)[TM]
     // 768 rows went 170 -> 153 us, a SigLIP block of 729 101 -> 91.  In-place
     // operands are safe: an element's are read by the thread that later stores
     // it.
-    constexpr int CS = CSTAGE, T = TM * TN, GT = T <= 4 ? T : 2;
-    static_assert(T % GT == 0, "whole groups");
-    const int srow = lane >> 3, scol = (lane & 7) * 4;
-    const bool epv = !ws && p.vec_ep;
+    const bool epv = p.vec_ep;
     u32x4 bias[TN], mul[GT][4], res[GT][4];
     auto load_group = [&](auto G) {
         static_for<GT>([&](auto X) {
@@ -303,17 +324,12 @@ __device__ __forceinline__ void store_tiles(const GemmArgs& p, f32x16 (&acc)[TM]
                 bias[j] = load_operand4(p.ep.bias, min(col_of(j) + scol, p.N - 4), p.ep.dtype);
         load_group(std::integral_constant<int, 0>{});
     }
-    __syncthreads();   // every wave is done with the ring (all its loads have landed)
-    // (compile-time tile indices: a rolled tile loop would index acc at run time
-    // and move it to scratch memory)
+    __syncthreads();   // the ring is idle, as above
     static_for<T>([&](auto IJ) {
         constexpr int ij = decltype(IJ)::value, i = ij / TN, j = ij % TN;
         if constexpr (ij > 0 && ij % GT == 0)
             if (epv) load_group(std::integral_constant<int, ij / GT>{});
-#pragma unroll
-        for (int r = 0; r < 16; ++r)
-            cst[(8 * (r >> 2) + 4 * (lane >> 5) + (r & 3)) * CS + (lane & 31)] = acc[i][j][r];
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // this wave's writes, before its reads
+        stage_tile(acc[i][j]);
         const int row0 = row_of(i), col = col_of(j) + scol;
         if (epv) {
             // in a loop and back to LDS: unrolled over every element of the
@@ -338,8 +354,7 @@ __device__ __forceinline__ void store_tiles(const GemmArgs& p, f32x16 (&acc)[TM]
                 const int row = row0 + srow + 8 * t;
                 const f32x4 v = *reinterpret_cast<const f32x4*>(cst + (srow + 8 * t) * CS + scol);
                 if (row >= p.M) continue;
-                if (ws) store_partial4(ws, (int64_t)row * p.N + col, v, p.N - col);
-                else store_c4(p, c_off + (int64_t)row * p.ldc, col, v, p.ep_on);
+                store_c4(p, c_off + (int64_t)row * p.ldc, col, v, p.ep_on);
             }
         }
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // reads done before the next tile's writes
