@@ -414,8 +414,9 @@ __global__ __launch_bounds__(64 * SK_WAVES) void gemm_skinny_kernel(const Skinny
                         sum[1] += from[w * 256 + 64];
                     }
                     if (ep) {
-                        // requested before the codes of the batch's refills
-                        if (ub + SK_BATCH + L::DEPTH <= u1) asm_wait_vmcnt<SK_BATCH * L::NDMA>();
+                        // requested before the codes of the batch's refills, of
+                        // which a wave without blocks has none
+                        if (cnt > 0 && ub + SK_BATCH + L::DEPTH <= u1) asm_wait_vmcnt<SK_BATCH * L::NDMA>();
                         else asm_wait_vmcnt<0>();
                         float v[SK_EP_LOADS];
 #pragma unroll

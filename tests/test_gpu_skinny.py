@@ -82,6 +82,24 @@ def test_epilogue_operands(dev, orc, qt, M, ep):
         assert ok, (N, K, worst)
 
 
+# blocks of K that leave the last or most of the eight waves of a workgroup
+# without work, and enough row groups per workgroup (10 and more for Q8_0, 12
+# for Q4_0) that epilogue operands are requested again while codes still follow
+@pytest.mark.parametrize("qt,N,K", [(Q8, 40005, 28 * 32), (Q8, 40005, 9 * 32), (Q8, 57301, 2 * 32),
+                                    (Q4, 50005, 28 * 32), (Q4, 50005, 18 * 32), (Q4, 57301, 2 * 32)])
+@pytest.mark.parametrize("M", [5, 9, 16])
+def test_epilogue_of_waves_without_blocks(dev, orc, qt, N, K, M):
+    X, blocks = orc.normal_f32(M * K, 671), make_quant(orc, qt, N, K, 672)
+    ref, S = reference(orc, qt, X, blocks, M, N, K)
+    bias, mul, res = orc.normal_f32(N, 673), orc.normal_f32(M * N, 674).reshape(M, N), orc.normal_f32(M * N, 675).reshape(M, N)
+    y = dev.upload(np.full(M * N, np.nan, np.float32))
+    dev.gemm_quant_grouped(M, [(dev.upload(X), F32, dev.pack(blocks, qt, N, K), y, F32)],
+                           epilogues=[{"bias": dev.upload(bias), "mul": dev.upload(mul), "residual": dev.upload(res)}])
+    want = (ref.astype(np.float64) + bias) * mul + res
+    ok, worst = within(y.download(np.float32).reshape(M, N), want, (S + np.abs(bias)) * np.abs(mul) + np.abs(res), 1e-5)
+    assert ok, worst
+
+
 @pytest.mark.parametrize("qt", [Q8, Q4])
 def test_not_a_number_stays_in_its_row(dev, orc, qt):
     M, N, K = 9, 70, 300 * 32
