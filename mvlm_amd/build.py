@@ -76,7 +76,11 @@ def _compile(src: str) -> str:
         raise RuntimeError(f"hipcc failed for {src}:\n{' '.join(cmd)}\n{msgs}")
     if msgs.strip():
         print(msgs, file=sys.stderr)
-    bad = _stack_kernels("\n".join(l.split("remark: ", 1)[1] for l in out.splitlines() if "remark: " in l))
+    remarks = "\n".join(l.split("remark: ", 1)[1] for l in out.splitlines() if "remark: " in l)
+    if src.endswith(".hip"):
+        with open(usage_path(src), "w") as f:
+            f.write(remarks)
+    bad = _stack_kernels(remarks)
     if bad:
         os.remove(obj)
         raise RuntimeError(f"{src}: kernels with scratch memory beyond their register spills:\n  " + "\n  ".join(bad))
@@ -87,8 +91,15 @@ def _object(src: str) -> str:
     return os.path.join(OBJ, os.path.relpath(src, PKG).replace(os.sep, "_") + ".o")
 
 
+def usage_path(src: str) -> str:
+    """Where the compiler's kernel-resource-usage remarks of a source are kept."""
+    return _object(src)[:-2] + ".usage.txt"
+
+
 def _stale(src: str, newest_header: float) -> bool:
     obj = _object(src)
+    if src.endswith(".hip") and not os.path.exists(usage_path(src)):
+        return True
     return not os.path.exists(obj) or os.path.getmtime(obj) < max(os.path.getmtime(src), newest_header)
 
 

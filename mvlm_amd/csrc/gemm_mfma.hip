@@ -215,7 +215,7 @@ __device__ __forceinline__ void stage_guarded(const uint16_t* __restrict__ base,
 // partials ws: tile (i, j) has its first element at row row_of(i), column
 // col_of(j).  cst: the wave's 32 x CSTAGE floats of LDS staging.
 constexpr int CSTAGE = 36;
-template <int TM, int TN, typename RowOf, typename ColOf>
+template <int TM, int TN, int GT, typename RowOf, typename ColOf>
 __device__ __forceinline__ void store_tiles(const GemmArgs& p, f32x16 (&acc)[TM][TN], float* cst, int64_t c_off,
                                             float* ws, int lane, RowOf row_of, ColOf col_of) {
     const bool vec = ws ? p.vec_ws : p.vec_c;
@@ -271,7 +271,7 @@ __device__ __forceinline__ void store_tiles(const GemmArgs& p, f32x16 (&acc)[TM]
     // banks apart), and reads it back as 4 consecutive columns per lane, 8 rows
     // per pass: 16-byte global stores, and per-element code (epilogue, dtype)
     // in a loop rather than unrolled over the 16 * TM * TN accumulators.
-    constexpr int CS = CSTAGE, T = TM * TN, GT = T <= 4 ? T : 2;
+    constexpr int CS = CSTAGE, T = TM * TN;
     static_assert(T % GT == 0, "whole groups");
     const int srow = lane >> 3, scol = (lane & 7) * 4;
     auto stage_tile = [&](f32x16& c) {
@@ -361,8 +361,11 @@ __device__ __forceinline__ void store_tiles(const GemmArgs& p, f32x16 (&acc)[TM]
     });
 }
 
-template <bool BF16, int BM, int BN, int BK, int STAGES, int WGM, int WGN>
-__global__ __launch_bounds__(64 * WGM * WGN) void gemm_mfma_kernel(const GemmArgs p) {
+// PER_CU blocks are resident on a CU: the registers of their waves must fit too.
+// (128 x 128 with 32-wide stages and the operands of two tiles held at once took
+// 132 registers, one block instead of two: 3264 x 20864 x 128 104 us, now 82.)
+template <bool BF16, int BM, int BN, int BK, int STAGES, int WGM, int WGN, int PER_CU>
+__global__ __launch_bounds__(64 * WGM * WGN, PER_CU* WGM* WGN > 8 ? PER_CU * WGM * WGN / 4 : 2) void gemm_mfma_kernel(const GemmArgs p) {
     using G = StageGeom<BK>;
     constexpr int ROWH = G::ROWH;
     constexpr int NW = WGM * WGN;                // waves per block (WGM x WGN grid)
@@ -507,7 +510,8 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_mfma_kernel(const GemmArg
 
     const int64_t c_off = (int64_t)batch * p.sC;
     float* ws = p.splits > 1 ? p.ws + (int64_t)blockIdx.z * p.M * p.N : nullptr;
-    store_tiles<TM, TN>(p, acc, reinterpret_cast<float*>(smem) + wave * 32 * CSTAGE, c_off, ws, lane,
+    constexpr int GT = PER_CU * NW > 8 ? 1 : TM * TN;   // four waves to a SIMD: 128 registers each
+    store_tiles<TM, TN, GT>(p, acc, reinterpret_cast<float*>(smem) + wave * 32 * CSTAGE, c_off, ws, lane,
                         [&](int i) { return m0 + wm * WM + i * 32; }, [&](int j) { return n0 + wn * WN + j * 32; });
 }
 
@@ -741,7 +745,7 @@ __global__ __launch_bounds__(512, 2) void gemm_pingpong_kernel(const GemmArgs p)
 
     const int64_t c_off = (int64_t)batch * p.sC;
     float* ws = p.splits > 1 ? p.ws + (int64_t)blockIdx.z * p.M * p.N : nullptr;
-    store_tiles<NA * TA, NB>(p, acc, reinterpret_cast<float*>(smem) + wave * 32 * CSTAGE, c_off, ws, lane,
+    store_tiles<NA * TA, NB, NA * TA * NB <= 4 ? NA * TA * NB : 2>(p, acc, reinterpret_cast<float*>(smem) + wave * 32 * CSTAGE, c_off, ws, lane,
                              [&](int i) { return m0 + UA * (i / TA) + wm * (UA / 2) + 32 * (i % TA); },
                              [&](int j) { return n0 + 128 * j + wn * 32; });
 }
@@ -808,8 +812,8 @@ struct TileCfg {
 };
 
 #define MVLM_TILE(BMv, BNv, BKv, Sv, WMv, WNv, PER_CU, EFF)                                     \
-    TileCfg{BMv, BNv, BKv, Sv, WMv * WNv, PER_CU, EFF, false, gemm_mfma_kernel<false, BMv, BNv, BKv, Sv, WMv, WNv>, \
-            gemm_mfma_kernel<true, BMv, BNv, BKv, Sv, WMv, WNv>}
+    TileCfg{BMv, BNv, BKv, Sv, WMv * WNv, PER_CU, EFF, false, gemm_mfma_kernel<false, BMv, BNv, BKv, Sv, WMv, WNv, PER_CU>, \
+            gemm_mfma_kernel<true, BMv, BNv, BKv, Sv, WMv, WNv, PER_CU>}
 #define MVLM_PINGPONG(NAv, NBv, UAv, Sv, EFF)                                                   \
     TileCfg{NAv * UAv, NBv * 128, 64, Sv, 8, 1, EFF, true, gemm_pingpong_kernel<false, NAv, NBv, UAv, Sv>, \
             gemm_pingpong_kernel<true, NAv, NBv, UAv, Sv>}

@@ -61,3 +61,23 @@ def test_compiler_remarks_have_the_parsed_fields(tmp_path):
     assert re.search(r"ScratchSize \[bytes/lane\]: \d+", remarks)
     bad = build._stack_kernels(remarks)
     assert len(bad) == 1 and "_Z1kPKiPf" in bad[0]
+
+
+def test_tiles_that_share_a_cu_fit_its_registers():
+    """The GEMM's tile table says how many blocks of a tile are resident on a CU
+    (the kernel's last template argument); a tile of 8 waves of which two share
+    one needs 4 waves on each of the CU's 4 SIMDs, i.e. at most 128 registers."""
+    path = build.usage_path(os.path.join(build.CSRC, "gemm_mfma.hip"))
+    if not os.path.exists(path):
+        build.build(verbose=False)
+    seen = 0
+    for block in open(path).read().split("Function Name: ")[1:]:
+        name = block.split()[0]
+        if "gemm_mfma_kernel" not in name:
+            continue
+        args = [int(v) for v in re.findall(r"L[bi](\d+)E", name)]
+        wgm, wgn, per_cu = args[-3:]
+        occupancy = int(re.search(r"Occupancy \[waves/SIMD\]: (\d+)", block).group(1))
+        assert occupancy * 4 >= per_cu * wgm * wgn, (name, occupancy)
+        seen += per_cu == 2 and wgm * wgn == 8
+    assert seen >= 2        # fp16 and bf16
