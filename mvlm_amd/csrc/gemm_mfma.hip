@@ -211,48 +211,31 @@ __device__ __forceinline__ void stage_guarded(const uint16_t* __restrict__ base,
     }
 }
 
-// The wave's TM x TN accumulator tiles to C (with the epilogue) or to the split
-// partials ws: tile (i, j) has its first element at row row_of(i), column
-// col_of(j).  cst: the wave's 32 x CSTAGE floats of LDS staging.
+// The wave's TM x TN accumulator tiles to C, with the epilogue (EP) or without,
+// or (not EP) to the split partials ws: tile (i, j) has its first element at row
+// row_of(i), column col_of(j).  cst: the wave's 32 x CSTAGE floats of LDS
+// staging.  EP is a kernel of its own: code that a launch jumps over costs it
+// instruction fetches.  With one kernel for both, 64 x 2048 x 64 took 6.0 us (now
+// 5.6), 4 x 64 x 320 with bias and GELU 6.7 (5.4), 4096^3 114 (111).
 constexpr int CSTAGE = 36;
-template <int TM, int TN, int GT, typename RowOf, typename ColOf>
+template <bool EP, int TM, int TN, int GT, typename RowOf, typename ColOf>
 __device__ __forceinline__ void store_tiles(const GemmArgs& p, f32x16 (&acc)[TM][TN], float* cst, int64_t c_off,
                                             float* ws, int lane, RowOf row_of, ColOf col_of) {
-    const bool vec = ws ? p.vec_ws : p.vec_c;
-    if (!vec) {   // rows off the vector grid: straight from the accumulators, 32 columns per row
-        if (ws) {
+    if (!(!EP && ws ? p.vec_ws : p.vec_c)) {   // rows off the vector grid: straight from the accumulators, 32 columns per row
 #pragma unroll
-            for (int i = 0; i < TM; ++i)
+        for (int i = 0; i < TM; ++i)
 #pragma unroll
-                for (int j = 0; j < TN; ++j) {
-                    const int col = col_of(j) + (lane & 31);
-                    if (col >= p.N) continue;
-#pragma unroll
-                    for (int r = 0; r < 16; ++r) {
-                        const int row = row_of(i) + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
-                        if (row < p.M) ws[(int64_t)row * p.N + col] = acc[i][j][r];
-                    }
-                }
-        } else if (!p.ep_on) {
-#pragma unroll
-            for (int i = 0; i < TM; ++i)
-#pragma unroll
-                for (int j = 0; j < TN; ++j) {
-                    const int col = col_of(j) + (lane & 31);
-                    if (col >= p.N) continue;
+            for (int j = 0; j < TN; ++j) {
+                const int col = col_of(j) + (lane & 31);
+                if (col >= p.N) continue;
+                auto each_row = [&](auto&& put) {
 #pragma unroll
                     for (int r = 0; r < 16; ++r) {
                         const int row = row_of(i) + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
-                        if (row < p.M) store_out(p.C, c_off + (int64_t)row * p.ldc + col, acc[i][j][r], p.c_dtype);
+                        if (row < p.M) put(row, acc[i][j][r]);
                     }
-                }
-        } else {   // fused epilogue: the per-element code is larger, so only the tile loops unroll
-#pragma unroll
-            for (int i = 0; i < TM; ++i)
-#pragma unroll
-                for (int j = 0; j < TN; ++j) {
-                    const int col = col_of(j) + (lane & 31);
-                    if (col >= p.N) continue;
+                };
+                if constexpr (EP) {   // the per-element code is larger: a quarter of the rows unrolled
 #pragma unroll 4
                     for (int r = 0; r < 16; ++r) {
                         const int row = row_of(i) + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
@@ -261,8 +244,12 @@ __device__ __forceinline__ void store_tiles(const GemmArgs& p, f32x16 (&acc)[TM]
                             store_out(p.C, idx, apply_epilogue(p.ep, acc[i][j][r], idx, col), p.c_dtype);
                         }
                     }
+                } else if (ws) {
+                    each_row([&](int row, float v) { ws[(int64_t)row * p.N + col] = v; });
+                } else {
+                    each_row([&](int row, float v) { store_out(p.C, c_off + (int64_t)row * p.ldc + col, v, p.c_dtype); });
                 }
-        }
+            }
         return;
     }
     // Aligned rows: through LDS.  Each wave writes one 32x32 accumulator tile
@@ -274,48 +261,36 @@ __device__ __forceinline__ void store_tiles(const GemmArgs& p, f32x16 (&acc)[TM]
     constexpr int CS = CSTAGE, T = TM * TN;
     static_assert(T % GT == 0, "whole groups");
     const int srow = lane >> 3, scol = (lane & 7) * 4;
+    // passes of 8 rows that a tile whose first row is row0 has inside C
+    auto passes = [&](int row0) { return min(4, (p.M - row0 + 7) >> 3); };
     auto stage_tile = [&](f32x16& c) {
 #pragma unroll
         for (int r = 0; r < 16; ++r) cst[(8 * (r >> 2) + 4 * (lane >> 5) + (r & 3)) * CS + (lane & 31)] = c[r];
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // this wave's writes, before its reads
     };
-    // (compile-time tile indices: a rolled tile loop would index acc at run time
-    // and move it to scratch memory)
-    if (ws) {
-        __syncthreads();   // every wave is done with the ring (all its loads have landed)
-        static_for<T>([&](auto IJ) {
-            constexpr int ij = decltype(IJ)::value, i = ij / TN, j = ij % TN;
-            stage_tile(acc[i][j]);
-            for (int t = 0; t < 4; ++t) {
-                const int row = row_of(i) + srow + 8 * t, col = col_of(j) + scol;
-                const f32x4 v = *reinterpret_cast<const f32x4*>(cst + (srow + 8 * t) * CS + scol);
-                if (row < p.M) store_partial4(ws, (int64_t)row * p.N + col, v, p.N - col);
-            }
-            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // reads done before the next tile's writes
-        });
-        return;
-    }
     // The epilogue's operands are requested four columns at a time for GT tiles
-    // at once (all of a wave's, but for the 128 accumulators of 256 x 256),
-    // before the tiles pass through LDS: one wait for a group's operands and
-    // not one per element, which with a tanhf per element made 768 x 8192 x
-    // 2048 with bias and GELU take 51 us against 34 without; a Phi-1.5 block of
-    // 768 rows went 170 -> 153 us, a SigLIP block of 729 101 -> 91.  In-place
-    // operands are safe: an element's are read by the thread that later stores
-    // it.
-    const bool epv = p.vec_ep;
+    // at once (all of a wave's, but for the 128 accumulators of 256 x 256 and
+    // tiles of which two share a CU), before the tiles pass through LDS: one wait
+    // for a group's operands and not one per element, which with a tanhf per
+    // element made 768 x 8192 x 2048 with bias and GELU take 51 us against 34
+    // without; a Phi-1.5 block of 768 rows went 170 -> 153 us, a SigLIP block of
+    // 729 101 -> 91.  In-place operands are safe: an element's are read by the
+    // thread that later stores it.
+    const bool epv = EP && p.vec_ep;
     u32x4 bias[TN], mul[GT][4], res[GT][4];
     auto load_group = [&](auto G) {
-        static_for<GT>([&](auto X) {
-            constexpr int x = decltype(X)::value, ij = decltype(G)::value * GT + x, i = ij / TN, j = ij % TN;
-            const int col = min(col_of(j) + scol, p.N - 4);
+        auto each = [&](const void* base, u32x4 (&to)[GT][4]) {
+            static_for<GT>([&](auto X) {
+                constexpr int x = decltype(X)::value, ij = decltype(G)::value * GT + x, i = ij / TN, j = ij % TN;
+                const int col = min(col_of(j) + scol, p.N - 4);
 #pragma unroll
-            for (int t = 0; t < 4; ++t) {
-                const int64_t idx = c_off + (int64_t)min(row_of(i) + srow + 8 * t, p.M - 1) * p.ldc + col;
-                if (p.ep.mul) mul[x][t] = load_operand4(p.ep.mul, idx, p.ep.dtype);
-                if (p.ep.res) res[x][t] = load_operand4(p.ep.res, idx, p.ep.dtype);
-            }
-        });
+                for (int t = 0; t < 4; ++t)
+                    to[x][t] = load_operand4(base, c_off + (int64_t)min(row_of(i) + srow + 8 * t, p.M - 1) * p.ldc + col,
+                                             p.ep.dtype);
+            });
+        };
+        if (p.ep.mul) each(p.ep.mul, mul);
+        if (p.ep.res) each(p.ep.res, res);
     };
     if (epv) {
         if (p.ep.bias)
@@ -324,20 +299,22 @@ __device__ __forceinline__ void store_tiles(const GemmArgs& p, f32x16 (&acc)[TM]
                 bias[j] = load_operand4(p.ep.bias, min(col_of(j) + scol, p.N - 4), p.ep.dtype);
         load_group(std::integral_constant<int, 0>{});
     }
-    __syncthreads();   // the ring is idle, as above
+    __syncthreads();   // every wave is done with the ring (all its loads have landed)
+    // (compile-time tile indices: a rolled tile loop would index acc at run time
+    // and move it to scratch memory)
     static_for<T>([&](auto IJ) {
         constexpr int ij = decltype(IJ)::value, i = ij / TN, j = ij % TN;
         if constexpr (ij > 0 && ij % GT == 0)
             if (epv) load_group(std::integral_constant<int, ij / GT>{});
         stage_tile(acc[i][j]);
-        const int row0 = row_of(i), col = col_of(j) + scol;
+        const int row0 = row_of(i), col = col_of(j) + scol, nt = passes(row0);
         if (epv) {
             // in a loop and back to LDS: unrolled over every element of the
             // wave this code alone would be tens of KB, run once (the Phi-1.5
             // block: 159 -> 153 us)
             if (p.ep.bias || p.ep.act) {
 #pragma unroll 1
-                for (int t = 0; t < 4; ++t) {
+                for (int t = 0; t < nt; ++t) {
                     f32x4* v = reinterpret_cast<f32x4*>(cst + (srow + 8 * t) * CS + scol);
                     *v = activate4(p.ep, *v, bias[j]);
                 }
@@ -350,11 +327,12 @@ __device__ __forceinline__ void store_tiles(const GemmArgs& p, f32x16 (&acc)[TM]
                 if (row < p.M) store_c4(p, c_off + (int64_t)row * p.ldc, col, v, false);
             }
         } else {
-            for (int t = 0; t < 4; ++t) {
+            for (int t = 0; t < nt; ++t) {
                 const int row = row0 + srow + 8 * t;
                 const f32x4 v = *reinterpret_cast<const f32x4*>(cst + (srow + 8 * t) * CS + scol);
                 if (row >= p.M) continue;
-                store_c4(p, c_off + (int64_t)row * p.ldc, col, v, p.ep_on);
+                if (!EP && ws) store_partial4(ws, (int64_t)row * p.N + col, v, p.N - col);
+                else store_c4(p, c_off + (int64_t)row * p.ldc, col, v, EP);
             }
         }
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // reads done before the next tile's writes
@@ -364,7 +342,7 @@ __device__ __forceinline__ void store_tiles(const GemmArgs& p, f32x16 (&acc)[TM]
 // PER_CU blocks are resident on a CU: the registers of their waves must fit too.
 // (128 x 128 with 32-wide stages and the operands of two tiles held at once took
 // 132 registers, one block instead of two: 3264 x 20864 x 128 104 us, now 82.)
-template <bool BF16, int BM, int BN, int BK, int STAGES, int WGM, int WGN, int PER_CU>
+template <bool BF16, bool EP, int BM, int BN, int BK, int STAGES, int WGM, int WGN, int PER_CU>
 __global__ __launch_bounds__(64 * WGM * WGN, PER_CU* WGM* WGN > 8 ? PER_CU * WGM * WGN / 4 : 2) void gemm_mfma_kernel(const GemmArgs p) {
     using G = StageGeom<BK>;
     constexpr int ROWH = G::ROWH;
@@ -511,7 +489,7 @@ __global__ __launch_bounds__(64 * WGM * WGN, PER_CU* WGM* WGN > 8 ? PER_CU * WGM
     const int64_t c_off = (int64_t)batch * p.sC;
     float* ws = p.splits > 1 ? p.ws + (int64_t)blockIdx.z * p.M * p.N : nullptr;
     constexpr int GT = PER_CU * NW > 8 ? 1 : TM * TN;   // four waves to a SIMD: 128 registers each
-    store_tiles<TM, TN, GT>(p, acc, reinterpret_cast<float*>(smem) + wave * 32 * CSTAGE, c_off, ws, lane,
+    store_tiles<EP, TM, TN, GT>(p, acc, reinterpret_cast<float*>(smem) + wave * 32 * CSTAGE, c_off, ws, lane,
                         [&](int i) { return m0 + wm * WM + i * 32; }, [&](int j) { return n0 + wn * WN + j * 32; });
 }
 
@@ -540,7 +518,7 @@ __global__ __launch_bounds__(64 * WGM * WGN, PER_CU* WGM* WGN > 8 ? PER_CU * WGM
 // interval, and nearly the whole ring is in flight.  Loads past the split's K are
 // issued out of the descriptor's range: they write zeros to LDS and move
 // nothing, which serves the K tail and keeps the counts the same to the end.
-template <bool BF16, int NA, int NB, int UA, int S>
+template <bool BF16, bool EP, int NA, int NB, int UA, int S>
 __global__ __launch_bounds__(512, 2) void gemm_pingpong_kernel(const GemmArgs p) {
     constexpr int BM = NA * UA, BN = NB * 128, BK = 64;
     constexpr int ABYTES = UA * BK * 2, BBYTES = 128 * BK * 2, STAGE = NA * ABYTES + NB * BBYTES;
@@ -745,7 +723,7 @@ __global__ __launch_bounds__(512, 2) void gemm_pingpong_kernel(const GemmArgs p)
 
     const int64_t c_off = (int64_t)batch * p.sC;
     float* ws = p.splits > 1 ? p.ws + (int64_t)blockIdx.z * p.M * p.N : nullptr;
-    store_tiles<NA * TA, NB, NA * TA * NB <= 4 ? NA * TA * NB : 2>(p, acc, reinterpret_cast<float*>(smem) + wave * 32 * CSTAGE, c_off, ws, lane,
+    store_tiles<EP, NA * TA, NB, NA * TA * NB <= 4 ? NA * TA * NB : 2>(p, acc, reinterpret_cast<float*>(smem) + wave * 32 * CSTAGE, c_off, ws, lane,
                              [&](int i) { return m0 + UA * (i / TA) + wm * (UA / 2) + 32 * (i % TA); },
                              [&](int j) { return n0 + 128 * j + wn * 32; });
 }
@@ -808,15 +786,19 @@ struct TileCfg {
     int per_cu;       // resident blocks per CU (LDS ring and registers)
     int eff;          // TFLOP/s of a launch that fills every slot (selection weight)
     bool buf;         // buffer-addressed direct loads: operands below 4 GiB only
-    GemmKernel f16, bf16;
+    GemmKernel kernel[2][2];   // [bf16][epilogue at the store]
 };
 
-#define MVLM_TILE(BMv, BNv, BKv, Sv, WMv, WNv, PER_CU, EFF)                                     \
-    TileCfg{BMv, BNv, BKv, Sv, WMv * WNv, PER_CU, EFF, false, gemm_mfma_kernel<false, BMv, BNv, BKv, Sv, WMv, WNv, PER_CU>, \
-            gemm_mfma_kernel<true, BMv, BNv, BKv, Sv, WMv, WNv, PER_CU>}
-#define MVLM_PINGPONG(NAv, NBv, UAv, Sv, EFF)                                                   \
-    TileCfg{NAv * UAv, NBv * 128, 64, Sv, 8, 1, EFF, true, gemm_pingpong_kernel<false, NAv, NBv, UAv, Sv>, \
-            gemm_pingpong_kernel<true, NAv, NBv, UAv, Sv>}
+#define MVLM_TILE(BMv, BNv, BKv, Sv, WMv, WNv, PER_CU, EFF)                                                     \
+    TileCfg{BMv, BNv, BKv, Sv, WMv * WNv, PER_CU, EFF, false,                                                   \
+            {{gemm_mfma_kernel<false, false, BMv, BNv, BKv, Sv, WMv, WNv, PER_CU>,                              \
+              gemm_mfma_kernel<false, true, BMv, BNv, BKv, Sv, WMv, WNv, PER_CU>},                              \
+             {gemm_mfma_kernel<true, false, BMv, BNv, BKv, Sv, WMv, WNv, PER_CU>,                               \
+              gemm_mfma_kernel<true, true, BMv, BNv, BKv, Sv, WMv, WNv, PER_CU>}}}
+#define MVLM_PINGPONG(NAv, NBv, UAv, Sv, EFF)                                                                   \
+    TileCfg{NAv * UAv, NBv * 128, 64, Sv, 8, 1, EFF, true,                                                      \
+            {{gemm_pingpong_kernel<false, false, NAv, NBv, UAv, Sv>, gemm_pingpong_kernel<false, true, NAv, NBv, UAv, Sv>}, \
+             {gemm_pingpong_kernel<true, false, NAv, NBv, UAv, Sv>, gemm_pingpong_kernel<true, true, NAv, NBv, UAv, Sv>}}}
 // All but the last are the automatic choices.  eff: fp16 rate of a launch that
 // fills every slot at K = 2048 .. 4096.  Plain fp16 products, the tile's time
 // against the best tile with all waves in step: 4096^3 113 us (256 x 256; 134),
@@ -1005,7 +987,7 @@ hipError_t launch_gemm_mfma(hipStream_t s, const void* A, int ab_dtype, const vo
         a.B = bp; a.ldb = w.kp; a.sB = (int64_t)N * w.kp; a.kread_b = w.kp;
     }
     dim3 grid((unsigned)(a.tiles_m * a.tiles_n), 1, (unsigned)(batch * g.splits));
-    GemmKernel k = ab_dtype == MVLM_BF16 ? t.bf16 : t.f16;
+    const GemmKernel k = t.kernel[ab_dtype == MVLM_BF16][a.ep_on && g.splits == 1];
     launch_seq(idx++, n, k, grid, dim3(64 * t.waves), s, a);
     if (g.splits > 1) {
         const int64_t mn = (int64_t)M * N;

@@ -103,6 +103,24 @@ def test_gemm_packed_epilogue(dev, orc, bias, act, mul, residual, cd):
     check(orc, got, Y64, S, vals, act, cd, 1e-4)
 
 
+# rows that end in each of a 32-row tile's four passes of 8, columns on and off
+# the vector grid, K of the short-K tile and of the others
+@pytest.mark.parametrize("M", [1, 7, 8, 9, 17, 24, 31, 33, 57])
+@pytest.mark.parametrize("N,K,cd", [(72, 64, F16), (72, 264, F32), (75, 64, F32), (75, 264, F16)])
+def test_gemm_epilogue_row_passes(dev, orc, M, N, K, cd):
+    A, Wt = orc.normal_f16(M * K, 0x74), orc.normal_f16(N * K, 0x75, 0.05)
+    W = dev.pack(Wt, F16, N, K)
+    ops, vals = make_operands(dev, orc, M, N, cd, 0x76, True, True, True)
+    dA, dC = dev.upload(A), dev.upload(np.full(M * N + 64, 9, np.float32))
+    dev.gemm_packed_ex(dA, F16, W, dC, cd, M, N, K, bias=ops["bias"], act=GELU, mul=ops["mul"], residual=ops["residual"])
+    raw = dC.download(np.float32 if cd == F32 else np.uint16)
+    got = from_storage(orc, raw[:M * N], cd).reshape(M, N)
+    Y64, S = orc.gemm_f64(from_storage(orc, A, F16).reshape(M, K), from_storage(orc, Wt, F16).reshape(N, K), M, N, K)
+    check(orc, got, Y64, S, vals, GELU, cd, 1e-4)
+    past = raw[M * N:].view(np.uint8)
+    assert np.array_equal(past, np.full(M * N + 64, 9, np.float32).view(np.uint8)[-past.size:])
+
+
 def test_patch_embedding_gemm_with_bias(dev, orc):
     """SigLIP's patch embedding as one GEMM: 729 patches x 588 values (3 x 14 x 14,
     K not a multiple of 8) against a 1152 x 588 weight, bias in the store, fp16
