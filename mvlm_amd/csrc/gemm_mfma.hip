@@ -109,6 +109,9 @@ __device__ __forceinline__ f32x4 widen_operand4(u32x4 r, int dtype) {
     for (int e = 0; e < 4; ++e) v[e] = dtype == 1 ? f16_bits_to_f32(h[e]) : bf16_bits_to_f32(h[e]);
     return v;
 }
+__device__ __forceinline__ float widen_operand(uint32_t r, int dtype) {
+    return dtype == 0 ? __uint_as_float(r) : dtype == 1 ? f16_bits_to_f32((uint16_t)r) : bf16_bits_to_f32((uint16_t)r);
+}
 // apply_epilogue's two halves on four consecutive columns, the operands loaded
 // before: act(v + bias), then * mul + res
 __device__ __forceinline__ f32x4 activate4(const Epilogue& e, f32x4 v, u32x4 bias) {
@@ -128,20 +131,12 @@ __device__ __forceinline__ f32x4 combine4(const Epilogue& e, f32x4 v, u32x4 mul,
     return v;
 }
 
-// C row `row_off` (element offset of the row), columns col..col+3: epilogue
-// (`ep`; false where it has been applied), output dtype, one 16- or 8-byte
-// store when the row is aligned for it, written through L2 (C is tens of MB at
-// the prefill shapes)
-__device__ __forceinline__ void store_c4(const GemmArgs& p, int64_t row_off, int col, f32x4 v, bool ep) {
+// C row `row_off` (element offset of the row), columns col..col+3: output dtype,
+// one 16- or 8-byte store when the row is aligned for it, written through L2 (C
+// is tens of MB at the prefill shapes)
+__device__ __forceinline__ void store_c4(const GemmArgs& p, int64_t row_off, int col, f32x4 v) {
     const int n_left = p.N - col;
     if (n_left <= 0) return;
-    if (ep) {
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const int64_t idx = row_off + col + e;
-            if (e < n_left) v[e] = apply_epilogue(p.ep, v[e], idx, col + e);
-        }
-    }
     const int64_t i = row_off + col;
     if (p.vec_c && n_left >= 4) {
         if (p.c_dtype == 0) {
@@ -221,36 +216,26 @@ constexpr int CSTAGE = 36;
 template <bool EP, int TM, int TN, int GT, typename RowOf, typename ColOf>
 __device__ __forceinline__ void store_tiles(const GemmArgs& p, f32x16 (&acc)[TM][TN], float* cst, int64_t c_off,
                                             float* ws, int lane, RowOf row_of, ColOf col_of) {
-    if (!(!EP && ws ? p.vec_ws : p.vec_c)) {   // rows off the vector grid: straight from the accumulators, 32 columns per row
+    if constexpr (!EP) {
+        if (!(ws ? p.vec_ws : p.vec_c)) {   // rows off the vector grid: straight from the accumulators, 32 columns per row
 #pragma unroll
-        for (int i = 0; i < TM; ++i)
+            for (int i = 0; i < TM; ++i)
 #pragma unroll
-            for (int j = 0; j < TN; ++j) {
-                const int col = col_of(j) + (lane & 31);
-                if (col >= p.N) continue;
-                auto each_row = [&](auto&& put) {
+                for (int j = 0; j < TN; ++j) {
+                    const int col = col_of(j) + (lane & 31);
+                    if (col >= p.N) continue;
+                    auto each_row = [&](auto&& put) {
 #pragma unroll
-                    for (int r = 0; r < 16; ++r) {
-                        const int row = row_of(i) + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
-                        if (row < p.M) put(row, acc[i][j][r]);
-                    }
-                };
-                if constexpr (EP) {   // the per-element code is larger: a quarter of the rows unrolled
-#pragma unroll 4
-                    for (int r = 0; r < 16; ++r) {
-                        const int row = row_of(i) + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
-                        if (row < p.M) {
-                            const int64_t idx = c_off + (int64_t)row * p.ldc + col;
-                            store_out(p.C, idx, apply_epilogue(p.ep, acc[i][j][r], idx, col), p.c_dtype);
+                        for (int r = 0; r < 16; ++r) {
+                            const int row = row_of(i) + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
+                            if (row < p.M) put(row, acc[i][j][r]);
                         }
-                    }
-                } else if (ws) {
-                    each_row([&](int row, float v) { ws[(int64_t)row * p.N + col] = v; });
-                } else {
-                    each_row([&](int row, float v) { store_out(p.C, c_off + (int64_t)row * p.ldc + col, v, p.c_dtype); });
+                    };
+                    if (ws) each_row([&](int row, float v) { ws[(int64_t)row * p.N + col] = v; });
+                    else each_row([&](int row, float v) { store_out(p.C, c_off + (int64_t)row * p.ldc + col, v, p.c_dtype); });
                 }
-            }
-        return;
+            return;
+        }
     }
     // Aligned rows: through LDS.  Each wave writes one 32x32 accumulator tile
     // at a time into its own region of the (now idle) ring, row-major with a
@@ -268,6 +253,58 @@ __device__ __forceinline__ void store_tiles(const GemmArgs& p, f32x16 (&acc)[TM]
         for (int r = 0; r < 16; ++r) cst[(8 * (r >> 2) + 4 * (lane >> 5) + (r & 3)) * CS + (lane & 31)] = c[r];
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // this wave's writes, before its reads
     };
+    if constexpr (EP) {
+        if (!p.vec_ep) {
+            // Rows or operands off the vector grid: element by element, 32
+            // columns of two rows at a time, in a loop of four such passes whose
+            // operands are requested one round ahead (729 x 3457 x 1152 with bias
+            // and residual 33.6 us when each waited for its own).
+            const int ecol = lane & 31, erow = lane >> 5;
+            __syncthreads();   // every wave is done with the ring (all its loads have landed)
+            static_for<T>([&](auto IJ) {
+                constexpr int i = decltype(IJ)::value / TN, j = decltype(IJ)::value % TN;
+                const int row0 = row_of(i) + erow, col = col_of(j) + ecol, ccol = min(col, p.N - 1);
+                const int rounds = passes(row_of(i));
+                if (rounds <= 0 || col_of(j) >= p.N) return;
+                uint32_t mul[4], res[4];
+                auto request = [&](const void* base, int t0, uint32_t (&to)[4]) {
+#pragma unroll
+                    for (int t = 0; t < 4; ++t) {
+                        const int64_t idx = c_off + (int64_t)min(row0 + 2 * (t0 + t), p.M - 1) * p.ldc + ccol;
+                        to[t] = p.ep.dtype == 0 ? ((const uint32_t*)base)[idx] : ((const uint16_t*)base)[idx];
+                    }
+                };
+                if (p.ep.mul) request(p.ep.mul, 0, mul);
+                if (p.ep.res) request(p.ep.res, 0, res);
+                const float bias = p.ep.bias ? load_as_f32(p.ep.bias, ccol, p.ep.dtype) : 0.0f;
+                stage_tile(acc[i][j]);
+#pragma unroll 1
+                for (int q = 0; q < rounds; ++q) {
+                    uint32_t m[4], r[4];
+#pragma unroll
+                    for (int t = 0; t < 4; ++t) {
+                        m[t] = mul[t];
+                        r[t] = res[t];
+                    }
+                    if (p.ep.mul && q + 1 < rounds) request(p.ep.mul, 4 * q + 4, mul);
+                    if (p.ep.res && q + 1 < rounds) request(p.ep.res, 4 * q + 4, res);
+#pragma unroll
+                    for (int t = 0; t < 4; ++t) {
+                        const int row = 8 * q + 2 * t;
+                        float x = cst[(row + erow) * CS + ecol] + bias;
+                        if (p.ep.act == 1) x = gelu_tanh(x);
+                        else if (p.ep.act == 2) x = silu(x);
+                        if (p.ep.mul) x *= widen_operand(m[t], p.ep.dtype);
+                        if (p.ep.res) x += widen_operand(r[t], p.ep.dtype);
+                        if (row0 + row < p.M && col < p.N)
+                            store_out(p.C, c_off + (int64_t)(row0 + row) * p.ldc + col, x, p.c_dtype);
+                    }
+                }
+                asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // reads done before the next tile's writes
+            });
+            return;
+        }
+    }
     // The epilogue's operands are requested four columns at a time for GT tiles
     // at once (all of a wave's, but for the 128 accumulators of 256 x 256 and
     // tiles of which two share a CU), before the tiles pass through LDS: one wait
@@ -276,7 +313,6 @@ __device__ __forceinline__ void store_tiles(const GemmArgs& p, f32x16 (&acc)[TM]
     // without; a Phi-1.5 block of 768 rows went 170 -> 153 us, a SigLIP block of
     // 729 101 -> 91.  In-place operands are safe: an element's are read by the
     // thread that later stores it.
-    const bool epv = EP && p.vec_ep;
     u32x4 bias[TN], mul[GT][4], res[GT][4];
     auto load_group = [&](auto G) {
         auto each = [&](const void* base, u32x4 (&to)[GT][4]) {
@@ -292,7 +328,7 @@ __device__ __forceinline__ void store_tiles(const GemmArgs& p, f32x16 (&acc)[TM]
         if (p.ep.mul) each(p.ep.mul, mul);
         if (p.ep.res) each(p.ep.res, res);
     };
-    if (epv) {
+    if constexpr (EP) {
         if (p.ep.bias)
 #pragma unroll
             for (int j = 0; j < TN; ++j)
@@ -304,11 +340,11 @@ __device__ __forceinline__ void store_tiles(const GemmArgs& p, f32x16 (&acc)[TM]
     // and move it to scratch memory)
     static_for<T>([&](auto IJ) {
         constexpr int ij = decltype(IJ)::value, i = ij / TN, j = ij % TN;
-        if constexpr (ij > 0 && ij % GT == 0)
-            if (epv) load_group(std::integral_constant<int, ij / GT>{});
-        stage_tile(acc[i][j]);
+        if constexpr (EP && ij > 0 && ij % GT == 0) load_group(std::integral_constant<int, ij / GT>{});
         const int row0 = row_of(i), col = col_of(j) + scol, nt = passes(row0);
-        if (epv) {
+        if (nt <= 0 || col_of(j) >= p.N) return;
+        stage_tile(acc[i][j]);
+        if constexpr (EP) {
             // in a loop and back to LDS: unrolled over every element of the
             // wave this code alone would be tens of KB, run once (the Phi-1.5
             // block: 159 -> 153 us)
@@ -324,15 +360,15 @@ __device__ __forceinline__ void store_tiles(const GemmArgs& p, f32x16 (&acc)[TM]
                 const int row = row0 + srow + 8 * t;
                 const f32x4 v = combine4(p.ep, *reinterpret_cast<const f32x4*>(cst + (srow + 8 * t) * CS + scol),
                                          mul[ij % GT][t], res[ij % GT][t]);
-                if (row < p.M) store_c4(p, c_off + (int64_t)row * p.ldc, col, v, false);
+                if (row < p.M) store_c4(p, c_off + (int64_t)row * p.ldc, col, v);
             }
         } else {
             for (int t = 0; t < nt; ++t) {
                 const int row = row0 + srow + 8 * t;
                 const f32x4 v = *reinterpret_cast<const f32x4*>(cst + (srow + 8 * t) * CS + scol);
                 if (row >= p.M) continue;
-                if (!EP && ws) store_partial4(ws, (int64_t)row * p.N + col, v, p.N - col);
-                else store_c4(p, c_off + (int64_t)row * p.ldc, col, v, EP);
+                if (ws) store_partial4(ws, (int64_t)row * p.N + col, v, p.N - col);
+                else store_c4(p, c_off + (int64_t)row * p.ldc, col, v);
             }
         }
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // reads done before the next tile's writes
@@ -755,7 +791,10 @@ __global__ __launch_bounds__(256) void gemm_splitk_reduce_kernel(const GemmArgs 
             }
             for (int s = 1; s < p.splits; ++s) acc += *reinterpret_cast<const f32x4*>(ws + s * mn);
             if (EP && p.vec_ep) acc = combine4(p.ep, activate4(p.ep, acc, bias), mul, res);
-            store_c4(p, idx - col, col, acc, EP && !p.vec_ep);
+            if (EP && !p.vec_ep)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) acc[e] = apply_epilogue(p.ep, acc[e], idx + e, col + e);
+            store_c4(p, idx - col, col, acc);
             return;
         }
     }
