@@ -823,41 +823,50 @@ typedef void (*GemmKernel)(const GemmArgs);
 struct TileCfg {
     int bm, bn, bk, stages, waves;
     int per_cu;       // resident blocks per CU (LDS ring and registers)
-    int eff;          // TFLOP/s of a launch that fills every slot (selection weight)
+    int eff;          // TFLOP/s of a round that fills every slot, and what the
+    float fixed;      // round takes besides its products (us)
     bool buf;         // buffer-addressed direct loads: operands below 4 GiB only
     GemmKernel kernel[2][2];   // [bf16][epilogue at the store]
 };
 
-#define MVLM_TILE(BMv, BNv, BKv, Sv, WMv, WNv, PER_CU, EFF)                                                     \
-    TileCfg{BMv, BNv, BKv, Sv, WMv * WNv, PER_CU, EFF, false,                                                   \
+#define MVLM_TILE(BMv, BNv, BKv, Sv, WMv, WNv, PER_CU, EFF, FIXED)                                              \
+    TileCfg{BMv, BNv, BKv, Sv, WMv * WNv, PER_CU, EFF, FIXED, false,                                            \
             {{gemm_mfma_kernel<false, false, BMv, BNv, BKv, Sv, WMv, WNv, PER_CU>,                              \
               gemm_mfma_kernel<false, true, BMv, BNv, BKv, Sv, WMv, WNv, PER_CU>},                              \
              {gemm_mfma_kernel<true, false, BMv, BNv, BKv, Sv, WMv, WNv, PER_CU>,                               \
               gemm_mfma_kernel<true, true, BMv, BNv, BKv, Sv, WMv, WNv, PER_CU>}}}
-#define MVLM_PINGPONG(NAv, NBv, UAv, Sv, EFF)                                                                   \
-    TileCfg{NAv * UAv, NBv * 128, 64, Sv, 8, 1, EFF, true,                                                      \
+#define MVLM_PINGPONG(NAv, NBv, UAv, Sv, EFF, FIXED)                                                            \
+    TileCfg{NAv * UAv, NBv * 128, 64, Sv, 8, 1, EFF, FIXED, true,                                               \
             {{gemm_pingpong_kernel<false, false, NAv, NBv, UAv, Sv>, gemm_pingpong_kernel<false, true, NAv, NBv, UAv, Sv>}, \
              {gemm_pingpong_kernel<true, false, NAv, NBv, UAv, Sv>, gemm_pingpong_kernel<true, true, NAv, NBv, UAv, Sv>}}}
-// All but the last are the automatic choices.  eff: fp16 rate of a launch that
-// fills every slot at K = 2048 .. 4096.  Plain fp16 products, the tile's time
-// against the best tile with all waves in step: 4096^3 113 us (256 x 256; 134),
+// All but the last are the automatic choices.  What each costs in plan_gemm's
+// model was fitted to the times of every tile and K split over 2100 fp16 products
+// (M 1 .. 16384, N 16 .. 51200, K 136 .. 14336; the choice is 1.6% from the
+// fastest on average, and 12 products are more than 3% from the better of the
+// choice before and the one of the tiles before these).  eff is the rate of a round's products with every slot
+// busy, fixed what a round takes besides (first loads, last stores).  Without
+// the latter, a 128 x 128 tile whose K is cut into splits of a few stages looked
+// faster than it is: 121 x 2945 x 2112 15.6 us with six splits, 13.2 with two of
+// 64 x 64 tiles; 66 x 5836 x 1024 11.3 against 8.3 us.  Plain fp16 products, the
+// tile's time against the best tile with all waves in step: 4096^3 105 us (256 x 256; 134),
 // 1536 x 6144 x 2048 44 (256 x 256; 67), 2048 x 4096 x 600 16.6 (256 x 128; 18.0),
-// 768 x 6144 x 2048 28.3 (192 x 128; 31.9), 768 x 8192 x 2048 30.1 (192 x 128;
-// 33.7), 729 x 3456 x 1152 13.0 (128 x 128; 14.1), 729 x 4304 x 1152 13.5 (128 x
-// 128; 15.3), 2048^3 22.8 (128 x 128; 25.7).  A fifth slot for 128 x 128 (160
+// 768 x 6144 x 2048 26.7 (192 x 128; 31.9), 768 x 8192 x 2048 30.2 (192 x 128;
+// 33.7), 729 x 3456 x 1152 13.9 (128 x 128; 14.1), 729 x 4304 x 1152 14.2 (128 x
+// 128; 15.3), 2048^3 23.5 (128 x 128; 25.7).  A fifth slot for 128 x 128 (160
 // KiB) is slower, 13.9 us at 729 x 3456 x 1152.  Products of few tiles stay with
 // 64 x 64, two blocks to a CU: 729 x 1152 x 1152 takes 8.8 us with two 128-wide
 // stages, 12.8 with 128 x 128; 64-wide stages serve the many-way K splits of
 // few-row products.  128 x 128 in step (two 128-wide stages) serves operands
-// beyond the buffer descriptors' 4 GiB.
+// beyond the buffer descriptors' 4 GiB, 96 x 192 up to 96 rows by many columns
+// (64 x 46656 x 3840 79 us, 86 with 64 x 64).
 static const TileCfg kTiles[] = {
-    MVLM_PINGPONG(2, 2, 128, 2, 1216), MVLM_PINGPONG(4, 1, 64, 3, 1000),
-    MVLM_PINGPONG(3, 1, 64, 4, 880), MVLM_PINGPONG(2, 1, 64, 4, 760),
-    MVLM_TILE(64, 64, 64, 4, 2, 2, 2, 401), MVLM_TILE(64, 64, 128, 2, 2, 2, 2, 460),
-    MVLM_TILE(128, 128, 128, 2, 4, 2, 1, 682),
-    MVLM_TILE(128, 128, 32, 4, 4, 2, 2, 689),
+    MVLM_PINGPONG(2, 2, 128, 2, 1415, 4.9), MVLM_PINGPONG(4, 1, 64, 3, 990, 2.4),
+    MVLM_PINGPONG(3, 1, 64, 4, 905, 2.5), MVLM_PINGPONG(2, 1, 64, 4, 785, 2.5),
+    MVLM_TILE(64, 64, 64, 4, 2, 2, 2, 380, 1.4), MVLM_TILE(64, 64, 128, 2, 2, 2, 2, 420, 1.1),
+    MVLM_TILE(128, 128, 128, 2, 4, 2, 1, 650, 5.7), MVLM_TILE(96, 192, 128, 2, 3, 2, 1, 535, 3.8),
+    MVLM_TILE(128, 128, 32, 4, 4, 2, 2, 690, 2.0),
 };
-constexpr int kAutoTiles = 7;
+constexpr int kAutoTiles = 8;
 #undef MVLM_TILE
 #undef MVLM_PINGPONG
 
@@ -866,13 +875,15 @@ struct GemmPlan {
     int splits, split_stages;
 };
 
-// The tile and K split with the least modelled time: block rounds x one
-// block's share of the tile's full-chip throughput (eff, all slots busy),
-// plus, for a split, writing and re-reading the fp32 partials (~4 TB/s) and a
-// second launch.  MVLM_GEMM_TILE=<bm>x<bn>s<stages>w<waves>[k<bk>] forces a
-// compiled tile and MVLM_GEMM_SPLITS=<n> a split count (tuning runs; read at
-// every launch).
-static GemmPlan plan_gemm(int M, int N, int K, int batch, int num_cus, bool buf_ok) {
+// The tile and K split with the least modelled time: block rounds x (one
+// block's share of the tile's full-chip throughput and the round's fixed cost),
+// plus, for a split, writing and re-reading the fp32 partials (3.7 TB/s) and a
+// second launch, or else the epilogue, which costs a tile's store pass more than
+// it does that launch (186 x 1300 x 832 with bias and residual 9.7 us in one
+// launch, 8.9 in three splits; 186 x 1299 x 832, element by element, 12.7 and
+// 9.6).  MVLM_GEMM_TILE=<bm>x<bn>s<stages>w<waves>[k<bk>] forces a compiled tile
+// and MVLM_GEMM_SPLITS=<n> a split count (tuning runs; read at every launch).
+static GemmPlan plan_gemm(int M, int N, int K, int batch, int num_cus, bool buf_ok, bool ep) {
     GemmPlan best{&kTiles[4], 1, 0};
     double best_t = 1e30;
     const char* force = std::getenv("MVLM_GEMM_TILE");
@@ -908,8 +919,9 @@ static GemmPlan plan_gemm(int M, int N, int K, int batch, int num_cus, bool buf_
             const int64_t slots = (int64_t)num_cus * c.per_cu;
             const int64_t rounds = (tiles + slots - 1) / slots;
             const double block_flops = 2.0 * c.bm * c.bn * (double)ss * c.bk;
-            double t = rounds * block_flops / (c.eff * 1e12 / (double)slots);
-            if (splits > 1) t += (double)M * N * batch * 4.0 * (2.0 * splits + 1.0) / 4e12 + 3e-6;
+            double t = rounds * (block_flops / (c.eff * 1e12 / (double)slots) + c.fixed * 1e-6);
+            if (splits > 1) t += (double)M * N * batch * 4.0 * (2.0 * splits + 1.0) / 3.7e12 + 3.4e-6;
+            else if (ep) t += N % 4 == 0 ? 1.0e-6 : 2.5e-6;
             if (t < best_t) { best_t = t; best = GemmPlan{&c, splits, ss}; }
         }
     }
@@ -941,7 +953,7 @@ struct GemmWorkspace {
 static size_t align256(size_t v) { return (v + 255) & ~(size_t)255; }
 
 static GemmWorkspace gemm_workspace(int batch, int M, int N, int K, int64_t lda, int64_t ldb, int64_t sA,
-                                   int64_t sB, int kread_b, int num_cus) {
+                                   int64_t sB, int kread_b, int num_cus, bool ep) {
     GemmWorkspace w;
     const int k8 = (int)round_up(K, 8);
     w.pad_a = K % 8 != 0 || lda % 8 != 0 || (batch > 1 && sA % 8 != 0);
@@ -950,7 +962,7 @@ static GemmWorkspace gemm_workspace(int batch, int M, int N, int K, int64_t lda,
     // buffer-addressed tiles need each operand's rows within a 32-bit byte range
     const int64_t lda_k = w.pad_a ? w.kp : lda, ldb_k = w.pad_b ? w.kp : ldb;
     const bool buf_ok = (int64_t)M * lda_k * 2 < ((int64_t)1 << 32) - 256 && (int64_t)N * ldb_k * 2 < ((int64_t)1 << 32) - 256;
-    w.plan = plan_gemm(M, N, w.kp, batch, num_cus > 0 ? num_cus : 256, buf_ok);
+    w.plan = plan_gemm(M, N, w.kp, batch, num_cus > 0 ? num_cus : 256, buf_ok, ep);
     w.split_bytes = w.plan.splits > 1 ? align256((size_t)w.plan.splits * batch * M * N * sizeof(float)) : 0;
     w.a_off = w.split_bytes;
     const size_t a_bytes = w.pad_a ? align256((size_t)batch * M * w.kp * 2) : 0;
@@ -961,8 +973,8 @@ static GemmWorkspace gemm_workspace(int batch, int M, int N, int K, int64_t lda,
 }
 
 size_t gemm_workspace_bytes(int batch, int M, int N, int K, int64_t lda, int64_t ldb, int64_t sA, int64_t sB,
-                            int kread_b, int num_cus) {
-    return gemm_workspace(batch, M, N, K, lda, ldb, sA, sB, kread_b, num_cus).total;
+                            int kread_b, int num_cus, bool ep) {
+    return gemm_workspace(batch, M, N, K, lda, ldb, sA, sB, kread_b, num_cus, ep).total;
 }
 
 // Launches kernel `idx` of an op made of `n` kernels (plan profiling times the
@@ -984,7 +996,7 @@ hipError_t launch_gemm_mfma(hipStream_t s, const void* A, int ab_dtype, const vo
                             int batch, int M, int N, int K, int64_t lda, int64_t ldb, int64_t ldc,
                             int64_t strideA, int64_t strideB, int64_t strideC, int kread_b, int num_cus,
                             const Epilogue* ep, void* workspace, size_t workspace_bytes) {
-    const GemmWorkspace w = gemm_workspace(batch, M, N, K, lda, ldb, strideA, strideB, kread_b, num_cus);
+    const GemmWorkspace w = gemm_workspace(batch, M, N, K, lda, ldb, strideA, strideB, kread_b, num_cus, ep && ep->any());
     if (w.total > 0 && (!workspace || workspace_bytes < w.total)) return hipErrorInvalidValue;
     const GemmPlan& g = w.plan;
     const TileCfg& t = *g.tile;

@@ -137,7 +137,7 @@ int make_gemv_exact(mvlm_device* dev, const mvlm_buffer* x, const mvlm_weight* W
 // The op of a packed-weight GEMM, all but its workspace (op->workspace_bytes
 // says how much it needs).
 int make_gemm_packed_op(mvlm_device* dev, const mvlm_buffer* A, int a_dtype, const mvlm_weight* W, mvlm_buffer* C,
-                        int c_dtype, int M, int N, int K, const char* fn, Op* op) {
+                        int c_dtype, int M, int N, int K, const mvlm_epilogue* ep, const char* fn, Op* op) {
     REQUIRE(dev && A && W && C, "%s: null argument", fn);
     REQUIRE(A->dev == dev && W->dev == dev && C->dev == dev, "%s: handles belong to another device", fn);
     REQUIRE(M > 0 && N > 0 && K > 0, "%s: M=%d N=%d K=%d must be positive", fn, M, N, K);
@@ -155,13 +155,15 @@ int make_gemm_packed_op(mvlm_device* dev, const mvlm_buffer* A, int a_dtype, con
     op->lda = K; op->ldb = W->ld; op->ldc = N;
     op->kread_b = (int)W->ld;     // packed rows are zero padded to ld = roundup(K, 64)
     op->num_cus = dev->prop.multiProcessorCount;
-    op->workspace_bytes = gemm_workspace_bytes(1, M, N, K, op->lda, op->ldb, 0, 0, op->kread_b, op->num_cus);
+    const int st = make_epilogue(dev, ep, M, N, c_dtype, fn, &op->ep);
+    if (st != MVLM_OK) return st;
+    op->workspace_bytes = gemm_workspace_bytes(1, M, N, K, op->lda, op->ldb, 0, 0, op->kread_b, op->num_cus, op->ep.any());
     return MVLM_OK;
 }
 
 int make_gemm_packed(mvlm_device* dev, const mvlm_buffer* A, int a_dtype, const mvlm_weight* W, mvlm_buffer* C,
-                     int c_dtype, int M, int N, int K, const char* fn, Op* op) {
-    const int st = make_gemm_packed_op(dev, A, a_dtype, W, C, c_dtype, M, N, K, fn, op);
+                     int c_dtype, int M, int N, int K, const mvlm_epilogue* ep, const char* fn, Op* op) {
+    const int st = make_gemm_packed_op(dev, A, a_dtype, W, C, c_dtype, M, N, K, ep, fn, op);
     return st != MVLM_OK ? st : device_scratch(dev, op->workspace_bytes, &op->workspace);
 }
 
@@ -185,7 +187,7 @@ int make_gemm_batched(mvlm_device* dev, const mvlm_buffer* A, const mvlm_buffer*
     op->lda = lda; op->ldb = ldb; op->ldc = ldc; op->sA = sA; op->sB = sB; op->sC = sC;
     op->kread_b = K;
     op->num_cus = dev->prop.multiProcessorCount;
-    op->workspace_bytes = gemm_workspace_bytes(batch, M, N, K, lda, ldb, sA, sB, K, op->num_cus);
+    op->workspace_bytes = gemm_workspace_bytes(batch, M, N, K, lda, ldb, sA, sB, K, op->num_cus, false);
     return device_scratch(dev, op->workspace_bytes, &op->workspace);
 }
 
@@ -514,15 +516,14 @@ extern "C" int mvlm_gemv_exact(mvlm_device* dev, const mvlm_buffer* x, const mvl
 extern "C" int mvlm_gemm_packed(mvlm_device* dev, const mvlm_buffer* A, int a_dtype, const mvlm_weight* W,
                                 mvlm_buffer* C, int c_dtype, int M, int N, int K, mvlm_event** ev) {
     const char* fn = __func__;
-    RUN(make_gemm_packed(dev, A, a_dtype, W, C, c_dtype, M, N, K, fn, &op));
+    RUN(make_gemm_packed(dev, A, a_dtype, W, C, c_dtype, M, N, K, nullptr, fn, &op));
 }
 
 extern "C" int mvlm_gemm_packed_ex(mvlm_device* dev, const mvlm_buffer* A, int a_dtype, const mvlm_weight* W,
                                    mvlm_buffer* C, int c_dtype, int M, int N, int K, const mvlm_epilogue* ep,
                                    mvlm_event** ev) {
     const char* fn = __func__;
-    RUN(then(make_gemm_packed(dev, A, a_dtype, W, C, c_dtype, M, N, K, fn, &op),
-             [&] { return make_epilogue(dev, ep, M, N, c_dtype, fn, &op.ep); }));
+    RUN(make_gemm_packed(dev, A, a_dtype, W, C, c_dtype, M, N, K, ep, fn, &op));
 }
 
 extern "C" int mvlm_gemm_packed_ex_noalloc(mvlm_device* dev, const mvlm_buffer* A, int a_dtype, const mvlm_weight* W,
@@ -530,8 +531,7 @@ extern "C" int mvlm_gemm_packed_ex_noalloc(mvlm_device* dev, const mvlm_buffer* 
                                            const mvlm_epilogue* ep) {
     const char* fn = __func__;
     Op op{};
-    int st = make_gemm_packed_op(dev, A, a_dtype, W, C, c_dtype, M, N, K, fn, &op);
-    if (st == MVLM_OK) st = make_epilogue(dev, ep, M, N, c_dtype, fn, &op.ep);
+    const int st = make_gemm_packed_op(dev, A, a_dtype, W, C, c_dtype, M, N, K, ep, fn, &op);
     if (st != MVLM_OK) return st;
     if (op.workspace_bytes > (size_t)MVLM_NOALLOC_SCRATCH_BYTES)
         return set_error(MVLM_ERR_UNSUPPORTED, "%s: %dx%dx%d needs %zu bytes of workspace, above the %zu bytes this "
@@ -847,8 +847,7 @@ extern "C" int mvlm_plan_add_gemm_packed_ex(mvlm_plan* plan, const mvlm_buffer* 
     const char* fn = __func__;
     REQUIRE(plan && W, "%s: null argument", fn);
     Op op{};
-    int st = make_gemm_packed(plan->dev, A, a_dtype, W, C, c_dtype, M, W->N, W->K, fn, &op);
-    if (st == MVLM_OK) st = make_epilogue(plan->dev, ep, M, W->N, c_dtype, fn, &op.ep);
+    const int st = make_gemm_packed(plan->dev, A, a_dtype, W, C, c_dtype, M, W->N, W->K, ep, fn, &op);
     return st != MVLM_OK ? st : plan_push(plan, op);
 }
 
@@ -893,7 +892,7 @@ extern "C" int mvlm_plan_add_gemm_packed(mvlm_plan* plan, const mvlm_buffer* A, 
     const char* fn = __func__;
     REQUIRE(plan && W, "%s: null argument", fn);
     Op op{};
-    int st = make_gemm_packed(plan->dev, A, a_dtype, W, C, c_dtype, M, W->N, W->K, fn, &op);
+    const int st = make_gemm_packed(plan->dev, A, a_dtype, W, C, c_dtype, M, W->N, W->K, nullptr, fn, &op);
     return st != MVLM_OK ? st : plan_push(plan, op);
 }
 
