@@ -206,8 +206,9 @@ int mvlm_gemv_ex(mvlm_device* dev, const mvlm_buffer* x, int x_dtype, const mvlm
  * capture, tight serving loops, harnesses that forbid hipMalloc).  The
  * workspace (K-split partials, zero-padded copies of A when K % 8 != 0) comes
  * from one fixed device array of MVLM_NOALLOC_SCRATCH_BYTES per GPU, reserved
- * by the library for the life of the process; a shape that needs more is
- * refused with MVLM_ERR_UNSUPPORTED.  Results are identical to
+ * by the library for the life of the process; where the partials of all of C
+ * need more, C is covered in bands, and a shape whose copy of A leaves no room
+ * for one row's is refused with MVLM_ERR_UNSUPPORTED.  Results are identical to
  * mvlm_gemm_packed_ex's.  All calls on one GPU share the array: calls through
  * one device handle run in order on its stream, calls that overlap on one GPU
  * (several handles or streams) race.  No event is returned. */

@@ -270,6 +270,8 @@ inline int64_t weight_row_bytes(const mvlm_weight* w) { return is_dense(w->dtype
 // kread_b < K rounded up to 8.
 size_t gemm_workspace_bytes(int batch, int M, int N, int K, int64_t lda, int64_t ldb, int64_t sA, int64_t sB,
                             int kread_b, int num_cus, bool ep);
+// The least of it that launch_gemm_mfma (batch 1) runs in, band by band of C.
+size_t gemm_workspace_least(int M, int N, int K, int64_t lda, int64_t ldb, int kread_b, int num_cus, bool ep);
 // Batched NT products with K <= 128 (a multiple of 8) and a dense fp32 C per
 // batch (ldc == N <= 1024), A/B/C 16-byte aligned: C's rows in blocks of 16,
 // each written as one contiguous range (gemm_smallk.hip).

@@ -37,6 +37,7 @@
 #include "common.h"
 #include "device_math.h"
 
+#include <algorithm>
 #include <cstdio>
 #include <cstdlib>
 
@@ -878,10 +879,10 @@ struct GemmPlan {
 // The tile and K split with the least modelled time: block rounds x (one
 // block's share of the tile's full-chip throughput and the round's fixed cost),
 // plus, for a split, writing and re-reading the fp32 partials (3.7 TB/s) and a
-// second launch, or else the epilogue, which costs a tile's store pass more than
-// it does that launch (186 x 1300 x 832 with bias and residual 9.7 us in one
-// launch, 8.9 in three splits; 186 x 1299 x 832, element by element, 12.7 and
-// 9.6).  MVLM_GEMM_TILE=<bm>x<bn>s<stages>w<waves>[k<bk>] forces a compiled tile
+// second launch, or else the epilogue, which costs a tile of 32 rows more in the
+// store pass than it does that launch (186 x 1300 x 832 with bias and residual
+// 9.7 us in one launch, 8.9 in three splits; 186 x 1299 x 832 10.5 and 9.6; with
+// 1 us for it 1408 x 448 x 1240 took two splits, 14.4 against 13.1).  MVLM_GEMM_TILE=<bm>x<bn>s<stages>w<waves>[k<bk>] forces a compiled tile
 // and MVLM_GEMM_SPLITS=<n> a split count (tuning runs; read at every launch).
 static GemmPlan plan_gemm(int M, int N, int K, int batch, int num_cus, bool buf_ok, bool ep) {
     GemmPlan best{&kTiles[4], 1, 0};
@@ -921,7 +922,7 @@ static GemmPlan plan_gemm(int M, int N, int K, int batch, int num_cus, bool buf_
             const double block_flops = 2.0 * c.bm * c.bn * (double)ss * c.bk;
             double t = rounds * (block_flops / (c.eff * 1e12 / (double)slots) + c.fixed * 1e-6);
             if (splits > 1) t += (double)M * N * batch * 4.0 * (2.0 * splits + 1.0) / 3.7e12 + 3.4e-6;
-            else if (ep) t += N % 4 == 0 ? 1.0e-6 : 2.5e-6;
+            else if (ep) t += 0.3e-6 * std::min(M, 32) / 32;
             if (t < best_t) { best_t = t; best = GemmPlan{&c, splits, ss}; }
         }
     }
@@ -977,6 +978,43 @@ size_t gemm_workspace_bytes(int batch, int M, int N, int K, int64_t lda, int64_t
     return gemm_workspace(batch, M, N, K, lda, ldb, sA, sB, kread_b, num_cus, ep).total;
 }
 
+// The part of C (whole tiles, if one fits) whose split partials fit `room` bytes;
+// rows == 0 if not even one row of a tile does.  A launch with less workspace than all partials take
+// covers C band by band, with the same tile and splits and so the same sums.
+struct GemmBand {
+    int rows, cols;
+};
+static GemmBand gemm_band(const GemmPlan& g, int M, int N, size_t room) {
+    const int64_t fit = (int64_t)(room / ((size_t)g.splits * sizeof(float)));   // outputs per band
+    if (g.splits == 1 || (int64_t)M * N <= fit) return {M, N};
+    const int bm = g.tile->bm, bn = g.tile->bn;
+    auto even = [](int64_t all, int64_t most, int64_t tile) {   // as few bands, of nearly one size
+        const int64_t bands = (all + most - 1) / most;
+        return (int)std::min(all, ((all + bands - 1) / bands + tile - 1) / tile * tile);
+    };
+    int64_t rows = fit / N / bm * bm, cols = N;
+    if (rows == 0) {
+        rows = std::min(M, bm);
+        cols = fit / rows / bn * bn;
+        if (cols == 0) {             // less than a tile: rows of one
+            cols = std::min(N, bn);
+            rows = fit / cols;
+            if (rows == 0) return {0, 0};
+            return {(int)rows, even(N, cols, bn)};
+        }
+    }
+    return {even(M, rows, bm), even(N, cols, bn)};
+}
+
+// The least workspace a launch runs in.  A split count forced from outside is
+// refused where it does not fit whole: a tuning run measures what it asked for.
+size_t gemm_workspace_least(int M, int N, int K, int64_t lda, int64_t ldb, int kread_b, int num_cus, bool ep) {
+    const GemmWorkspace w = gemm_workspace(1, M, N, K, lda, ldb, 0, 0, kread_b, num_cus, ep);
+    if (w.plan.splits == 1 || std::getenv("MVLM_GEMM_SPLITS")) return w.total;
+    const size_t row = (size_t)std::min(N, w.plan.tile->bn) * w.plan.splits * sizeof(float);
+    return w.total - w.split_bytes + std::min(w.split_bytes, align256(row));
+}
+
 // Launches kernel `idx` of an op made of `n` kernels (plan profiling times the
 // first kernel's start to the last one's stop).
 template <typename... KArgs, typename... Args>
@@ -997,9 +1035,19 @@ hipError_t launch_gemm_mfma(hipStream_t s, const void* A, int ab_dtype, const vo
                             int64_t strideA, int64_t strideB, int64_t strideC, int kread_b, int num_cus,
                             const Epilogue* ep, void* workspace, size_t workspace_bytes) {
     const GemmWorkspace w = gemm_workspace(batch, M, N, K, lda, ldb, strideA, strideB, kread_b, num_cus, ep && ep->any());
-    if (w.total > 0 && (!workspace || workspace_bytes < w.total)) return hipErrorInvalidValue;
+    if (w.total > 0 && !workspace) return hipErrorInvalidValue;
     const GemmPlan& g = w.plan;
     const TileCfg& t = *g.tile;
+    GemmBand band{M, N};
+    size_t split_bytes = w.split_bytes;
+    if (workspace_bytes < w.total) {
+        const size_t pads = w.total - w.split_bytes;
+        if (batch > 1 || workspace_bytes < pads) return hipErrorInvalidValue;
+        split_bytes = (workspace_bytes - pads) & ~(size_t)255;
+        band = gemm_band(g, M, N, split_bytes);
+        if (band.rows == 0) return hipErrorInvalidValue;
+    }
+    const size_t a_off = split_bytes, b_off = a_off + (w.b_off - w.a_off);
     GemmArgs a{};
     a.A = (const uint16_t*)A; a.B = (const uint16_t*)B; a.C = C; a.c_dtype = c_dtype;
     a.M = M; a.N = N; a.K = w.kp; a.lda = lda; a.ldb = ldb; a.ldc = ldc;
@@ -1009,44 +1057,60 @@ hipError_t launch_gemm_mfma(hipStream_t s, const void* A, int ab_dtype, const vo
         a.ep = *ep;
         a.ep_on = 1;
     }
-    a.tiles_m = (M + t.bm - 1) / t.bm;
-    a.tiles_n = (N + t.bn - 1) / t.bn;
     a.splits = g.splits;
     a.split_stages = g.split_stages;
     a.ws = (float*)workspace;
     {
         const int es = c_dtype == MVLM_F32 ? 4 : 2;
         a.vec_c = ((uintptr_t)C % (4 * es) == 0) && (ldc % 4 == 0) && (strideC % 4 == 0);
-        a.vec_ws = N % 4 == 0;
+        a.vec_ws = N % 4 == 0;   // (of a band too: it ends at C's last column or is whole tiles wide)
         const uintptr_t operands = (uintptr_t)a.ep.bias | (uintptr_t)a.ep.mul | (uintptr_t)a.ep.res;
         a.vec_ep = a.ep_on && a.vec_c && N % 4 == 0 && operands % (4 * es) == 0;
     }
-    const int n = (int)w.pad_a + (int)w.pad_b + 1 + (g.splits > 1 ? 1 : 0);
+    const int bands = ((M + band.rows - 1) / band.rows) * ((N + band.cols - 1) / band.cols);
+    const int n = (int)w.pad_a + (int)w.pad_b + bands * (g.splits > 1 ? 2 : 1);
     int idx = 0;
     if (w.pad_a) {
-        uint16_t* ap = (uint16_t*)((char*)workspace + w.a_off);
+        uint16_t* ap = (uint16_t*)((char*)workspace + a_off);
         const int64_t total = (int64_t)batch * M * w.kp;
         launch_seq(idx++, n, gemm_pad_rows_kernel, dim3(pad_grid(total)), dim3(256), s, (const uint16_t*)A, lda,
                    strideA, M, K, ap, w.kp, total);
         a.A = ap; a.lda = w.kp; a.sA = (int64_t)M * w.kp;
     }
     if (w.pad_b) {
-        uint16_t* bp = (uint16_t*)((char*)workspace + w.b_off);
+        uint16_t* bp = (uint16_t*)((char*)workspace + b_off);
         const int64_t total = (int64_t)batch * N * w.kp;
         launch_seq(idx++, n, gemm_pad_rows_kernel, dim3(pad_grid(total)), dim3(256), s, (const uint16_t*)B, ldb,
                    strideB, N, min(K, kread_b), bp, w.kp, total);
         a.B = bp; a.ldb = w.kp; a.sB = (int64_t)N * w.kp; a.kread_b = w.kp;
     }
-    dim3 grid((unsigned)(a.tiles_m * a.tiles_n), 1, (unsigned)(batch * g.splits));
     const GemmKernel k = t.kernel[ab_dtype == MVLM_BF16][a.ep_on && g.splits == 1];
-    launch_seq(idx++, n, k, grid, dim3(64 * t.waves), s, a);
-    if (g.splits > 1) {
-        const int64_t mn = (int64_t)M * N;
-        const int v = mn % 4 == 0 ? 4 : 1;
-        const auto reduce = v == 4 ? (a.ep_on ? gemm_splitk_reduce_kernel<4, true> : gemm_splitk_reduce_kernel<4, false>)
-                                   : (a.ep_on ? gemm_splitk_reduce_kernel<1, true> : gemm_splitk_reduce_kernel<1, false>);
-        launch_seq(idx++, n, reduce, dim3((unsigned)((mn / v + 255) / 256), (unsigned)batch), dim3(256), s, a);
-    }
+    const size_t cs = dtype_size(c_dtype);
+    auto at = [](const void* base, int64_t offset) { return base ? (const char*)base + offset : nullptr; };
+    for (int r0 = 0; r0 < M; r0 += band.rows)
+        for (int c0 = 0; c0 < N; c0 += band.cols) {
+            GemmArgs b = a;
+            const int64_t c_off = ((int64_t)r0 * ldc + c0) * (int64_t)cs;
+            b.M = std::min(band.rows, M - r0);
+            b.N = std::min(band.cols, N - c0);
+            b.A = a.A + (int64_t)r0 * a.lda;
+            b.B = a.B + (int64_t)c0 * a.ldb;
+            b.C = (char*)C + c_off;
+            b.ep.bias = at(a.ep.bias, c0 * (int64_t)cs);
+            b.ep.mul = at(a.ep.mul, c_off);
+            b.ep.res = at(a.ep.res, c_off);
+            b.tiles_m = (b.M + t.bm - 1) / t.bm;
+            b.tiles_n = (b.N + t.bn - 1) / t.bn;
+            launch_seq(idx++, n, k, dim3((unsigned)(b.tiles_m * b.tiles_n), 1, (unsigned)(batch * g.splits)),
+                       dim3(64 * t.waves), s, b);
+            if (g.splits > 1) {
+                const int64_t mn = (int64_t)b.M * b.N;
+                const int v = mn % 4 == 0 ? 4 : 1;
+                const auto reduce = v == 4 ? (a.ep_on ? gemm_splitk_reduce_kernel<4, true> : gemm_splitk_reduce_kernel<4, false>)
+                                           : (a.ep_on ? gemm_splitk_reduce_kernel<1, true> : gemm_splitk_reduce_kernel<1, false>);
+                launch_seq(idx++, n, reduce, dim3((unsigned)((mn / v + 255) / 256), (unsigned)batch), dim3(256), s, b);
+            }
+        }
     return hipGetLastError();
 }
 

@@ -533,10 +533,14 @@ extern "C" int mvlm_gemm_packed_ex_noalloc(mvlm_device* dev, const mvlm_buffer* 
     Op op{};
     const int st = make_gemm_packed_op(dev, A, a_dtype, W, C, c_dtype, M, N, K, ep, fn, &op);
     if (st != MVLM_OK) return st;
-    if (op.workspace_bytes > (size_t)MVLM_NOALLOC_SCRATCH_BYTES)
-        return set_error(MVLM_ERR_UNSUPPORTED, "%s: %dx%dx%d needs %zu bytes of workspace, above the %zu bytes this "
-                         "entry point holds; use mvlm_gemm_packed_ex", fn, M, N, K, op.workspace_bytes,
-                         (size_t)MVLM_NOALLOC_SCRATCH_BYTES);
+    if (op.workspace_bytes > (size_t)MVLM_NOALLOC_SCRATCH_BYTES) {
+        const size_t least = gemm_workspace_least(M, N, K, op.lda, op.ldb, op.kread_b, op.num_cus, op.ep.any());
+        if (least > (size_t)MVLM_NOALLOC_SCRATCH_BYTES)
+            return set_error(MVLM_ERR_UNSUPPORTED, "%s: %dx%dx%d needs %zu bytes of workspace, above the %zu bytes this "
+                             "entry point holds; use mvlm_gemm_packed_ex", fn, M, N, K, least,
+                             (size_t)MVLM_NOALLOC_SCRATCH_BYTES);
+        op.workspace_bytes = (size_t)MVLM_NOALLOC_SCRATCH_BYTES;
+    }
     if (op.workspace_bytes > 0) {
         if (!dev->noalloc_scratch) return set_error(MVLM_ERR_HIP, "%s: the fixed workspace was not resolved", fn);
         op.workspace = dev->noalloc_scratch;

@@ -2,8 +2,9 @@
 partials, the zero-padded copy of A when K % 8 != 0) in the library's fixed
 per-GPU array instead of an allocation.  Its output must equal
 mvlm_gemm_packed_ex's bit for bit (same kernels, same split order), on calls
-in a row whose second one is smaller, and a shape needing more than the fixed
-array is refused on the host."""
+in a row whose second one is smaller and where the partials of all of C exceed
+the array, and a forced split needing more than the fixed array is refused on
+the host."""
 from __future__ import annotations
 
 import numpy as np
@@ -59,6 +60,32 @@ def test_noalloc_matches_allocating_entry(dev, orc, monkeypatch, order):
             monkeypatch.delenv("MVLM_GEMM_SPLITS", raising=False)
         print(f"[noalloc] {order} call {i}: {M}x{N}x{K} splits={splits}", flush=True)
         run_both(dev, orc, M, N, K, cd, 0x900 + 16 * i)
+
+
+# K-split products whose partials exceed the array: in bands of rows (two or three
+# splits of more than 4Mi outputs; the second off the vector grid) and, where one
+# row of tiles does not fit (eight splits of 150 x 8192), of columns, to the same
+# bits; the last one's copy of A leaves 16 KiB, less than a tile's
+BANDED = [(16384, 300, 8192, F16), (10000, 573, 8192, F16), (6144, 768, 8192, F32), (150, 8192, 32768, F32),
+          (4086, 64, 4101, F32)]
+
+
+@pytest.mark.parametrize("M,N,K,cd", BANDED)
+def test_noalloc_covers_large_outputs_in_bands(dev, M, N, K, cd):
+    print(f"[noalloc] bands {M}x{N}x{K}", flush=True)
+    es = 4 if cd == F32 else 2
+    A, W = dev.alloc(M * K * 2), dev.random_weight(F16, N, K, 0x960)
+    dev.fill_normal(A, F16, M * K, 0x961)
+    bias, mul, res = dev.alloc(N * es), dev.alloc(M * N * es), dev.alloc(M * N * es)
+    for i, (buf, n) in enumerate(((bias, N), (mul, M * N), (res, M * N))):
+        dev.fill_normal(buf, cd, n, 0x962 + i)
+    c_ref, c_new = poisoned(dev, M * N * es), dev.upload(res.download(np.uint8))
+    dev.gemm_packed_ex(A, F16, W, c_ref, cd, M, N, K, bias=bias, act=native.ACT_GELU_TANH, mul=mul, residual=res)
+    dev.gemm_packed_ex_noalloc(A, F16, W, c_new, cd, M, N, K, bias=bias, act=native.ACT_GELU_TANH, mul=mul,
+                               residual=c_new)                 # in place
+    got, ref = c_new.download(np.uint8), c_ref.download(np.uint8)
+    assert np.array_equal(got, ref)
+    assert np.all(np.isfinite(got.view(np.float32 if cd == F32 else np.float16)))
 
 
 def test_noalloc_refuses_workspace_beyond_the_array(dev, orc, monkeypatch):
