@@ -254,11 +254,11 @@ hipError_t stream_attn_check(int count, const void* const* xs, int x_dtype, cons
 // The same attention as launches of its own (no sync area needed).
 hipError_t launch_attn_decode(hipStream_t s, const StreamAttnDesc& d, int num_cus);
 // Skinny GEMM over up to 8 independent problems (quantized weights of one
-// dtype, fp32 X [M][K] and Y [M][N] each, 1 <= M <= 16) in one launch, and a
-// second one that adds the partial sums of rows longer than 2048 weights;
-// those are parked in the workspace (skinny_workspace_bytes; without it one
-// launch does all of it, slower).
-size_t skinny_workspace_bytes(int M, int count, const mvlm_weight* const* ws);
+// dtype, fp32 X [M][K] and Y [M][N] each, 1 <= M <= 16) in one launch, or in two
+// with the partial sums of rows longer than 2048 weights parked in the workspace
+// (skinny_workspace_bytes; a launch that has less does without, on a kernel that
+// is slower for it and rounds differently).
+size_t skinny_workspace_bytes(int M, int count, const mvlm_weight* const* ws, int num_cus);
 hipError_t launch_gemm_skinny_group(hipStream_t s, int M, int count, const float* const* Xs,
                                     const mvlm_weight* const* ws, float* const* Ys, int num_cus,
                                     const Epilogue* eps, void* workspace, size_t workspace_bytes);

@@ -18,6 +18,12 @@
 //    block), that sum coming from one more product of the split x with a
 //    ones operand.
 // One MFMA covers 16 weight rows x one block of 32 weights x 16 rows of X.
+//
+// Two kernels share that arithmetic, chosen per launch by size (skinny_keeps_x).
+// The one in gemm_skinny_kwalk.hip reads X again for every one to four row groups
+// of the weight; the one here keeps X in registers.  The last bits of an output
+// depend on the kernel and so on what else its launch holds.
+//
 // Operand layout of v_mfma_f32_16x16x32_bf16: lane l supplies
 // A[l%16][8*(l/16) .. +7] and B[8*(l/16) .. +7][l%16]; accumulator register i
 // of lane l is D[4*(l/16) + i][l%16].  Here A = X (row m = l%16) and B = w^T
@@ -26,27 +32,28 @@
 // Q4_0 lanes take its bytes 4q..4q+3, i.e. weights 4q..4q+3 (low nibbles) and
 // 16+4q..16+4q+3 (high nibbles).
 //
-// X stays in registers.  A workgroup of 8 waves spans up to 64 blocks of K (a
-// chunk of 2048 weights; longer rows are cut into equal chunks), eight blocks a
-// wave: the wave loads and splits its 16 x 256 slice of X once (96 registers)
-// and then streams the same columns of one 16-row group of the weight after
-// another.  Reading X again for every row group, as a kernel with waves of
-// independent rows does, costs 4 * M * K bytes per row group, 14 times the
-// Q4_0 codes of the group at M = 16, and that traffic (from L2, through the
-// CU's one vector cache) set the time.  The waves' partial tiles meet in LDS
-// after every four row groups.  One workgroup per CU; the row groups of a launch
-// are dealt out so that it takes one round (up to 14 row groups per workgroup).
+// A workgroup of 8 waves spans up to 64 blocks of K (a chunk of 2048 weights;
+// longer rows are cut into equal chunks), eight blocks a wave: the wave loads and
+// splits its 16 x 256 slice of X once (96 registers) and then streams the same
+// columns of one 16-row group of the weight after another.  Reading X again for
+// every row group, as the other kernel does, costs 4 * M * K bytes per row group,
+// 14 times the Q4_0 codes of the group at M = 16, and that traffic (from L2,
+// through the CU's one vector cache) sets the time of a launch of many row
+// groups.  The waves' partial tiles meet in LDS after every four row groups.  One
+// workgroup per CU; the row groups of a launch are dealt out in whole rounds (up
+// to 14 row groups per workgroup).
 //
-// Against a kernel whose workgroups each read all of X for one to four row
-// groups, a Phi-1.5 step (49 grouped launches) of M = 16 went 831 -> 680 us
-// (Q4_0) and 867 -> 720 us (Q8_0), of M = 8 785 -> 626 and 806 -> 672 us, its LM
-// head 37 -> 22 and 38 -> 27 us.  What bounds a launch now (time stamps of the
-// M = 16 QKV + fc1 launch, 10.5 us): 128 KiB of X into every CU and its split,
-// 5 us before the first products, then 0.8 us (Q4_0, vector ALU and matrix core
-// in turn) to 1.2 us (Q8_0, HBM) per row group.  Sixteen waves of four blocks
-// each spend longer in the barriers (Q4_0 M = 16 707 us, Q8_0 691 us); codes
-// requested before X, with deeper rings, delay X by more than they gain (697
-// and 822 us).
+// Against the other kernel, a Phi-1.5 step (49 grouped launches) of M = 16 went
+// 831 -> 670 us (Q4_0) and 867 -> 720 us (Q8_0), of M = 8 785 -> 626 and 806 ->
+// 672 us, its LM head 39 -> 22 and 39 -> 27 us.  What bounds a launch now (time
+// stamps of the M = 16 QKV + fc1 launch, 10.5 us): 128 KiB of X into every CU and
+// its split, 5 us before the first products, then 0.8 us (Q4_0, vector ALU and
+// matrix core in turn) to 1.2 us (Q8_0, HBM) per row group.  Sixteen waves of
+// four blocks each spend longer in the barriers (Q4_0 M = 16 707 us, Q8_0 691
+// us); codes requested before X, with deeper rings, delay X by more than they
+// gain (697 and 822 us).  A wave loads eight blocks of X and codes even where it
+// owns fewer (rows below 2048 weights), which costs little of that, but makes up
+// most of a launch of short rows: the other kernel's part.
 //
 // Codes go to the wave's own LDS ring with direct 16-byte loads, several row
 // groups ahead, and are read back per lane (loading the MFMA layout straight
@@ -55,41 +62,14 @@
 //
 // Rows of more than one chunk (K > 2048): a workgroup takes one chunk of its
 // rows and writes its sums to the device workspace, and a second launch adds
-// the chunks in order and applies the epilogue.  Without workspace a workgroup
-// walks the chunks itself, reloading X for every row group.  The
-// order of every sum depends on K alone, so an output has the same bits in a
-// single and in a grouped call.
-#include "common.h"
-#include "device_math.h"
+// the chunks in order and applies the epilogue.  Without workspace the launch
+// goes to the other kernel.
+#include "gemm_skinny.h"
 
 #include <algorithm>
+#include <cstdlib>
 
 namespace mvlm {
-
-typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8v;
-
-// top 16 bits of two floats -> one packed bf16 pair (truncation)
-__device__ __forceinline__ uint32_t pack_hi16(float lo_elem, float hi_elem) {
-    return __builtin_amdgcn_perm(__float_as_uint(hi_elem), __float_as_uint(lo_elem), 0x07060302u);
-}
-
-// x[0..7] -> three bf16x8 parts with x = p1 + p2 + p3 (+ |residual| < 2^-24 |x|)
-__device__ __forceinline__ void split3(const float (&x)[8], u32x4& p1, u32x4& p2, u32x4& p3) {
-    float r1[8], r2[8];
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-        const float a = __uint_as_float(__float_as_uint(x[j]) & 0xFFFF0000u);
-        r1[j] = x[j] - a;                                   // exact
-        const float b = __uint_as_float(__float_as_uint(r1[j]) & 0xFFFF0000u);
-        r2[j] = r1[j] - b;                                  // exact
-    }
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        p1[j] = pack_hi16(x[2 * j], x[2 * j + 1]);
-        p2[j] = pack_hi16(r1[2 * j], r1[2 * j + 1]);
-        p3[j] = pack_hi16(r2[2 * j], r2[2 * j + 1]);
-    }
-}
 
 // A lane's 8 codes of a block as bf16 (small integers, exact).  Q4_0: raw is
 // one dword, the result the raw nibbles c (0..15), low nibbles first; the -8
@@ -113,11 +93,6 @@ __device__ __forceinline__ u32x4 codes_to_bf16(u32x2 raw) {
         for (int j = 0; j < 4; ++j) out[j] = pack_hi16(v[2 * j], v[2 * j + 1]);
     }
     return out;
-}
-
-__device__ __forceinline__ f32x4 mfma16(u32x4 a, u32x4 b, f32x4 c) {
-    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8v, a), __builtin_bit_cast(bf16x8v, b), c,
-                                                   0, 0, 0);
 }
 
 // Barrier that orders the workgroup's LDS accesses and leaves loads from
@@ -163,7 +138,7 @@ struct SkinnyProblem {
     const uint8_t* codes;
     const uint16_t* scales;
     float* Y;
-    float* part;                   // [chunks][M][N] sums of the chunks, or null: one workgroup walks them
+    float* part;                   // [chunks][M][N] sums of the chunks; null if there is one
     uint32_t ld;                   // code bytes per row
     int N, nb;                     // rows, blocks of K
     int chunks, chunk_blocks;      // chunks of K and blocks per chunk (the last may have fewer)
@@ -172,7 +147,6 @@ struct SkinnyProblem {
     int ep_on;
     Epilogue ep;
 };
-constexpr int SKINNY_MAX_GROUP = 8;
 struct SkinnyGroup {
     int count, M;
     int block_begin[SKINNY_MAX_GROUP];   // first workgroup of each problem in the grid
@@ -203,11 +177,10 @@ __global__ __launch_bounds__(64 * SK_WAVES) void gemm_skinny_kernel(const Skinny
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int l16 = lane & 15, q = lane >> 4;
 
-    // this workgroup's row groups [rg0, rg0 + units) and chunks [c_begin, c_end)
+    // this workgroup's row groups [rg0, rg0 + units) and chunk c
     const int bid = (int)blockIdx.x - g.block_begin[pi];
-    const bool split = cpart != nullptr;
-    const int range = split && chunks > 1 ? (int)__umulhi((uint32_t)bid, chunk_div) : bid;
-    const int c_begin = split ? bid - range * chunks : 0, c_end = split ? c_begin + 1 : chunks;
+    const int range = chunks > 1 ? (int)__umulhi((uint32_t)bid, chunk_div) : bid;
+    const int c = bid - range * chunks;
     const int rg0 = range * rows;
     const int units = min(rows, (N + 15) / 16 - rg0);
     const int n0 = 16 * rg0;
@@ -254,197 +227,186 @@ __global__ __launch_bounds__(64 * SK_WAVES) void gemm_skinny_kernel(const Skinny
     f32x4 sx[SK_KB];                                  // Q4_0: -8 times its block sums
     f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
 
-    // Row groups u0..u1 of chunk c.  A workgroup with one chunk has one such
-    // segment; one that walks several takes each row group through all of them.
-    const int span = c_end - c_begin == 1 ? units : 1;
-    for (int u0 = 0; u0 < units; u0 += span) {
-        const int u1 = min(u0 + span, units);
-        for (int c = c_begin; c < c_end; ++c) {
-            const int cb0 = c * chunk_blocks, cb = min(chunk_blocks, nb - cb0);
-            const int per = (cb + SK_WAVES - 1) / SK_WAVES;
-            const int cnt = max(0, min(per, cb - wave * per));   // this wave's blocks
-            const int b0 = cb0 + wave * per;
-            const bool last_chunk = c + 1 == c_end;
-            if (u0 > 0 || c > c_begin) block_sync();             // the scales are about to be replaced
+    const int cb0 = c * chunk_blocks, cb = min(chunk_blocks, nb - cb0);
+    const int per = (cb + SK_WAVES - 1) / SK_WAVES;
+    const int cnt = max(0, min(per, cb - wave * per));   // this wave's blocks
+    const int b0 = cb0 + wave * per;
 
-            // a lane's byte of the codes for each direct load of row group 0,
-            // and its last one in bounds (rows past N repeat row N - 1)
-            uint32_t voff[L::NDMA], vmax[L::NDMA];
+    // a lane's byte of the codes for each direct load of row group 0,
+    // and its last one in bounds (rows past N repeat row N - 1)
+    uint32_t voff[L::NDMA], vmax[L::NDMA];
 #pragma unroll
-            for (int t = 0; t < L::NDMA; ++t) {
-                const int r = t * L::RPI + dma_row;
-                const uint32_t off = (uint32_t)min(b0 * L::BB + 16 * L::piece(dma_piece, r), nb * L::BB - 16);
-                voff[t] = (uint32_t)(n0 + r) * ld + off;
-                vmax[t] = (uint32_t)(N - 1) * ld + off;
-            }
-            auto issue = [&](int u, int slot) {
-                const uint32_t dst = __builtin_amdgcn_readfirstlane(ring + (uint32_t)(slot * L::SLOT));
+    for (int t = 0; t < L::NDMA; ++t) {
+        const int r = t * L::RPI + dma_row;
+        const uint32_t off = (uint32_t)min(b0 * L::BB + 16 * L::piece(dma_piece, r), nb * L::BB - 16);
+        voff[t] = (uint32_t)(n0 + r) * ld + off;
+        vmax[t] = (uint32_t)(N - 1) * ld + off;
+    }
+    auto issue = [&](int u, int slot) {
+        const uint32_t dst = __builtin_amdgcn_readfirstlane(ring + (uint32_t)(slot * L::SLOT));
 #pragma unroll
-                for (int t = 0; t < L::NDMA; ++t)
-                    asm_buffer_load_lds_b128(crs, min(voff[t] + (uint32_t)(16 * u) * ld, vmax[t]), dst + t * 1024);
-            };
+        for (int t = 0; t < L::NDMA; ++t)
+            asm_buffer_load_lds_b128(crs, min(voff[t] + (uint32_t)(16 * u) * ld, vmax[t]), dst + t * 1024);
+    };
 
-            // The scales, the first epilogue operands, X, then the first row
-            // groups of codes (past the last one, and in waves without blocks,
-            // the clamped addresses repeat loads: no branch may stand between
-            // the X loads and the wait for them, where the compiler could move
-            // their registers).  Scales: dwords of the rows' scales of this
-            // chunk, from the dword its first block lies in; past the array
-            // they are clamped to its last dword.
-            {
-                const int total = (u1 - u0) * 16 * SK_SCALE_DW;
-                const uint32_t last = ((uint32_t)N * (uint32_t)nb * 2 - 1) & ~3u;
-                for (int i = wave * 64; i < total; i += 64 * SK_WAVES) {
-                    const uint32_t e = (uint32_t)min(i + lane, total - 1), r = e / SK_SCALE_DW, dw = e - r * SK_SCALE_DW;
-                    const uint32_t row = min((uint32_t)(n0 + 16 * u0) + r, (uint32_t)(N - 1));
-                    const uint32_t off = (((row * (uint32_t)nb + (uint32_t)cb0) * 2) & ~3u) + 4 * dw;
-                    asm_buffer_load_lds_b32(srs, min(off, last),
-                                            __builtin_amdgcn_readfirstlane(scale_base + 4u * (uint32_t)i));
-                }
-            }
-            if (ep && last_chunk && u0 + duty < u1) issue_ep(u0 + duty);
-            u32x4 xr[SK_KB][2];
+    // The scales, the first epilogue operands, X, then the first row
+    // groups of codes (past the last one, and in waves without blocks,
+    // the clamped addresses repeat loads: no branch may stand between
+    // the X loads and the wait for them, where the compiler could move
+    // their registers).  Scales: dwords of the rows' scales of this
+    // chunk, from the dword its first block lies in; past the array
+    // they are clamped to its last dword.
+    {
+        const int total = units * 16 * SK_SCALE_DW;
+        const uint32_t last = ((uint32_t)N * (uint32_t)nb * 2 - 1) & ~3u;
+        for (int i = wave * 64; i < total; i += 64 * SK_WAVES) {
+            const uint32_t e = (uint32_t)min(i + lane, total - 1), r = e / SK_SCALE_DW, dw = e - r * SK_SCALE_DW;
+            const uint32_t row = min((uint32_t)n0 + r, (uint32_t)(N - 1));
+            const uint32_t off = (((row * (uint32_t)nb + (uint32_t)cb0) * 2) & ~3u) + 4 * dw;
+            asm_buffer_load_lds_b32(srs, min(off, last),
+                                    __builtin_amdgcn_readfirstlane(scale_base + 4u * (uint32_t)i));
+        }
+    }
+    if (ep && duty < units) issue_ep(duty);
+    u32x4 xr[SK_KB][2];
 #pragma unroll
-            for (int j = 0; j < SK_KB; ++j) {
-                const uint32_t base = (uint32_t)(xm * nb + min(b0 + j, nb - 1)) * 128u;
-                xr[j][0] = asm_buffer_load_b128(xrs, base + 4u * (uint32_t)(xodd ? x1 : x0));
-                xr[j][1] = asm_buffer_load_b128(xrs, base + 4u * (uint32_t)(xodd ? x0 : x1));
-            }
+    for (int j = 0; j < SK_KB; ++j) {
+        const uint32_t base = (uint32_t)(xm * nb + min(b0 + j, nb - 1)) * 128u;
+        xr[j][0] = asm_buffer_load_b128(xrs, base + 4u * (uint32_t)(xodd ? x1 : x0));
+        xr[j][1] = asm_buffer_load_b128(xrs, base + 4u * (uint32_t)(xodd ? x0 : x1));
+    }
 #pragma unroll
-            for (int d = 0; d < L::DEPTH; ++d) issue(min(u0 + d, u1 - 1), d);
-            asm_wait_vmcnt<L::DEPTH * L::NDMA>();
+    for (int d = 0; d < L::DEPTH; ++d) issue(min(d, units - 1), d);
+    asm_wait_vmcnt<L::DEPTH * L::NDMA>();
 #pragma unroll
-            for (int j = 0; j < SK_KB; ++j) {
-                asm_pin(xr[j][0]);
-                asm_pin(xr[j][1]);
-                if (j >= cnt) xr[j][0] = xr[j][1] = u32x4{0u, 0u, 0u, 0u};   // blocks past the wave's range
-            }
+    for (int j = 0; j < SK_KB; ++j) {
+        asm_pin(xr[j][0]);
+        asm_pin(xr[j][1]);
+        if (j >= cnt) xr[j][0] = xr[j][1] = u32x4{0u, 0u, 0u, 0u};   // blocks past the wave's range
+    }
 #pragma unroll
-            for (int j = 0; j < SK_KB; ++j) {
-                float x[8];
+    for (int j = 0; j < SK_KB; ++j) {
+        float x[8];
 #pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    x[e] = __uint_as_float(xodd ? xr[j][1][e] : xr[j][0][e]);
-                    x[4 + e] = __uint_as_float(xodd ? xr[j][0][e] : xr[j][1][e]);
-                }
-                split3(x, xp[j][0], xp[j][1], xp[j][2]);
-                sx[j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-                if constexpr (Q4) {
-                    const u32x4 ones = {0x3F803F80u, 0x3F803F80u, 0x3F803F80u, 0x3F803F80u};   // bf16 1.0 pairs
-                    sx[j] = mfma16(xp[j][0], ones, sx[j]);
-                    sx[j] = mfma16(xp[j][1], ones, sx[j]);
-                    sx[j] = mfma16(xp[j][2], ones, sx[j]);
+        for (int e = 0; e < 4; ++e) {
+            x[e] = __uint_as_float(xodd ? xr[j][1][e] : xr[j][0][e]);
+            x[4 + e] = __uint_as_float(xodd ? xr[j][0][e] : xr[j][1][e]);
+        }
+        split3(x, xp[j][0], xp[j][1], xp[j][2]);
+        sx[j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+        if constexpr (Q4) {
+            const u32x4 ones = {0x3F803F80u, 0x3F803F80u, 0x3F803F80u, 0x3F803F80u};   // bf16 1.0 pairs
+            sx[j] = mfma16(xp[j][0], ones, sx[j]);
+            sx[j] = mfma16(xp[j][1], ones, sx[j]);
+            sx[j] = mfma16(xp[j][2], ones, sx[j]);
 #pragma unroll
-                    for (int i = 0; i < 4; ++i) sx[j][i] *= -8.0f;
-                }
-            }
-            if (cnt == 0) asm_wait_vmcnt<0>();        // nothing waits for this wave's repeats below
-            block_sync();                             // the scales of every wave have landed
+            for (int i = 0; i < 4; ++i) sx[j][i] *= -8.0f;
+        }
+    }
+    if (cnt == 0) asm_wait_vmcnt<0>();        // nothing waits for this wave's repeats below
+    block_sync();                             // the scales of every wave have landed
 
-            // a lane's scales: row l16 of the row group, from the wave's first
-            // block; its codes of block j: a dword (Q4_0) or two (Q8_0)
-            const uint32_t s_lane = scale_base + (uint32_t)(l16 * SK_SCALE_DW * 4 + 2 * (((l16 * nb + cb0) & 1) + wave * per));
-            const uint32_t c_lane = ring + (uint32_t)(l16 * L::CB + 16 * L::piece(Q4 ? 0 : q >> 1, l16) +
-                                                      (Q4 ? 4 * q : 8 * (q & 1)));
-            // extra: epilogue loads of the wave issued after this row group's codes
-            auto unit = [&](int u, int slot, bool extra) {
-                if (cnt == 0) return;
-                if (u + L::DEPTH > u1) asm_wait_vmcnt<0>();
-                else if (extra) asm_wait_vmcnt<(L::DEPTH - 1) * L::NDMA + SK_EP_LOADS>();
-                else asm_wait_vmcnt<(L::DEPTH - 1) * L::NDMA>();
-                const uint32_t src = c_lane + (uint32_t)(slot * L::SLOT);
-                const uint32_t ssrc = s_lane + (uint32_t)((u - u0) * SK_SCALE_ROWS);
-                u32x2 raw[SK_KB];
-                uint32_t dh[SK_KB];
-                static_for<SK_KB>([&](auto J) {
-                    constexpr int j = decltype(J)::value;
-                    // a row's slot is aligned to its size: XOR moves between pieces
-                    if constexpr (Q4) raw[j][0] = asm_lds_read_b32(src ^ (uint32_t)(16 * j));
-                    else raw[j] = asm_lds_read_b64(src ^ (uint32_t)(32 * j));
-                    dh[j] = asm_lds_read_u16<2 * j>(ssrc);
-                });
-                asm_wait_lgkmcnt<0>();
+    // a lane's scales: row l16 of the row group, from the wave's first
+    // block; its codes of block j: a dword (Q4_0) or two (Q8_0)
+    const uint32_t s_lane = scale_base + (uint32_t)(l16 * SK_SCALE_DW * 4 + 2 * (((l16 * nb + cb0) & 1) + wave * per));
+    const uint32_t c_lane = ring + (uint32_t)(l16 * L::CB + 16 * L::piece(Q4 ? 0 : q >> 1, l16) +
+                                              (Q4 ? 4 * q : 8 * (q & 1)));
+    // extra: epilogue loads of the wave issued after this row group's codes
+    auto unit = [&](int u, int slot, bool extra) {
+        if (cnt == 0) return;
+        if (u + L::DEPTH > units) asm_wait_vmcnt<0>();
+        else if (extra) asm_wait_vmcnt<(L::DEPTH - 1) * L::NDMA + SK_EP_LOADS>();
+        else asm_wait_vmcnt<(L::DEPTH - 1) * L::NDMA>();
+        const uint32_t src = c_lane + (uint32_t)(slot * L::SLOT);
+        const uint32_t ssrc = s_lane + (uint32_t)(u * SK_SCALE_ROWS);
+        u32x2 raw[SK_KB];
+        uint32_t dh[SK_KB];
+        static_for<SK_KB>([&](auto J) {
+            constexpr int j = decltype(J)::value;
+            // a row's slot is aligned to its size: XOR moves between pieces
+            if constexpr (Q4) raw[j][0] = asm_lds_read_b32(src ^ (uint32_t)(16 * j));
+            else raw[j] = asm_lds_read_b64(src ^ (uint32_t)(32 * j));
+            dh[j] = asm_lds_read_u16<2 * j>(ssrc);
+        });
+        asm_wait_lgkmcnt<0>();
 #pragma unroll
-                for (int j = 0; j < SK_KB; ++j) {
-                    asm_pin(raw[j]);
-                    asm_pin(dh[j]);
-                }
-                if (u + L::DEPTH < u1) issue(u + L::DEPTH, slot);
-                // four blocks at a time (those past the wave's range: X and d are zero)
+        for (int j = 0; j < SK_KB; ++j) {
+            asm_pin(raw[j]);
+            asm_pin(dh[j]);
+        }
+        if (u + L::DEPTH < units) issue(u + L::DEPTH, slot);
+        // four blocks at a time (those past the wave's range: X and d are zero)
 #pragma unroll
-                for (int h = 0; h < SK_KB; h += 4) {
-                    if (h >= cnt) break;
-                    f32x4 p[4];
-                    u32x4 w[4];
+        for (int h = 0; h < SK_KB; h += 4) {
+            if (h >= cnt) break;
+            f32x4 p[4];
+            u32x4 w[4];
 #pragma unroll
-                    for (int j = 0; j < 4; ++j) w[j] = codes_to_bf16<Q4>(raw[h + j]);
+            for (int j = 0; j < 4; ++j) w[j] = codes_to_bf16<Q4>(raw[h + j]);
 #pragma unroll
-                    for (int j = 0; j < 4; ++j) p[j] = mfma16(xp[h + j][0], w[j], sx[h + j]);
+            for (int j = 0; j < 4; ++j) p[j] = mfma16(xp[h + j][0], w[j], sx[h + j]);
 #pragma unroll
-                    for (int j = 0; j < 4; ++j) p[j] = mfma16(xp[h + j][1], w[j], p[j]);
+            for (int j = 0; j < 4; ++j) p[j] = mfma16(xp[h + j][1], w[j], p[j]);
 #pragma unroll
-                    for (int j = 0; j < 4; ++j) p[j] = mfma16(xp[h + j][2], w[j], p[j]);
+            for (int j = 0; j < 4; ++j) p[j] = mfma16(xp[h + j][2], w[j], p[j]);
 #pragma unroll
-                    for (int j = 0; j < 4; ++j) {
-                        const float d = h + j < cnt ? f16_bits_to_f32((uint16_t)dh[h + j]) : 0.0f;
+            for (int j = 0; j < 4; ++j) {
+                const float d = h + j < cnt ? f16_bits_to_f32((uint16_t)dh[h + j]) : 0.0f;
 #pragma unroll
-                        for (int i = 0; i < 4; ++i) acc[i] = __builtin_fmaf(d, p[j][i], acc[i]);
-                    }
-                }
-            };
-
-            int slot = 0;
-            for (int ub = u0; ub < u1; ub += SK_BATCH) {
-                const int un = min(SK_BATCH, u1 - ub);
-                for (int k = 0; k < un; ++k) {
-                    if (c == c_begin) acc = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-                    unit(ub + k, slot, ep && ub > u0 && k < L::DEPTH && ub + duty < u1);
-                    slot = slot + 1 == L::DEPTH ? 0 : slot + 1;
-                    if (last_chunk) *(reinterpret_cast<f32x4*>(part) + (k * SK_WAVES + wave) * 64 + lane) = acc;
-                }
-                if (!last_chunk) continue;
-                block_sync();
-                if (duty < un && 8 * (wave & 1) < M) {
-                    const int u = ub + duty, n = n0 + 16 * u + l16;
-                    const float* from = part + duty * SK_WAVES * 256 + ((wave & 1) * 32 + l16) * 4 + q;
-                    float sum[2] = {from[0], from[64]};
-#pragma unroll
-                    for (int w = 1; w < SK_WAVES; ++w) {        // in wave order
-                        sum[0] += from[w * 256];
-                        sum[1] += from[w * 256 + 64];
-                    }
-                    if (ep) {
-                        // requested before the codes of the batch's refills, of
-                        // which a wave without blocks has none
-                        if (cnt > 0 && ub + SK_BATCH + L::DEPTH <= u1) asm_wait_vmcnt<SK_BATCH * L::NDMA>();
-                        else asm_wait_vmcnt<0>();
-                        float v[SK_EP_LOADS];
-#pragma unroll
-                        for (int i = 0; i < SK_EP_LOADS; ++i)
-                            v[i] = __uint_as_float(asm_lds_read_b32(ep_base + (uint32_t)(256 * i + 4 * lane)));
-                        asm_wait_lgkmcnt<0>();
-#pragma unroll
-                        for (int i = 0; i < SK_EP_LOADS; ++i) asm_pin(v[i]);
-                        if (u + SK_BATCH < u1) issue_ep(u + SK_BATCH);
-#pragma unroll
-                        for (int i = 0; i < 2; ++i) {
-                            float o = sum[i];
-                            if (P.ep.bias) o += v[0];
-                            if (P.ep.act == 1) o = gelu_tanh(o);
-                            else if (P.ep.act == 2) o = silu(o);
-                            if (P.ep.mul) o *= v[1 + i];
-                            if (P.ep.res) o += v[3 + i];
-                            sum[i] = o;
-                        }
-                    }
-                    float* out = split ? cpart + (int64_t)c * M * N : P.Y;
-#pragma unroll
-                    for (int i = 0; i < 2; ++i)
-                        if (om + 4 * i < M && n < N) out[(int64_t)(om + 4 * i) * N + n] = sum[i];
-                }
-                if (ub + SK_BATCH < u1) block_sync();   // the sums are read before the next batch's are written
+                for (int i = 0; i < 4; ++i) acc[i] = __builtin_fmaf(d, p[j][i], acc[i]);
             }
         }
+    };
+
+    int slot = 0;
+    for (int ub = 0; ub < units; ub += SK_BATCH) {
+        const int un = min(SK_BATCH, units - ub);
+        for (int k = 0; k < un; ++k) {
+            acc = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+            unit(ub + k, slot, ep && ub > 0 && k < L::DEPTH && ub + duty < units);
+            slot = slot + 1 == L::DEPTH ? 0 : slot + 1;
+            *(reinterpret_cast<f32x4*>(part) + (k * SK_WAVES + wave) * 64 + lane) = acc;
+        }
+        block_sync();
+        if (duty < un && 8 * (wave & 1) < M) {
+            const int u = ub + duty, n = n0 + 16 * u + l16;
+            const float* from = part + duty * SK_WAVES * 256 + ((wave & 1) * 32 + l16) * 4 + q;
+            float sum[2] = {from[0], from[64]};
+#pragma unroll
+            for (int w = 1; w < SK_WAVES; ++w) {        // in wave order
+                sum[0] += from[w * 256];
+                sum[1] += from[w * 256 + 64];
+            }
+            if (ep) {
+                // requested before the codes of the batch's refills, of
+                // which a wave without blocks has none
+                if (cnt > 0 && ub + SK_BATCH + L::DEPTH <= units) asm_wait_vmcnt<SK_BATCH * L::NDMA>();
+                else asm_wait_vmcnt<0>();
+                float v[SK_EP_LOADS];
+#pragma unroll
+                for (int i = 0; i < SK_EP_LOADS; ++i)
+                    v[i] = __uint_as_float(asm_lds_read_b32(ep_base + (uint32_t)(256 * i + 4 * lane)));
+                asm_wait_lgkmcnt<0>();
+#pragma unroll
+                for (int i = 0; i < SK_EP_LOADS; ++i) asm_pin(v[i]);
+                if (u + SK_BATCH < units) issue_ep(u + SK_BATCH);
+#pragma unroll
+                for (int i = 0; i < 2; ++i) {
+                    float o = sum[i];
+                    if (P.ep.bias) o += v[0];
+                    if (P.ep.act == 1) o = gelu_tanh(o);
+                    else if (P.ep.act == 2) o = silu(o);
+                    if (P.ep.mul) o *= v[1 + i];
+                    if (P.ep.res) o += v[3 + i];
+                    sum[i] = o;
+                }
+            }
+            float* out = cpart ? cpart + (int64_t)c * M * N : P.Y;
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+                if (om + 4 * i < M && n < N) out[(int64_t)(om + 4 * i) * N + n] = sum[i];
+        }
+        if (ub + SK_BATCH < units) block_sync();   // the sums are read before the next batch's are written
     }
 }
 
@@ -461,7 +423,60 @@ __global__ __launch_bounds__(256) void skinny_reduce_kernel(const SkinnyGroup g)
 
 static int skinny_chunks(int K) { return (K / 32 + SK_CHUNK - 1) / SK_CHUNK; }
 
-size_t skinny_workspace_bytes(int M, int count, const mvlm_weight* const* ws) {
+// How a launch of the X-stationary kernel is dealt out: row groups per workgroup,
+// workgroups, and rounds of one workgroup per CU (the fewest, of the fewest row
+// groups each).
+struct SkinnyDeal {
+    int rows;
+    int64_t blocks, rounds;
+};
+static SkinnyDeal skinny_deal(int count, const mvlm_weight* const* ws, int num_cus) {
+    int64_t units = 0;
+    for (int i = 0; i < count; ++i) units += (int64_t)((ws[i]->N + 15) / 16) * skinny_chunks(ws[i]->K);
+    for (int64_t rounds = (units + (int64_t)num_cus * SK_MAX_RG - 1) / ((int64_t)num_cus * SK_MAX_RG);; ++rounds)
+        for (int rows = (int)((units + num_cus * rounds - 1) / (num_cus * rounds)); rows <= SK_MAX_RG; ++rows) {
+            int64_t blocks = 0;
+            for (int i = 0; i < count; ++i)
+                blocks += (int64_t)(((ws[i]->N + 15) / 16 + rows - 1) / rows) * skinny_chunks(ws[i]->K);
+            if (blocks <= num_cus * rounds) return {rows, blocks, rounds};
+        }
+}
+
+// Whether the X-stationary kernel takes a launch: where its modelled time is no
+// longer than that of the kernel that walks K.  Bringing X in once (2.2 us, and a
+// second launch of 2.5 us where rows are cut) pays for launches of many row
+// groups or long rows; the other kernel is ahead on few row groups, on short rows
+// and on rows little longer than a whole number of chunks.  Both measured at
+// M = 16, Q8_0: 2048 x 64 4.6 us (K walked) and 7.0 (X kept), 8192 x 768 7.1 and
+// 9.2, 8192 x 3072 12.1 and 15.0; 51200 x 2048 38.7 and 27.3, 2048 x 8192 16.6 and
+// 14.0, 32000 x 1024 15.4 and 14.3.  The costs are fitted to the times of both
+// over 2700 launches (N 64 .. 51200, K 64 .. 11008, M 5 .. 16, single and
+// grouped): the choice is 0.3% from the faster one on average, and more than 6%
+// from it in 2% of them.  MVLM_SKINNY_FORM=x or k forces one (tests, tuning; read
+// at every launch).
+static bool skinny_keeps_x(int M, int count, const mvlm_weight* const* ws, int num_cus) {
+    if (const char* force = std::getenv("MVLM_SKINNY_FORM")) return force[0] == 'x';
+    struct Cost {
+        double launch, row_group, block, row, cut, partial, round;
+    };
+    constexpr Cost kQ8{5.7, 0.50, 0.0168, 0.091, 2.5, 1.9, 5.2}, kQ4{5.5, 0.48, 0.0116, 0.084, 2.4, 2.0, 4.2};
+    const Cost& c = ws[0]->dtype == MVLM_Q4_0 ? kQ4 : kQ8;
+    const SkinnyDeal deal = skinny_deal(count, ws, num_cus);
+    double units = 0, blocks = 0, parts = 0;   // row groups times chunks, their blocks of K, 10^6 partial sums
+    for (int i = 0; i < count; ++i) {
+        const int chunks = skinny_chunks(ws[i]->K), nb = ws[i]->K / 32;
+        const double u = (double)((ws[i]->N + 15) / 16) * chunks;
+        units += u;
+        blocks += u * ((nb + chunks - 1) / chunks);
+        if (chunks > 1) parts += 1e-6 * M * ws[i]->N * chunks;
+    }
+    const double busy = std::min((double)deal.blocks / num_cus, (double)deal.rounds) * deal.rows;
+    const double us = c.launch + c.row_group * deal.rounds * deal.rows + c.block * busy * (blocks / units) + c.row * M +
+                      (parts > 0 ? c.cut + c.partial * parts : 0.0) + c.round * (deal.rounds - 1);
+    return us < 1.01 * skinny_kwalk_us(M, count, ws, num_cus);
+}
+
+static size_t skinny_partial_bytes(int M, int count, const mvlm_weight* const* ws) {
     size_t bytes = 0;
     for (int i = 0; i < count; ++i) {
         const int chunks = skinny_chunks(ws[i]->K);
@@ -470,63 +485,41 @@ size_t skinny_workspace_bytes(int M, int count, const mvlm_weight* const* ws) {
     return bytes;
 }
 
+size_t skinny_workspace_bytes(int M, int count, const mvlm_weight* const* ws, int num_cus) {
+    return skinny_keeps_x(M, count, ws, num_cus > 0 ? num_cus : 256) ? skinny_partial_bytes(M, count, ws) : 0;
+}
+
 // Which launches are taken: K a multiple of 32, codes and X within 32-bit
-// buffer offsets, and rows whose scales fit beside the code slots of the
-// workgroup that a launch of this many row groups took when a workgroup staged
-// whole rows (the limit callers know; nothing below depends on it).
+// buffer offsets, and rows whose scales fit the LDS of the kernel that walks K,
+// which any launch may come down to (it needs no workspace).
 bool skinny_supported(int count, const mvlm_weight* const* ws, int num_cus) {
-    if (num_cus <= 0) num_cus = 256;
-    int64_t groups = 0;
-    for (int i = 0; i < count; ++i) groups += (ws[i]->N + 15) / 16;
-    const bool q4 = count > 0 && ws[0]->dtype == MVLM_Q4_0;
-    int rows = 16;                                    // rows and code-slot bytes of that workgroup
-    size_t slots = q4 ? 32 * 1024 : 64 * 1024;
-    if (q4 && groups >= 3 * (int64_t)num_cus && groups <= 4 * (int64_t)num_cus) { rows = 64; slots = 64 * 1024; }
-    else if (groups >= 2 * (int64_t)num_cus) rows = 32;
-    else if (groups >= num_cus && !q4) slots = 32 * 1024;
     for (int i = 0; i < count; ++i) {
         const mvlm_weight* w = ws[i];
         if (!is_quant(w->dtype) || w->K % 32 != 0) return false;
         if (w->bytes > 0x7FFFFFFF || (int64_t)16 * w->K * 4 > 0x7FFFFFFF) return false;   // 32-bit buffer offsets
-        if (((size_t)rows * (w->K / 32) * 2 + 255) / 256 * 256 + slots > 160 * 1024) return false;
     }
-    return true;
+    return skinny_kwalk_fits(count, ws, num_cus > 0 ? num_cus : 256);
 }
 
 template <bool Q4>
-static hipError_t launch_skinny(hipStream_t s, SkinnyGroup& g, int num_cus) {
+static hipError_t launch_skinny(hipStream_t s, SkinnyGroup& g, const SkinnyDeal& deal) {
     constexpr auto kernel = gemm_skinny_kernel<Q4>;
     constexpr int lds = SkinnyLayout<Q4>::LDS;
     if (const hipError_t e = allow_dynamic_lds<kernel>(lds); e != hipSuccess) return e;
-    // Row groups per workgroup: the fewest that deal the launch out in whole
-    // rounds of one workgroup per CU.
-    int64_t units = 0;
-    for (int i = 0; i < g.count; ++i) units += (int64_t)((g.p[i].N + 15) / 16) * (g.p[i].part ? g.p[i].chunks : 1);
-    const int64_t rounds = (units + (int64_t)num_cus * SK_MAX_RG - 1) / ((int64_t)num_cus * SK_MAX_RG);
-    int rows = (int)((units + num_cus * rounds - 1) / (num_cus * rounds));
-    unsigned blocks = 0;
-    for (;; ++rows) {
-        blocks = 0;
-        for (int i = 0; i < g.count; ++i) {
-            SkinnyProblem& p = g.p[i];
-            p.rows = rows;
-            g.block_begin[i] = (int)blocks;
-            blocks += (unsigned)(((p.N + 15) / 16 + rows - 1) / rows * (p.part ? p.chunks : 1));
-        }
-        if (blocks <= num_cus * rounds || rows >= SK_MAX_RG) break;
+    int64_t most = 0, begin = 0;   // outputs of the largest problem cut over K; workgroups dealt out
+    for (int i = 0; i < g.count; ++i) {
+        SkinnyProblem& p = g.p[i];
+        p.rows = deal.rows;
+        g.block_begin[i] = (int)begin;
+        begin += (int64_t)(((p.N + 15) / 16 + p.rows - 1) / p.rows) * p.chunks;
+        if (p.part) most = std::max(most, (int64_t)g.M * p.N);
     }
-    bool split = false;
-    int64_t most = 0;
-    for (int i = 0; i < g.count; ++i)
-        if (g.p[i].part) {
-            split = true;
-            most = std::max(most, (int64_t)g.M * g.p[i].N);
-        }
-    if (!split) {
-        launch_kernel(kernel, dim3(blocks), dim3(64 * SK_WAVES), (uint32_t)lds, s, g);
+    const dim3 grid((unsigned)deal.blocks), block(64 * SK_WAVES);
+    if (most == 0) {
+        launch_kernel(kernel, grid, block, (uint32_t)lds, s, g);
         return hipGetLastError();
     }
-    launch_kernel_part(LaunchPart::First, kernel, dim3(blocks), dim3(64 * SK_WAVES), (uint32_t)lds, s, g);
+    launch_kernel_part(LaunchPart::First, kernel, grid, block, (uint32_t)lds, s, g);
     launch_kernel_part(LaunchPart::Last, skinny_reduce_kernel, dim3((unsigned)((most + 255) / 256), (unsigned)g.count),
                        dim3(256), 0, s, g);
     return hipGetLastError();
@@ -536,14 +529,18 @@ hipError_t launch_gemm_skinny_group(hipStream_t s, int M, int count, const float
                                     const mvlm_weight* const* ws, float* const* Ys, int num_cus,
                                     const Epilogue* eps, void* workspace, size_t workspace_bytes) {
     if (M < 1 || M > 16 || count < 1 || count > SKINNY_MAX_GROUP) return hipErrorInvalidValue;
-    const bool have = workspace && workspace_bytes >= skinny_workspace_bytes(M, count, ws);
+    if (num_cus <= 0) num_cus = 256;
+    for (int i = 0; i < count; ++i)
+        if (ws[i]->K % 32 != 0 || !is_quant(ws[i]->dtype) || ws[i]->dtype != ws[0]->dtype) return hipErrorInvalidValue;
+    const size_t need = skinny_partial_bytes(M, count, ws);
+    if ((need > 0 && (!workspace || workspace_bytes < need)) || !skinny_keeps_x(M, count, ws, num_cus))
+        return launch_skinny_kwalk(s, M, count, Xs, ws, Ys, num_cus, eps);
     float* part = (float*)workspace;
     SkinnyGroup g{};
     g.count = count;
     g.M = M;
     for (int i = 0; i < count; ++i) {
         const mvlm_weight* W = ws[i];
-        if (W->K % 32 != 0 || !is_quant(W->dtype) || W->dtype != ws[0]->dtype) return hipErrorInvalidValue;
         SkinnyProblem& p = g.p[i];
         p.X = Xs[i];
         p.codes = (const uint8_t*)W->data;
@@ -555,7 +552,7 @@ hipError_t launch_gemm_skinny_group(hipStream_t s, int M, int count, const float
         p.chunks = skinny_chunks(W->K);
         p.chunk_blocks = (W->K / 32 + p.chunks - 1) / p.chunks;
         p.chunk_div = (uint32_t)((((uint64_t)1 << 32) + p.chunks - 1) / p.chunks);   // (not used for one chunk)
-        if (p.chunks > 1 && have) {
+        if (p.chunks > 1) {
             p.part = part;
             part += (size_t)p.chunks * M * W->N;
         }
@@ -564,8 +561,8 @@ hipError_t launch_gemm_skinny_group(hipStream_t s, int M, int count, const float
             p.ep_on = 1;
         }
     }
-    if (num_cus <= 0) num_cus = 256;
-    return ws[0]->dtype == MVLM_Q4_0 ? launch_skinny<true>(s, g, num_cus) : launch_skinny<false>(s, g, num_cus);
+    const SkinnyDeal deal = skinny_deal(count, ws, num_cus);
+    return ws[0]->dtype == MVLM_Q4_0 ? launch_skinny<true>(s, g, deal) : launch_skinny<false>(s, g, deal);
 }
 
 }  // namespace mvlm

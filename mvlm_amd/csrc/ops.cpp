@@ -306,7 +306,7 @@ bool stream_serves(const mvlm_weight* w, int M) { return M <= STREAM_ROWS && str
 void skinny_workspace(mvlm_device* dev, int count, Op* op) {
     const char* use = std::getenv("MVLM_SKINNY_WORKSPACE");
     if (use && use[0] == '0') return;
-    const size_t bytes = skinny_workspace_bytes(op->M, count, op->gw);
+    const size_t bytes = skinny_workspace_bytes(op->M, count, op->gw, op->num_cus);
     if (bytes > 0 && device_scratch(dev, bytes, &op->workspace) == MVLM_OK) op->workspace_bytes = bytes;
 }
 

@@ -2,8 +2,9 @@
 cut: K of one chunk, of a full one (64 blocks), of two and more chunks that
 start at even and odd blocks, with fewer blocks than waves; row counts that are
 no multiple of 16; one row group per workgroup, more than a batch of four, and
-more than one round of workgroups; each epilogue operand; and the form that
-walks the chunks without workspace."""
+more than one round of workgroups; each epilogue operand; and without
+workspace.  Each on the kernel that keeps X, on the one that walks K, and on the
+one that the launch's size picks."""
 import numpy as np
 import pytest
 
@@ -13,6 +14,13 @@ from tests.test_gpu_parity import make_quant, within
 pytestmark = pytest.mark.gpu
 
 F32, Q8, Q4 = m.F32, m.Q8_0, m.Q4_0
+
+
+@pytest.fixture(autouse=True, params=["x", "k", None])
+def form(request, monkeypatch):
+    if request.param:
+        monkeypatch.setenv("MVLM_SKINNY_FORM", request.param)
+    return request.param
 
 
 def reference(orc, qt, X, blocks, M, N, K):
@@ -44,10 +52,10 @@ def test_cuts(dev, orc, qt, M, N, K):
 @pytest.mark.parametrize("qt", [Q8, Q4])
 @pytest.mark.parametrize("M,N,K", [(16, 37, 65 * 32), (5, 4200, 130 * 32), (12, 300, 8192)])
 def test_without_workspace(dev, orc, monkeypatch, qt, M, N, K):
-    """the same sums, chunk by chunk in one workgroup"""
+    """on the kernel that needs none"""
     with_ws = run(dev, orc, qt, M, N, K)
     monkeypatch.setenv("MVLM_SKINNY_WORKSPACE", "0")
-    # fma chains that run through the chunks against chunk sums that are added
+    # one kernel's chunk sums against the other's fma chains
     assert np.allclose(run(dev, orc, qt, M, N, K), with_ws, rtol=0, atol=1e-5 * np.abs(with_ws).max())
 
 
