@@ -112,6 +112,9 @@ inline int64_t round_up(int64_t v, int64_t m) { return (v + m - 1) / m * m; }
 
 // Device workspace of at least `bytes` (see mvlm_device::scratch_blocks).
 int device_scratch(mvlm_device* dev, size_t bytes, void** out);
+// The same for an op that runs without: null where it cannot be had, which is no
+// error (none is recorded).
+void* device_scratch_if_any(mvlm_device* dev, size_t bytes);
 // The device's sync words (mvlm_device::sync_words), zeroed when first allocated.
 int device_sync_words(mvlm_device* dev, void** out);
 // Looks up the fixed workspace array's address on the current device

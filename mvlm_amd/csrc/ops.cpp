@@ -301,13 +301,13 @@ constexpr int STREAM_ROWS = 4;
 bool stream_serves(const mvlm_weight* w, int M) { return M <= STREAM_ROWS && stream_supported(w, M); }
 
 // Workspace of a skinny GEMM over op->gw[0..count).  An op that gets none still
-// runs (launch_gemm_skinny_group), so a failed allocation is not an error.
-// MVLM_SKINNY_WORKSPACE=0: take none (tests).
+// runs (launch_gemm_skinny_group).  MVLM_SKINNY_WORKSPACE=0: take none (tests).
 void skinny_workspace(mvlm_device* dev, int count, Op* op) {
     const char* use = std::getenv("MVLM_SKINNY_WORKSPACE");
     if (use && use[0] == '0') return;
     const size_t bytes = skinny_workspace_bytes(op->M, count, op->gw, op->num_cus);
-    if (bytes > 0 && device_scratch(dev, bytes, &op->workspace) == MVLM_OK) op->workspace_bytes = bytes;
+    op->workspace = device_scratch_if_any(dev, bytes);
+    op->workspace_bytes = op->workspace ? bytes : 0;
 }
 
 // Dense GEMV (M == 1) or dequantizing GEMV / skinny GEMM (M <= 16).

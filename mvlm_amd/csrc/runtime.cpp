@@ -139,26 +139,32 @@ extern "C" int mvlm_device_destroy(mvlm_device* dev) {
 }
 
 namespace mvlm {
-int device_scratch(mvlm_device* dev, size_t bytes, void** out) {
-    *out = nullptr;
-    if (bytes == 0) return MVLM_OK;
+void* device_scratch_if_any(mvlm_device* dev, size_t bytes) {
+    if (bytes == 0) return nullptr;
     if (bytes > dev->scratch_bytes) {
-        HIP_TRY(hipSetDevice(dev->ordinal));
         const size_t want = (bytes + 0xFFFFF) & ~(size_t)0xFFFFF;      // whole MiB
         void* p = nullptr;
-        if (hipMalloc(&p, want) != hipSuccess || !p) {
+        if (hipSetDevice(dev->ordinal) != hipSuccess || hipMalloc(&p, want) != hipSuccess || !p) {
             (void)hipGetLastError();
-            return set_error(MVLM_ERR_OUT_OF_MEMORY, "workspace allocation of %zu bytes failed", want);
+            return nullptr;
         }
         try {
             dev->scratch_blocks.push_back(p);
         } catch (...) {
             (void)hipFree(p);
-            return set_error(MVLM_ERR_OUT_OF_MEMORY, "workspace bookkeeping failed");
+            return nullptr;
         }
         dev->scratch_bytes = want;
     }
-    *out = dev->scratch_blocks.back();
+    return dev->scratch_blocks.back();
+}
+
+int device_scratch(mvlm_device* dev, size_t bytes, void** out) {
+    *out = nullptr;
+    if (bytes > dev->scratch_bytes) HIP_TRY(hipSetDevice(dev->ordinal));
+    *out = device_scratch_if_any(dev, bytes);
+    if (bytes > 0 && !*out)
+        return set_error(MVLM_ERR_OUT_OF_MEMORY, "workspace allocation of %zu bytes failed", bytes);
     return MVLM_OK;
 }
 
