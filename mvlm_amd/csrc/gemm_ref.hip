@@ -49,8 +49,12 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_order_kernel(const uint16
     constexpr int PA = BK + 4, PB = BN + 16;
     constexpr int CA = BM * BK / 8 / NT, CB = BK * BN / 8 / NT;   // 8-element chunks per thread and slice
     static_assert(CA >= 1 && CB >= 1 && CA * 8 * NT == BM * BK && CB * 8 * NT == BK * BN, "chunks per thread");
-    __shared__ __attribute__((aligned(16))) uint16_t As[2][BM * PA];
-    __shared__ __attribute__((aligned(16))) uint16_t Bs[2][BK * PB];
+    constexpr int PC = BN + 8;                        // the C tile's, where the slices were
+    constexpr int SLICES = 2 * (BM * PA + BK * PB);
+    __shared__ __attribute__((aligned(16))) uint16_t smem[SLICES > BM * PC ? SLICES : BM * PC];
+    uint16_t (*As)[BM * PA] = reinterpret_cast<uint16_t (*)[BM * PA]>(smem);
+    uint16_t (*Bs)[BK * PB] = reinterpret_cast<uint16_t (*)[BK * PB]>(smem + 2 * BM * PA);
+    static_assert(2 * BM * PA % 8 == 0, "16-byte aligned slices of B");
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int l16 = lane & 15, q = lane >> 4;
     const int wm = (wave / WGN) * WM, wn = (wave % WGN) * WN;
@@ -131,18 +135,31 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_order_kernel(const uint16
         if (more) store(buf ^ 1);
         __syncthreads();
     }
+    // through LDS, rows of C as 16-byte pieces (stored two bytes at a time from
+    // the accumulators 2048 x 2048 x 8 took 9.0 us, now 6.9); the loop's last barrier ends
+    // the reads of the slices
 #pragma unroll
     for (int i = 0; i < TM; ++i)
 #pragma unroll
-        for (int j = 0; j < TN; ++j) {
-            const int col = n0 + wn + 16 * j + l16;
-            if (col >= N) continue;
+        for (int j = 0; j < TN; ++j)
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                const int row = m0 + wm + 16 * i + 4 * q + r;
-                if (row < M) C[(int64_t)row * N + col] = f32_to_f16_bits(acc[i][j][r]);
-            }
+            for (int r = 0; r < 4; ++r)
+                smem[(wm + 16 * i + 4 * q + r) * PC + wn + 16 * j + l16] = f32_to_f16_bits(acc[i][j][r]);
+    __syncthreads();
+#pragma unroll
+    for (int c = 0; c < (BM * BN / 8 + NT - 1) / NT; ++c) {
+        const int i = tid + c * NT;
+        if (i >= BM * BN / 8) break;
+        const int row = m0 + i / (BN / 8), col = n0 + 8 * (i % (BN / 8));
+        if (row >= M || col >= N) continue;
+        const uint16_t* v = smem + (i / (BN / 8)) * PC + 8 * (i % (BN / 8));
+        uint16_t* out = C + (int64_t)row * N + col;
+        if (N - col >= 8) {
+            __builtin_memcpy(out, v, 16);
+        } else {
+            for (int e = 0; e < N - col; ++e) out[e] = v[e];
         }
+    }
 }
 
 template <int BM, int BN, int BK, int WGM, int WGN>
@@ -153,18 +170,20 @@ static hipError_t launch_order(hipStream_t s, const uint16_t* A, const uint16_t*
     return hipGetLastError();
 }
 
-// Serves mvlm_gemm_naive and mvlm_gemm_tiled.  The tile with the least work on
-// the busiest CU: block rounds x tile area, the smaller tiles weighted by the
-// operand bytes they move per product.  (1024^3 takes 256 blocks of 64: 30 us;
-// 2048^3 takes 256 blocks of 128.)
+// Serves mvlm_gemm_naive and mvlm_gemm_tiled.  The tile with the least time on
+// the busiest CU: its blocks times what a block takes, `fixed` and `slice` us for
+// each slice of K begun (fitted at 4096 x 4096: 17.0, 27.1 and 57.5 us at K = 32,
+// 75.6, 81.7 and 106 at K = 256).  1024^3 takes 256 blocks of 64 (30 us), 2048^3
+// 256 of 128, 1500 x 1500 x 8 144 of 128 (6.7 us; 10.2 with 2209 of 32, which
+// counting the products of whole slices alone would take).
 hipError_t launch_gemm_order(hipStream_t s, const uint16_t* A, const uint16_t* B, uint16_t* C, int M, int N, int K,
                              int num_cus) {
     const int cus = num_cus > 0 ? num_cus : 256;
-    auto cost = [&](int edge, double weight) {
+    auto cost = [&](int edge, int bk, double fixed, double slice) {
         const int64_t tiles = (int64_t)((M + edge - 1) / edge) * ((N + edge - 1) / edge);
-        return (double)((tiles + cus - 1) / cus) * edge * edge * weight;
+        return (double)((tiles + cus - 1) / cus) * (fixed + slice * (K / bk + (K % bk != 0)));
     };
-    const double c128 = cost(128, 1.0), c64 = cost(64, 1.1), c32 = cost(32, 1.35);
+    const double c128 = cost(128, 32, 1.18, 2.09), c64 = cost(64, 64, 0.31, 1.14), c32 = cost(32, 128, 0.08, 0.76);
     if (c128 <= c64 && c128 <= c32) return launch_order<128, 128, 32, 4, 2>(s, A, B, C, M, N, K);
     if (c64 <= c32) return launch_order<64, 64, 64, 2, 2>(s, A, B, C, M, N, K);
     return launch_order<32, 32, 128, 2, 2>(s, A, B, C, M, N, K);

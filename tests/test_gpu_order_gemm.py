@@ -11,7 +11,7 @@ pytestmark = pytest.mark.gpu
 
 # 32-wide tiles: up to a few hundred outputs on a side; 64: about 16 x 16
 # tiles; 128: more than 256 tiles of 64 that round up to 256 of 128
-SHAPES = [(31, 33, 127), (32, 64, 128), (33, 40, 129), (16, 256, 256), (1000, 1001, 65), (1024, 960, 64),
+SHAPES = [(1500, 1500, 8), (2045, 2043, 1), (128, 33000, 17), (31, 33, 127), (32, 64, 128), (33, 40, 129), (16, 256, 256), (1000, 1001, 65), (1024, 960, 64),
           (1985, 2047, 33), (2048, 1992, 40), (1921, 2048, 31)]
 
 
