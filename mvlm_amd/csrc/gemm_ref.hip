@@ -77,16 +77,16 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_order_kernel(const uint16
         }
         return v;
     };
-    auto load = [&](int k0) {
+    auto load = [&](int k0) {                         // k0 < K: sums with it stay off int's end
 #pragma unroll
         for (int c = 0; c < CA; ++c) {
-            const int i = tid + c * NT, r = i / (BK / 8), k = k0 + 8 * (i % (BK / 8));
-            ra[c] = load8(A + (int64_t)(m0 + r) * K + k, m0 + r < M ? K - k : 0);
+            const int i = tid + c * NT, r = i / (BK / 8), k = 8 * (i % (BK / 8));
+            ra[c] = load8(A + (int64_t)(m0 + r) * K + k0 + k, m0 + r < M ? K - k0 - k : 0);
         }
 #pragma unroll
         for (int c = 0; c < CB; ++c) {
-            const int i = tid + c * NT, k = k0 + i / (BN / 8), n = n0 + 8 * (i % (BN / 8));
-            rb[c] = load8(B + (int64_t)k * N + n, k < K ? N - n : 0);
+            const int i = tid + c * NT, k = i / (BN / 8), n = n0 + 8 * (i % (BN / 8));
+            rb[c] = load8(B + ((int64_t)k0 + k) * N + n, k < K - k0 ? N - n : 0);
         }
     };
     auto store = [&](int buf) {
@@ -113,9 +113,9 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_order_kernel(const uint16
     load(0);
     store(0);
     __syncthreads();
-    for (int k0 = 0, buf = 0; k0 < K; k0 += BK, buf ^= 1) {
-        const bool more = k0 + BK < K;
-        if (more) load(k0 + BK);
+    for (int left = K, buf = 0; left > 0; left -= BK, buf ^= 1) {
+        const bool more = left > BK;
+        if (more) load(K - left + BK);
         const uint16_t* as = As[buf] + (wm + l16) * PA + q;
         const uint16_t* bs = Bs[buf] + q * PB + wn + l16;
 #pragma unroll
