@@ -426,7 +426,7 @@ int mvlm_marker_elapsed_ms(mvlm_event* start, mvlm_event* end, float* ms);
  * 1: one flag per workgroup, every workgroup polls all flags; 2: counter whose
  * last arriver raises a done flag replicated on 32 lines.  background != 0:
  * the workgroups' other 8 waves stream HBM meanwhile.  Waits are bounded
- * (20 ms); a wait that gives up returns MVLM_ERR_HIP.  Synchronous; allocates
+ * (200 ms); a wait that gives up returns MVLM_ERR_HIP.  Synchronous; allocates
  * (512 MiB with background). */
 int mvlm_probe_grid_barrier(mvlm_device* dev, int variant, int rounds, int background, double* us_per_round);
 

@@ -13,7 +13,7 @@
 //      all flags
 //   2  returning atomic add; the last arriver raises a done flag replicated on
 //      32 lines, each workgroup polls its replica
-// Every wait is bounded (20 ms); a round that gives up ends the workgroup's
+// Every wait is bounded (200 ms); a round that gives up ends the workgroup's
 // rounds and is reported as MVLM_ERR_HIP.
 #include "common.h"
 
@@ -36,7 +36,7 @@ struct ProbeArgs {
     int nb, rounds, variant, background;
 };
 
-constexpr uint64_t PROBE_TIMEOUT = 2000000;   // 20 ms at 100 MHz
+constexpr uint64_t PROBE_TIMEOUT = 20000000;   // 200 ms at 100 MHz
 
 __device__ __forceinline__ uint32_t probe_ld(const uint32_t* p) {
     return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -243,7 +243,7 @@ extern "C" int mvlm_probe_grid_barrier(mvlm_device* dev, int variant, int rounds
     if (st == MVLM_OK) st = check_hip(hipMemcpy(&err, a.err, 4, hipMemcpyDeviceToHost), "probe read");
     (void)hipFree(mem);
     if (st != MVLM_OK) return st;
-    if (err) return set_error(MVLM_ERR_HIP, "mvlm_probe_grid_barrier: a barrier wait gave up after 20 ms");
+    if (err) return set_error(MVLM_ERR_HIP, "mvlm_probe_grid_barrier: a barrier wait gave up after 200 ms");
     uint64_t mx = 0;
     for (uint64_t t : ticks) mx = t > mx ? t : mx;
     *us_per_round = (double)mx / 100.0 / rounds;   // s_memrealtime: 100 MHz
