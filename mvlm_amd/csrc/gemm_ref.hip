@@ -11,6 +11,8 @@
 #include "common.h"
 #include "device_math.h"
 
+#include <algorithm>
+
 namespace mvlm {
 
 // The products run on v_mfma_f32_16x16x4_f32.  The product of two widened
@@ -29,7 +31,7 @@ namespace mvlm {
 // NW waves owns a BM x BN tile of C, a wave TM x TN tiles of 16 x 16; the next
 // BK-wide slice of A and B is in flight to registers while the current one is
 // multiplied, and the LDS slices alternate (one barrier per slice).  2048^3:
-// 399 -> 156 us (43 -> 110 TFLOP/s) against the vector-ALU kernel of 64 x 64
+// 399 -> 154 us (43 -> 112 TFLOP/s) against the vector-ALU kernel of 64 x 64
 // tiles this replaces; 256^3 36 -> 5.2 us, 32 x 2048 x 2048 253 -> 22 us,
 // rows off the 16-byte grid (1500^3) 293 -> 101 us.
 // Operand layout: lane l supplies A[l%16][k + l/16] and B[k + l/16][l%16];
@@ -49,12 +51,8 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_order_kernel(const uint16
     constexpr int PA = BK + 4, PB = BN + 16;
     constexpr int CA = BM * BK / 8 / NT, CB = BK * BN / 8 / NT;   // 8-element chunks per thread and slice
     static_assert(CA >= 1 && CB >= 1 && CA * 8 * NT == BM * BK && CB * 8 * NT == BK * BN, "chunks per thread");
-    constexpr int PC = BN + 8;                        // the C tile's, where the slices were
-    constexpr int SLICES = 2 * (BM * PA + BK * PB);
-    __shared__ __attribute__((aligned(16))) uint16_t smem[SLICES > BM * PC ? SLICES : BM * PC];
-    uint16_t (*As)[BM * PA] = reinterpret_cast<uint16_t (*)[BM * PA]>(smem);
-    uint16_t (*Bs)[BK * PB] = reinterpret_cast<uint16_t (*)[BK * PB]>(smem + 2 * BM * PA);
-    static_assert(2 * BM * PA % 8 == 0, "16-byte aligned slices of B");
+    __shared__ __attribute__((aligned(16))) uint16_t As[2][BM * PA];
+    __shared__ __attribute__((aligned(16))) uint16_t Bs[2][BK * PB];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int l16 = lane & 15, q = lane >> 4;
     const int wm = (wave / WGN) * WM, wn = (wave % WGN) * WN;
@@ -113,9 +111,10 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_order_kernel(const uint16
     load(0);
     store(0);
     __syncthreads();
-    for (int left = K, buf = 0; left > 0; left -= BK, buf ^= 1) {
-        const bool more = left > BK;
-        if (more) load(K - left + BK);
+    uint32_t buf = 0;
+    for (uint32_t k0 = 0; k0 < (uint32_t)K; k0 += BK, buf ^= 1) {   // (an int would overflow past the last slice)
+        const bool more = k0 + BK < (uint32_t)K;
+        if (more) load((int)(k0 + BK));
         const uint16_t* as = As[buf] + (wm + l16) * PA + q;
         const uint16_t* bs = Bs[buf] + q * PB + wn + l16;
 #pragma unroll
@@ -135,30 +134,35 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_order_kernel(const uint16
         if (more) store(buf ^ 1);
         __syncthreads();
     }
-    // through LDS, rows of C as 16-byte pieces (stored two bytes at a time from
-    // the accumulators 2048 x 2048 x 8 took 9.0 us, now 6.9); the loop's last barrier ends
-    // the reads of the slices
+    constexpr int PC = WN + 8;                        // pitch of a wave's 16 rows of C
+    static_assert(NT / 64 * 16 * PC <= 2 * BM * PA || NT / 64 * 16 * PC <= 2 * BK * PB, "staging");
+    // Through LDS, 16 rows of the wave at a time, stored as 16-byte pieces (two
+    // bytes at a time from the accumulators 2048 x 2048 x 8 took 9.2 us, now 6.5);
+    // the loop's last barrier ended the reads of the slices.  A region of its own
+    // per wave needs no further barrier: through one tile of the whole block
+    // 2048^3 took 161 us, so 154.
+    uint16_t* const cw = (NT / 64 * 16 * PC <= 2 * BM * PA ? As[0] : Bs[0]) + wave * 16 * PC;
 #pragma unroll
-    for (int i = 0; i < TM; ++i)
+    for (int i = 0; i < TM; ++i) {
 #pragma unroll
         for (int j = 0; j < TN; ++j)
 #pragma unroll
-            for (int r = 0; r < 4; ++r)
-                smem[(wm + 16 * i + 4 * q + r) * PC + wn + 16 * j + l16] = f32_to_f16_bits(acc[i][j][r]);
-    __syncthreads();
+            for (int r = 0; r < 4; ++r) cw[(4 * q + r) * PC + 16 * j + l16] = f32_to_f16_bits(acc[i][j][r]);
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // this wave's writes, before its reads
 #pragma unroll
-    for (int c = 0; c < (BM * BN / 8 + NT - 1) / NT; ++c) {
-        const int i = tid + c * NT;
-        if (i >= BM * BN / 8) break;
-        const int row = m0 + i / (BN / 8), col = n0 + 8 * (i % (BN / 8));
-        if (row >= M || col >= N) continue;
-        const uint16_t* v = smem + (i / (BN / 8)) * PC + 8 * (i % (BN / 8));
-        uint16_t* out = C + (int64_t)row * N + col;
-        if (N - col >= 8) {
-            __builtin_memcpy(out, v, 16);
-        } else {
-            for (int e = 0; e < N - col; ++e) out[e] = v[e];
+        for (int c = lane; c < 16 * WN / 8; c += 64) {
+            const int row = m0 + wm + 16 * i + c / (WN / 8), col = n0 + wn + 8 * (c % (WN / 8));
+            if (row >= M || col >= N) continue;
+            const uint16_t* v = cw + (c / (WN / 8)) * PC + 8 * (c % (WN / 8));
+            uint16_t* out = C + (int64_t)row * N + col;
+            if (N - col >= 8) {
+                u32x4 t = *reinterpret_cast<const u32x4*>(v);
+                __builtin_memcpy(out, &t, 16);
+            } else {
+                for (int e = 0; e < N - col; ++e) out[e] = v[e];
+            }
         }
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // its reads, before the next rows' writes
     }
 }
 
@@ -170,20 +174,21 @@ static hipError_t launch_order(hipStream_t s, const uint16_t* A, const uint16_t*
     return hipGetLastError();
 }
 
-// Serves mvlm_gemm_naive and mvlm_gemm_tiled.  The tile with the least time on
-// the busiest CU: its blocks times what a block takes, `fixed` and `slice` us for
-// each slice of K begun (fitted at 4096 x 4096: 17.0, 27.1 and 57.5 us at K = 32,
-// 75.6, 81.7 and 106 at K = 256).  1024^3 takes 256 blocks of 64 (30 us), 2048^3
-// 256 of 128, 1500 x 1500 x 8 144 of 128 (6.7 us; 10.2 with 2209 of 32, which
-// counting the products of whole slices alone would take).
+// Serves mvlm_gemm_naive and mvlm_gemm_tiled.  The tile with the least work on
+// the busiest CU: its blocks times what a block takes, the smaller tiles weighted
+// by the operand bytes they move per product, plus a block's fixed time and no
+// less than one slice of K (4096 x 4096: 17.0, 27.1 and 57.5 us with tiles of 128,
+// 64 and 32 at K = 32).  1024^3 takes 256 blocks of 64 (30 us), 2048^3 256 of 128,
+// 1500 x 1500 x 8 144 of 128 (6.7 us; 10.2 with 2209 of 32, which the products
+// alone would take).
 hipError_t launch_gemm_order(hipStream_t s, const uint16_t* A, const uint16_t* B, uint16_t* C, int M, int N, int K,
                              int num_cus) {
     const int cus = num_cus > 0 ? num_cus : 256;
-    auto cost = [&](int edge, int bk, double fixed, double slice) {
+    auto cost = [&](int edge, int bk, double fixed, double slice) {   // us a block, us a slice
         const int64_t tiles = (int64_t)((M + edge - 1) / edge) * ((N + edge - 1) / edge);
-        return (double)((tiles + cus - 1) / cus) * (fixed + slice * (K / bk + (K % bk != 0)));
+        return (double)((tiles + cus - 1) / cus) * (fixed + slice * std::max(1.0, (double)K / bk));
     };
-    const double c128 = cost(128, 32, 1.18, 2.09), c64 = cost(64, 64, 0.31, 1.14), c32 = cost(32, 128, 0.08, 0.76);
+    const double c128 = cost(128, 32, 1.18, 2.09), c64 = cost(64, 64, 0.31, 1.15), c32 = cost(32, 128, 0.08, 0.705);
     if (c128 <= c64 && c128 <= c32) return launch_order<128, 128, 32, 4, 2>(s, A, B, C, M, N, K);
     if (c64 <= c32) return launch_order<64, 64, 64, 2, 2>(s, A, B, C, M, N, K);
     return launch_order<32, 32, 128, 2, 2>(s, A, B, C, M, N, K);
