@@ -43,9 +43,9 @@
 // workgroup per CU; the row groups of a launch are dealt out in whole rounds (up
 // to 14 row groups per workgroup).
 //
-// Against the other kernel, a Phi-1.5 step (49 grouped launches) of M = 16 went
-// 831 -> 670 us (Q4_0) and 867 -> 720 us (Q8_0), of M = 8 785 -> 626 and 806 ->
-// 672 us, its LM head 39 -> 22 and 39 -> 27 us.  What bounds a launch now (time
+// Against the other kernel alone, a Phi-1.5 step (49 grouped launches) of M = 16
+// went 831 -> 650 us (Q4_0) and 867 -> 701 us (Q8_0), of M = 8 785 -> 592 and 806
+// -> 648 us, its LM head 39 -> 22 and 39 -> 27 us.  What bounds a launch now (time
 // stamps of the M = 16 QKV + fc1 launch, 10.5 us): 128 KiB of X into every CU and
 // its split, 5 us before the first products, then 0.8 us (Q4_0, vector ALU and
 // matrix core in turn) to 1.2 us (Q8_0, HBM) per row group.  Sixteen waves of

@@ -293,10 +293,10 @@ int make_argmax(mvlm_device* dev, const mvlm_buffer* x, int dtype, int rows, int
 
 // Whether a quantized weight's product with M rows of x runs on the streaming
 // kernel rather than the skinny GEMM.  The streaming kernel multiplies each
-// weight on the vector ALU once per row, the skinny GEMM pays ~5 us per launch
-// to bring X into its registers whatever M is: a Phi-1.5 step of M = 4 takes
-// 586 us (Q4_0) and 633 us (Q8_0) streaming and 612 / 656 us skinny, one of
-// M = 8 would be twice the former.
+// weight on the vector ALU once per row, the skinny GEMM pays for 16 rows
+// whatever M is: a Phi-1.5 step of M = 4 takes 566 us (Q4_0) and 597 us (Q8_0)
+// streaming and 576 / 634 us skinny, one of M = 2 440 / 467 and 570 / 627, and
+// one of M = 8 would be twice the time of M = 4.
 constexpr int STREAM_ROWS = 4;
 bool stream_serves(const mvlm_weight* w, int M) { return M <= STREAM_ROWS && stream_supported(w, M); }
 
