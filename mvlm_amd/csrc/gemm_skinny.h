@@ -37,6 +37,30 @@ __device__ __forceinline__ f32x4 mfma16(u32x4 a, u32x4 b, f32x4 c) {
                                                    0, 0, 0);
 }
 
+// A lane's 8 codes of a block as bf16 (small integers, exact).  Q4_0: raw is
+// one dword, the result the raw nibbles c (0..15), low nibbles first; the -8
+// of (c - 8) comes in through the block sums of x.  A nibble in a byte is the
+// fp8 (E4M3) number c * 2^-9, denormal or not, so one scaled conversion makes
+// two of them.
+template <bool Q4>
+__device__ __forceinline__ u32x4 codes_to_bf16(u32x2 raw) {
+    u32x4 out;
+    if constexpr (Q4) {
+        const uint32_t lo = raw[0] & 0x0F0F0F0Fu, hi = (raw[0] >> 4) & 0x0F0F0F0Fu;
+        out[0] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(lo, 512.0f, false));
+        out[1] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(lo, 512.0f, true));
+        out[2] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(hi, 512.0f, false));
+        out[3] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(hi, 512.0f, true));
+    } else {
+        float v[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) v[j] = (float)(int8_t)(raw[j >> 2] >> (8 * (j & 3)));
+#pragma unroll
+        for (int j = 0; j < 4; ++j) out[j] = pack_hi16(v[2 * j], v[2 * j + 1]);
+    }
+    return out;
+}
+
 constexpr int SKINNY_MAX_GROUP = 8;
 
 // The kernel that walks K (gemm_skinny_kwalk.hip): whether its LDS, which stages

@@ -21,8 +21,11 @@
 //
 // Two kernels share that arithmetic, chosen per launch by size (skinny_keeps_x).
 // The one in gemm_skinny_kwalk.hip reads X again for every one to four row groups
-// of the weight; the one here keeps X in registers.  The last bits of an output
-// depend on the kernel and so on what else its launch holds.
+// of the weight; the one here keeps X in registers.  Their sums over a block are
+// the same, the order of the blocks is not: the last bits of an output depend on
+// the kernel and so on what else its launch holds, its error (2-norm against 64
+// bits, 1.0e-7 to 1.2e-7 for Q8_0, 1.4e-7 to 1.8e-7 for Q4_0 over K = 512 ..
+// 14336) does not.
 //
 // Operand layout of v_mfma_f32_16x16x32_bf16: lane l supplies
 // A[l%16][8*(l/16) .. +7] and B[8*(l/16) .. +7][l%16]; accumulator register i
@@ -70,30 +73,6 @@
 #include <cstdlib>
 
 namespace mvlm {
-
-// A lane's 8 codes of a block as bf16 (small integers, exact).  Q4_0: raw is
-// one dword, the result the raw nibbles c (0..15), low nibbles first; the -8
-// of (c - 8) comes in through the block sums of x.  A nibble in a byte is the
-// fp8 (E4M3) number c * 2^-9, denormal or not, so one scaled conversion makes
-// two of them.
-template <bool Q4>
-__device__ __forceinline__ u32x4 codes_to_bf16(u32x2 raw) {
-    u32x4 out;
-    if constexpr (Q4) {
-        const uint32_t lo = raw[0] & 0x0F0F0F0Fu, hi = (raw[0] >> 4) & 0x0F0F0F0Fu;
-        out[0] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(lo, 512.0f, false));
-        out[1] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(lo, 512.0f, true));
-        out[2] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(hi, 512.0f, false));
-        out[3] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(hi, 512.0f, true));
-    } else {
-        float v[8];
-#pragma unroll
-        for (int j = 0; j < 8; ++j) v[j] = (float)(int8_t)(raw[j >> 2] >> (8 * (j & 3)));
-#pragma unroll
-        for (int j = 0; j < 4; ++j) out[j] = pack_hi16(v[2 * j], v[2 * j + 1]);
-    }
-    return out;
-}
 
 // Barrier that orders the workgroup's LDS accesses and leaves loads from
 // memory in flight (__syncthreads() would wait for all of them).
@@ -451,15 +430,17 @@ static SkinnyDeal skinny_deal(int count, const mvlm_weight* const* ws, int num_c
 // 9.2, 8192 x 3072 12.1 and 15.0; 51200 x 2048 38.7 and 27.3, 2048 x 8192 16.6 and
 // 14.0, 32000 x 1024 15.4 and 14.3.  The costs are fitted to the times of both
 // over 2700 launches (N 64 .. 51200, K 64 .. 11008, M 5 .. 16, single and
-// grouped): the choice is 0.3% from the faster one on average, and more than 6%
-// from it in 2% of them.  MVLM_SKINNY_FORM=x or k forces one (tests, tuning; read
+// grouped): the choice is 0.4% from the faster one on average, and more than 6%
+// from it in 2.5% of them.  MVLM_SKINNY_FORM=x or k forces one (tests, tuning; read
 // at every launch).
 static bool skinny_keeps_x(int M, int count, const mvlm_weight* const* ws, int num_cus) {
     if (const char* force = std::getenv("MVLM_SKINNY_FORM")) return force[0] == 'x';
+    for (int i = 0; i < count; ++i)
+        if (ws[i]->K > 16384) return true;   // beyond the fit (Q8_0 8192 x 32768: 72 us, 81 with K walked; 2048 rows 26 and 38)
     struct Cost {
         double launch, row_group, block, row, cut, partial, round;
     };
-    constexpr Cost kQ8{5.7, 0.50, 0.0168, 0.091, 2.5, 1.9, 5.2}, kQ4{5.5, 0.48, 0.0116, 0.084, 2.4, 2.0, 4.2};
+    constexpr Cost kQ8{5.7, 0.51, 0.0171, 0.092, 2.5, 2.0, 5.1}, kQ4{5.5, 0.49, 0.0116, 0.084, 2.3, 2.3, 4.2};
     const Cost& c = ws[0]->dtype == MVLM_Q4_0 ? kQ4 : kQ8;
     const SkinnyDeal deal = skinny_deal(count, ws, num_cus);
     double units = 0, blocks = 0, parts = 0;   // row groups times chunks, their blocks of K, 10^6 partial sums
@@ -473,7 +454,7 @@ static bool skinny_keeps_x(int M, int count, const mvlm_weight* const* ws, int n
     const double busy = std::min((double)deal.blocks / num_cus, (double)deal.rounds) * deal.rows;
     const double us = c.launch + c.row_group * deal.rounds * deal.rows + c.block * busy * (blocks / units) + c.row * M +
                       (parts > 0 ? c.cut + c.partial * parts : 0.0) + c.round * (deal.rounds - 1);
-    return us < 1.01 * skinny_kwalk_us(M, count, ws, num_cus);
+    return us < 1.02 * skinny_kwalk_us(M, count, ws, num_cus);
 }
 
 static size_t skinny_partial_bytes(int M, int count, const mvlm_weight* const* ws) {

@@ -1,13 +1,8 @@
 // The skinny GEMM's kernel whose waves walk K with their rows (gemm_skinny.hip
 // has the arithmetic's account and says which launches come here).
 //
-// Operand layout of v_mfma_f32_16x16x32_bf16: lane l supplies A[l%16][8*(l/16) ..
-// +7] and B[8*(l/16) .. +7][l%16]; accumulator register i of lane l is
-// D[4*(l/16) + i][l%16].  Here A = X (row m = l%16) and B = w^T (weight row n0 +
-// l%16), so lane l reads 8 consecutive codes of
-// its weight row: Q8_0 bytes 8q..8q+7 of the block (q = l/16), Q4_0 the low
-// (q < 2) or high (q >= 2) nibbles of bytes 8*(q&1)..+7 (byte j holds weights
-// j and j + 16).
+// The operand layout and the order of k inside a block are that file's, so a
+// block's sum has the same bits in both kernels.
 //
 // A block of NW waves owns R groups of 16 weight rows; wave w takes the w-th
 // NW-th of the K blocks and walks it in steps of G blocks (4, or 2 with four
@@ -17,7 +12,7 @@
 // each step's codes of the wave's rows (16R rows x 32G bytes for Q8_0, x 16G
 // bytes for Q4_0) are copied
 // into the wave's own LDS slot with direct 16-byte loads (1 KiB contiguous
-// per instruction), double-buffered, and read back per lane (ds_read_b64).
+// per instruction), double-buffered, and read back per lane.
 // The 16-byte pieces of each LDS row are XOR-swizzled with row bits so the
 // 16 lanes of a read hit distinct banks.  The block's scales (all K) are
 // staged once per block.  X goes straight to registers, one step ahead:
@@ -32,35 +27,6 @@
 #include <algorithm>
 
 namespace mvlm {
-
-// 8 small integers (exact in bf16) from 8 code bytes / nibbles.  Q4_0 gives
-// the raw nibbles c (0..15): masked into bytes, one byte-to-float conversion
-// each; the -8 of (c - 8) is applied per block through the block sums of x.
-template <bool Q4>
-__device__ __forceinline__ u32x4 kwalk_codes_to_bf16(u32x2 raw, int q) {
-    float v[8];
-    if constexpr (Q4) {
-        const int shift = (q >> 1) * 4;
-        uint32_t lo = (raw[0] >> shift) & 0x0F0F0F0Fu, hi = (raw[1] >> shift) & 0x0F0F0F0Fu;
-        // opaque to the compiler, which would otherwise fold each byte's
-        // shift and mask into a bit-field extract per code in front of the
-        // conversion; this way v_cvt_f32_ubyte{0..3} read the bytes directly
-        asm_pin(lo);
-        asm_pin(hi);
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            v[j] = (float)((lo >> (8 * j)) & 0xFFu);
-            v[4 + j] = (float)((hi >> (8 * j)) & 0xFFu);
-        }
-    } else {
-#pragma unroll
-        for (int j = 0; j < 8; ++j) v[j] = (float)(int8_t)(raw[j >> 2] >> (8 * (j & 3)));
-    }
-    u32x4 out;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) out[j] = pack_hi16(v[2 * j], v[2 * j + 1]);
-    return out;
-}
 
 constexpr size_t KWALK_LDS_MAX = 160 * 1024;
 
@@ -158,7 +124,7 @@ __global__ __launch_bounds__(64 * NW, 4) void skinny_kwalk_kernel(const KwalkGro
     const __amdgpu_buffer_rsrc_t crs = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<uint8_t*>(codes), 0, (int)min((int64_t)N * ld, (int64_t)0x7FFFFFFF), 0x00020000);
     const i32x4 xrs = raw_rsrc(X, (uint32_t)((int64_t)M * K * 4));
-    const uint32_t xrow = (uint32_t)(((int64_t)min(l16, M - 1) * K + 8 * q) * 4);
+    const uint32_t xrow = (uint32_t)(((int64_t)min(l16, M - 1) * K + (Q4 ? 4 : 8) * q) * 4);
     const int dma_row = lane / L::P, dma_piece = lane % L::P;
     auto issue_codes = [&](int step, int slot_idx) {
         const int kb = b0 + step * G;
@@ -181,18 +147,19 @@ __global__ __launch_bounds__(64 * NW, 4) void skinny_kwalk_kernel(const KwalkGro
     // at M <= 8 (at most 8 distinct lines) those selects cost more than the
     // conflicts (Q4_0 M = 5 707 -> 725 us), so XS is off there.
     const bool xodd = XS && (min(l16, M - 1) & 1) != 0;   // parity of the row actually read
-    const int xsw = xodd ? 4 : 0;
+    constexpr int XP = Q4 ? 16 : 4;                   // floats between a lane's two pieces
+    const int xsw = xodd ? XP : 0;
     auto load_x = [&](int step, int g, u32x4 (&xg)[2]) {
         const int bb = min(b0 + step * G + g, nb - 1);
         xg[0] = asm_buffer_load_b128(xrs, xrow + (uint32_t)(32 * bb + xsw) * 4);
-        xg[1] = asm_buffer_load_b128(xrs, xrow + (uint32_t)(32 * bb + 4 - xsw) * 4);
+        xg[1] = asm_buffer_load_b128(xrs, xrow + (uint32_t)(32 * bb + XP - xsw) * 4);
     };
 
     // Lanes whose X row is past M (clamped to row M - 1 above) only feed
     // output rows m >= M, which are never stored.
-    f32x4 acc[R];
+    f32x4 sum[R];                                     // of the steps' sums: two short chains round less than one long one
 #pragma unroll
-    for (int r = 0; r < R; ++r) acc[r] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    for (int r = 0; r < R; ++r) sum[r] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
     u32x4 xr[G][2];                                   // X of the current step
     if (steps > 0) {
         issue_codes(0, 0);
@@ -212,6 +179,9 @@ __global__ __launch_bounds__(64 * NW, 4) void skinny_kwalk_kernel(const KwalkGro
     // branches the loop-carried X registers need no copies, which would read
     // them while their loads are still in flight.
     auto compute = [&](int step, u32x4 (&xr)[G][2], auto refill) {
+        f32x4 acc[R];
+#pragma unroll
+        for (int r = 0; r < R; ++r) acc[r] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
         const int kb = b0 + step * G;
         const uint32_t slot = lds_offset(slots + (step & 1) * SLOT);
         u32x2 raw[G][R];
@@ -223,7 +193,9 @@ __global__ __launch_bounds__(64 * NW, 4) void skinny_kwalk_kernel(const KwalkGro
 #pragma unroll
             for (int rr = 0; rr < R; ++rr) {
                 const int r = 16 * rr + l16;
-                raw[g][rr] = asm_lds_read_b64(slot + r * L::CB + 16 * L::piece(lpiece, r) + 8 * (q & 1));
+                const uint32_t at = slot + r * L::CB + 16 * L::piece(lpiece, r);
+                if constexpr (Q4) raw[g][rr][0] = asm_lds_read_b32(at + 4 * q);
+                else raw[g][rr] = asm_lds_read_b64(at + 8 * (q & 1));
                 dh[g][rr] = asm_lds_read_u16(lds_base + 2 * (r * nb + bb));
             }
         }
@@ -246,30 +218,33 @@ __global__ __launch_bounds__(64 * NW, 4) void skinny_kwalk_kernel(const KwalkGro
             }
             u32x4 p1, p2, p3;
             split3(x, p1, p2, p3);
-            f32x4 sx = {0.0f, 0.0f, 0.0f, 0.0f};      // Q4_0: sum of the block's x per X row
+            // Q4_0: -8 times the sum of the block's x per X row, where the block's
+            // sum starts (applied after it, errors are a third larger)
+            f32x4 sx = {0.0f, 0.0f, 0.0f, 0.0f};
             if constexpr (Q4) {
                 const u32x4 ones = {0x3F803F80u, 0x3F803F80u, 0x3F803F80u, 0x3F803F80u};   // bf16 1.0 pairs
                 sx = mfma16(p1, ones, sx);
                 sx = mfma16(p2, ones, sx);
                 sx = mfma16(p3, ones, sx);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) sx[i] *= -8.0f;
             }
 #pragma unroll
             for (int rr = 0; rr < R; ++rr) {
-                const u32x4 w = kwalk_codes_to_bf16<Q4>(raw[g][rr], q);
-                f32x4 c = {0.0f, 0.0f, 0.0f, 0.0f};
-                c = mfma16(p1, w, c);
+                const u32x4 w = codes_to_bf16<Q4>(raw[g][rr]);
+                f32x4 c = mfma16(p1, w, sx);
                 c = mfma16(p2, w, c);
                 c = mfma16(p3, w, c);
-                if constexpr (Q4) {
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) c[i] = __builtin_fmaf(-8.0f, sx[i], c[i]);
-                }
                 const float d = live ? f16_bits_to_f32((uint16_t)dh[g][rr]) : 0.0f;
 #pragma unroll
                 for (int i = 0; i < 4; ++i) acc[rr][i] = __builtin_fmaf(d, c[i], acc[rr][i]);
             }
             if constexpr (decltype(refill)::value) load_x(step + 1, g, xr[g]);
         }
+#pragma unroll
+        for (int r = 0; r < R; ++r)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) sum[r][i] += acc[r][i];
     };
 
     // Per step: the next step's codes; waiting until only those remain in
@@ -301,17 +276,19 @@ __global__ __launch_bounds__(64 * NW, 4) void skinny_kwalk_kernel(const KwalkGro
     __syncthreads();
     f32x4* part = reinterpret_cast<f32x4*>(lds + scale_region);
 #pragma unroll
-    for (int r = 0; r < R; ++r) part[(wave * R + r) * 64 + lane] = acc[r];
+    for (int r = 0; r < R; ++r) part[(wave * R + r) * 64 + lane] = sum[r];
     __syncthreads();
     if (wave < R) {                                   // wave r sums row group r
         const int r = wave;
-        f32x4 sum = part[r * 64 + lane];
+        f32x4 t[NW];                                  // added in pairs: half the roundings in a row of a running sum
 #pragma unroll
-        for (int w = 1; w < NW; ++w) {
-            const f32x4 t = part[(w * R + r) * 64 + lane];
+        for (int w = 0; w < NW; ++w) t[w] = part[(w * R + r) * 64 + lane];
 #pragma unroll
-            for (int i = 0; i < 4; ++i) sum[i] += t[i];
-        }
+        for (int span = 1; span < NW; span *= 2)
+#pragma unroll
+            for (int w = 0; w + span < NW; w += 2 * span)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) t[w][i] += t[w + span][i];
         const int n = n0 + 16 * r + l16;
         if (n < N) {
 #pragma unroll
@@ -319,7 +296,7 @@ __global__ __launch_bounds__(64 * NW, 4) void skinny_kwalk_kernel(const KwalkGro
                 const int m = 4 * q + i;
                 if (m < M) {
                     const int64_t idx = (int64_t)m * N + n;
-                    Y[idx] = P.ep_on ? apply_epilogue(P.ep, sum[i], idx, n) : sum[i];
+                    Y[idx] = P.ep_on ? apply_epilogue(P.ep, t[0][i], idx, n) : t[0][i];
                 }
             }
         }
@@ -371,10 +348,10 @@ double skinny_kwalk_us(int M, int count, const mvlm_weight* const* ws, int num_c
     struct Cost {
         double launch, group, step, stream, step_row, longest;
     };
-    constexpr Cost kQ8[] = {{}, {3.9, 0.20, 1.53, 0.41, 0.027, 0.0}, {4.5, -0.28, 0.82, 0.45, 0.031, 0.9},
-                            {2.2, 2.20, 1.94, 0.42, 0.072, 3.1}};
-    constexpr Cost kQ4[] = {{2.2, 2.19, 3.13, 0.50, 0.022, 0.0}, {4.1, 0.39, 1.47, 0.28, 0.022, 0.0}, {},
-                            {2.2, 2.36, 2.22, 0.18, 0.053, 2.7}};
+    constexpr Cost kQ8[] = {{}, {3.9, 0.20, 1.51, 0.45, 0.029, 0.0}, {4.5, -0.28, 0.85, 0.42, 0.031, 0.9},
+                            {2.2, 2.24, 1.91, 0.41, 0.075, 2.9}};
+    constexpr Cost kQ4[] = {{2.1, 2.11, 2.69, 0.71, 0.021, 0.0}, {4.2, 0.20, 1.21, 0.44, 0.028, 0.0}, {},
+                            {2.5, 1.93, 2.08, 0.26, 0.061, 2.7}};
     const bool q4 = ws[0]->dtype == MVLM_Q4_0;
     int64_t groups = 0;
     for (int i = 0; i < count; ++i) groups += (ws[i]->N + 15) / 16;

@@ -117,3 +117,23 @@ def test_not_a_number_stays_in_its_row(dev, orc, qt):
     dev.gemm_quant(dev.upload(X), dev.pack(blocks, qt, N, K), dY, M, N, K)
     bad = ~np.isfinite(dY.download(np.float32).reshape(M, N))
     assert bad[[3, 6, 8]].all() and not bad[[0, 1, 2, 4, 5, 7]].any()
+
+
+@pytest.mark.parametrize("form", [None], indirect=True)
+@pytest.mark.parametrize("qt", [Q8, Q4])
+@pytest.mark.parametrize("N,K", [(2048, 768), (2048, 2048), (512, 8192)])
+def test_walking_k_is_no_less_exact(dev, orc, monkeypatch, form, qt, N, K):
+    """2-norm of the error against 64 bits: the kernel that walks K within 1.05
+    of the one that keeps X (with one chain per wave and -8 x applied to a
+    block's sum it was 1.1 to 1.4 of it)"""
+    M = 16
+    X, blocks = orc.normal_f32(M * K, 681), make_quant(orc, qt, N, K, 682)
+    deq = orc.dequant_q8_0 if qt == Q8 else orc.dequant_q4_0
+    want = X.astype(np.float64).reshape(M, K) @ deq(blocks).astype(np.float64).reshape(N, K).T
+    dX, W, err = dev.upload(X), dev.pack(blocks, qt, N, K), {}
+    for kernel in "xk":
+        monkeypatch.setenv("MVLM_SKINNY_FORM", kernel)
+        dY = dev.alloc(M * N * 4)
+        dev.gemm_quant(dX, W, dY, M, N, K)
+        err[kernel] = np.linalg.norm(dY.download(np.float32).reshape(M, N) - want) / np.linalg.norm(want)
+    assert err["k"] <= 1.05 * err["x"], err
