@@ -463,11 +463,29 @@ __global__ __launch_bounds__(64 * WGM * WGN, PER_CU* WGM* WGN > 8 ? PER_CU * WGM
 #pragma unroll
         for (int j = 0; j < TN; ++j) asm_pin(f.b[j]);
     };
-    auto mma = [&](const Frags& f) {
+    // A wave of one accumulator tile sums its k-steps in four chains, a quarter of
+    // the roundings in a row each: K = 2112 against 64 bits 2.75e-7 -> 1.34e-7
+    // without a split, 1.36e-7 -> 0.84e-7 with four.  Two chains left 66x5836x1024
+    // at 1.28e-7, where more splits had 0.95e-7; 0.94e-7 with four.  The time is
+    // one chain's within 1% (32x2048x2048 9.3 us); 122 and 156 registers, as many
+    // blocks on a CU.
+    constexpr int CHAINS = TM * TN == 1 ? 4 : 1;
+    static_assert(BK / 16 % CHAINS == 0, "a k-step's chain is the same in every stage");
+    f32x16 chain[CHAINS];                             // chain 0 is acc
 #pragma unroll
-        for (int i = 0; i < TM; ++i)
+    for (int c = 1; c < CHAINS; ++c)
 #pragma unroll
-            for (int j = 0; j < TN; ++j) acc[i][j] = mfma32<BF16>(f.a[i], f.b[j], acc[i][j]);
+        for (int r = 0; r < 16; ++r) chain[c][r] = 0.0f;
+    auto mma = [&](const Frags& f, auto KS) {
+        constexpr int c = decltype(KS)::value % CHAINS;
+        if constexpr (c > 0) {
+            chain[c] = mfma32<BF16>(f.a[0], f.b[0], chain[c]);
+        } else {
+#pragma unroll
+            for (int i = 0; i < TM; ++i)
+#pragma unroll
+                for (int j = 0; j < TN; ++j) acc[i][j] = mfma32<BF16>(f.a[i], f.b[j], acc[i][j]);
+        }
     };
     // Stage s has landed in LDS for every wave once this returns.  `later`
     // stages were issued after s; those issued by the direct path may stay in
@@ -505,8 +523,8 @@ __global__ __launch_bounds__(64 * WGM * WGN, PER_CU* WGM* WGN > 8 ? PER_CU * WGM
     load_frags(0, 0, f[0]);
     for (int kt = 0; kt < nk; ++kt) {
         const int slot_idx = kt % STAGES;
-#pragma unroll
-        for (int ks = 0; ks < BK / 16; ++ks) {
+        static_for<BK / 16>([&](auto KS) {
+            constexpr int ks = decltype(KS)::value;
             Frags& nxt = f[(ks + 1) & 1];
             if (ks < BK / 16 - 1) {
                 load_frags(slot_idx, ks + 1, nxt);
@@ -519,9 +537,12 @@ __global__ __launch_bounds__(64 * WGM * WGN, PER_CU* WGM* WGN > 8 ? PER_CU * WGM
             // issued last, lgkmcnt(TM+TN) means this set has landed.  (At the
             // last k-step of the last stage nothing newer is pending.)
             ready(f[ks & 1], ks < BK / 16 - 1 || kt + 1 < nk);
-            mma(f[ks & 1]);
-        }
+            mma(f[ks & 1], KS);
+        });
     }
+    if constexpr (CHAINS == 4)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[0][0][r] = (acc[0][0][r] + chain[1][r]) + (chain[2][r] + chain[3][r]);
 
     const int64_t c_off = (int64_t)batch * p.sC;
     float* ws = p.splits > 1 ? p.ws + (int64_t)blockIdx.z * p.M * p.N : nullptr;

@@ -84,6 +84,24 @@ def test_epilogue(dev, orc, monkeypatch, tile, dt, offset, splits, act, names):
     check(orc, got, Y64, S, vals, act, dt, 1e-4)
 
 
+@pytest.mark.parametrize("tile", ["64x64s4w4", "64x64s2w4k128"])
+@pytest.mark.parametrize("K", [2112, 2239, 4096])
+def test_one_accumulator_tiles_sum_in_four_chains(dev, orc, monkeypatch, tile, K):
+    """K without a split, error against 64 bits.  Normal factors: the roundings of a chain of K / 16 sums add up as a
+    random walk, so relative to the result they grow with the square root of its length.  K = 2112: 2.75e-7 with one
+    chain, half of that (1.34e-7 measured) with four a quarter as long.  The limit is sqrt(2) from both."""
+    monkeypatch.setenv("MVLM_GEMM_TILE", tile)
+    monkeypatch.setenv("MVLM_GEMM_SPLITS", "1")
+    M, N = 121, 200
+    A, Wt = gen(orc, BF16, M * K, 0x440), gen(orc, BF16, N * K, 0x441)
+    C = dev.alloc(M * N * 4)
+    dev.gemm_packed(dev.upload(A), BF16, dev.pack(Wt, BF16, N, K), C, F32, M, N, K)
+    exact, _ = orc.gemm_f64(widen(orc, A, BF16).reshape(M, K), widen(orc, Wt, BF16).reshape(N, K), M, N, K)
+    got = C.download(np.float32).reshape(M, N)
+    err = np.linalg.norm(got - exact) / np.linalg.norm(exact)
+    assert err < 1.94e-7 * (K / 2112) ** 0.5, err
+
+
 def test_gelu_extremes(dev, orc):
     """the values that the tanh form gives: inf and large x pass, large -x is zero, -inf (0 times inf) is NaN"""
     x = np.array([np.inf, 65504.0, 12.0, 0.0, -12.0, -65504.0, -np.inf, np.nan], np.float16)
